@@ -55,6 +55,7 @@ __device__ __forceinline__ float dexp_sel(float x) {
   p = __builtin_fmaf(p, r, 1.0f);
   int ni = (int)n;
   float e = (p * 2.0f) * __int_as_float((ni - 1 + 127) << 23);
+  asm("" : "+v"(e));  // formed for every lane: sunk under the selects it would become a branch per call
   e = x < -86.5f ? 0.0f : e;
   e = x > 89.0f ? __int_as_float(0x7f800000) : e;
   return x != x ? x : e;

@@ -119,6 +119,10 @@ hipError_t launch_moe_combine(hipStream_t s, const Dims& d, const StepBufs& b, i
 // ny * heads * splits * 66 floats).
 hipError_t launch_attn_batched(hipStream_t s, const LayerDev& L, const Dims& d, const int* lenp, int len_add, int ny,
                                const float* q, float* part, float* att);
+// The split kernel of launch_attn_batched (attn_mm.hip), for G <= 4 query heads per KV head and any tps.
+hipError_t launch_attn_mm(hipStream_t s, int G, int kvh, int tps, const float* q, const uint16_t* kc,
+                          const uint16_t* vc, const int* lenp, int len_add, int max_len, float scale, int ny,
+                          float* part);
 // Output projection + residual; the epilogue writes the MoE-norm partials of the new h into b.zpart. from_hc: the
 // residual input is b.hc (the attention block's combined h) instead of b.h; the result goes to b.h either way.
 hipError_t launch_oproj(hipStream_t s, const LayerDev& L, const Dims& d, const StepBufs& b, Tl tl = {},
