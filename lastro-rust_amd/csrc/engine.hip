@@ -531,15 +531,15 @@ struct moert_model {
     if (pf.h) return MOERT_OK;
     const int H = dims.hidden, qd = dims.heads * 64, I = dims.inter, M = kPfMaxPos, K8 = 8;
     const size_t parts = (size_t)M * dims.heads * attn_splits_for(max_len, dims.tps) * 66;
+    pf.cap = M;
     int rc;
     if ((rc = zeros(arena, stream, (size_t)M, &pf.toks)) || (rc = zeros(arena, stream, (size_t)1, &pf.pos0)) ||
-        (rc = zeros(arena, stream, (size_t)M * H, &pf.h)) || (rc = zeros(arena, stream, (size_t)M * qd, &pf.q)) ||
-        (rc = zeros(arena, stream, (size_t)M * qd, &pf.att)) || (rc = zeros(arena, stream, parts, &pf.part)) ||
-        (rc = zeros(arena, stream, (size_t)M * kNormItems, &pf.zpart)) ||
-        (rc = zeros(arena, stream, (size_t)M * H, &pf.xn)) || (rc = zeros(arena, stream, (size_t)M * K8, &pf.ids)) ||
-        (rc = zeros(arena, stream, (size_t)M * K8, &pf.w)) ||
+        (rc = zeros(arena, stream, (size_t)M * qd, &pf.q)) || (rc = zeros(arena, stream, (size_t)M * qd, &pf.att)) ||
+        (rc = zeros(arena, stream, parts, &pf.part)) || (rc = zeros(arena, stream, (size_t)M * H, &pf.xn)) ||
+        (rc = zeros(arena, stream, (size_t)M * K8, &pf.ids)) || (rc = zeros(arena, stream, (size_t)M * K8, &pf.w)) ||
+        (rc = zeros(arena, stream, (size_t)64, &pf.cnt)) || (rc = zeros(arena, stream, (size_t)64 * M, &pf.list)) ||
         (rc = zeros(arena, stream, (size_t)M * K8 * I, &pf.act)) ||
-        (rc = zeros(arena, stream, (size_t)M * K8 * H, &pf.o)))
+        (rc = zeros(arena, stream, (size_t)M * K8 * H, &pf.o)) || (rc = zeros(arena, stream, (size_t)M * H, &pf.h)))
       return rc;
     CHECK_HIP(hipStreamSynchronize(stream));
     return MOERT_OK;
@@ -590,18 +590,21 @@ struct moert_model {
   // left in b.h, as after a decode step.
   int enqueue_batched(int pos0, int nv) {
     CHECK_HIP(launch_embed_b(stream, embed, dims, pf, nv));
-    if (batched_mode == 1) CHECK_HIP(launch_norm_codes(stream, dims.hidden, nv, pf.h, layers[0].ln_attn, dims.eps, mg));
+    if (batched_mode == 1)
+      CHECK_HIP(launch_norm_codes(stream, dims.hidden, nv, pf.h, layers[0].ln_attn, dims.eps, mg));
+    else
+      CHECK_HIP(launch_norm_b(stream, dims, pf, nv, layers[0].ln_attn));
     for (size_t l = 0; l < layers.size(); l++) {
+      const float* next = l + 1 < layers.size() ? layers[l + 1].ln_attn : nullptr;
       if (batched_mode == 1) {
         GroupBufs g = mg;
         g.gu = tiled[l].gu;
         g.dn = tiled[l].dn;
         g.qkv = tiled[l].qkv;
         g.oproj = tiled[l].o;
-        const float* next = l + 1 < layers.size() ? layers[l + 1].ln_attn : nullptr;
         CHECK_HIP(launch_layer_grouped(stream, layers[l], dims, pf, pf.pos0, pos0, nv, b.rope, g, next));
       } else {
-        CHECK_HIP(launch_layer_b(stream, layers[l], dims, pf, pf.pos0, pos0, nv, b.rope));
+        CHECK_HIP(launch_layer_b(stream, layers[l], dims, pf, pf.pos0, pos0, nv, b.rope, next));
       }
     }
     StepBufs bl = b;

@@ -1,22 +1,19 @@
-// Multi-position step of the whole model: m <= 32 consecutive positions in one pass per layer (the block prefill
-// `le_ids`, rust/moe-rt/src/motor/leitura.rs:79-85, through begin_step_tokens and the per-position loops of the model
-// step, cuda_backend.rs:499-516, 751-917). Every weight row is read from HBM once per block of positions and applied
-// to each position's activation with the decode kernels' per-row chain (chunk j of a row accumulated by lane
-// j % 64 as an fmaf chain, then the pairwise lane tree), so the step equals m single-position decode steps bit for
-// bit: the KV rows it appends, every hidden state and the last position's logits.
+// Multi-position step of the whole model: consecutive positions in one pass per layer (the block prefill `le_ids`,
+// rust/moe-rt/src/motor/leitura.rs:79-85, through begin_step_tokens and the per-position loops of the model step,
+// cuda_backend.rs:499-516, 751-917). Every weight row is read once per block of positions and applied to each
+// position's activation with the decode kernels' per-row chain (chunk j of a row accumulated by lane j % 64 as an
+// fmaf chain, then the pairwise lane tree), so the step equals single-position decode steps bit for bit: the KV rows
+// it appends, every hidden state and the last position's logits.
 //
-// Kernels per layer (one stream, in order):
-//   k_qkv_b        rmsnorm of each position, [q; k; v] rows of the layer once for all positions, RoPE at each
-//                  position, q to qb[v], k and v to row pos0 + v of the KV cache
-//   attention      the decode attention kernels over a grid of positions, position v attending to pos0 + v + 1
-//   k_oproj_b      output projection once for all positions, h[v] += res * (Wo att[v]); MoE-norm partials of each
-//                  position's new rows (moe_norm.h)
-//   k_route_b      per position: rmsnorm scale, router logits from the partials, top-k and weights (the decode
-//                  router); xn[v] kept
-//   k_moe_up_b     per routed expert: its gate/up rows once, applied to the positions routed to it; SwiGLU into
-//                  act[v][j] (j = the expert's top-k rank at position v)
-//   k_moe_down_b   per routed expert: its down rows once for its positions, o[v][j] = down . act[v][j]
-//   k_moe_comb_b   h[v] += res * sum over j in top-k order of w[v][j] * o[v][j]
+// Kernels per layer (one stream, in order; xn holds the normalised input of the layer on entry):
+//   k_qkv_x        [q; k; v] of every position, RoPE, q to qb[v], k and v to row pos0 + v of the KV cache
+//   attention      attn_mm.hip over the positions, position v attending to pos0 + v + 1, and the decode combine
+//   k_oproj_x      output projection, h[v] += res * (Wo att[v])
+//   k_route_x      per position: the MoE norm and router in moe_norm.h's order, top-k and weights; xn[v] for the
+//                  experts; the position enters its experts' member lists
+//   k_moe_up_x     per expert and tile of its members: gate/up rows, SwiGLU into act[slot] (slot = v * k + rank)
+//   k_moe_down_x   per expert and tile of its members: o[slot] = down . act[slot]
+//   k_moe_comb_x   h[v] += res * sum over j in top-k order of w[v][j] * o[v][j], and the next layer's xn[v]
 #include <algorithm>
 
 #include "cache.h"
@@ -28,484 +25,491 @@
 
 namespace moert {
 
-constexpr int kPfWaves = 8;           // waves per workgroup of the row kernels
-constexpr int kPfNT = kPfWaves * 64;
-constexpr int kPfGroup = 8;           // positions staged in LDS at a time (one per wave for the norms)
+// ------------------------------------------------------------------------------------------------------------
+// The row products on the f32 matrix cores. v_mfma_f32_16x16x1 is one fmaf on every element of four 16x16 blocks, so
+// the chain of decode lane c of a row is a run of MFMAs over its elements in index order, block b of the instruction
+// being lane 4G + b: A = element i of chunk 4G + b of 16 rows (a lane dequantises its row's chunk from one 16-byte
+// load, as a decode lane does), B = element i of that chunk of 16 positions' activations. The pairwise lane tree then
+// adds blocks (0 + 1) + (2 + 3) inside a lane, groups of four lanes after that.
+//
+// A workgroup holds MT x NT tiles of 16 rows x 16 positions. Its waves share the groups of four chains: wave w takes
+// the runs of SUB adjacent groups w, w + KW, ... (so that the chunks past the row's 64th, which only the first groups
+// have, spread over all waves), one tree node per run goes to LDS, and every thread adds the NN nodes of its outputs.
+// Bound: the matrix cores (127 TFLOP/s for this instruction on 256 CUs, 32 cycles for 1024 products) where the tiles
+// are full; a row's dequantisation, two vector instructions an element, serves NT tiles and hides behind them.
+typedef float xg_f16 __attribute__((ext_vector_type(16)));
 
-// The dequantised elements of P rows' chunks, formed once and used for every position: element i of a chunk is
-// q_i * d (f32 rows: the value itself), the same rounded product the decode chain forms before each fma.
-template <int DT, int K, int P>
-struct DeqRows {
-  float w[P][Geo<DT, K>::NJ][Fmt<DT>::kElems];
+template <int DT, int K>
+struct XGeo {
+  using G = Geo<DT, K>;
+  static constexpr int SE = G::CE < 16 ? G::CE : 16;  // elements of a step (Q4_0: two steps per chunk)
+  static constexpr int HPC = G::CE / SE;              // steps per chunk
+  static constexpr int NG = G::LPR / 4;               // groups of four chains
+  static constexpr int KW = NG < 4 ? NG : 4;          // waves
+  static constexpr int NT_ = KW * 64;                 // threads
+  // Every wave of a round has the chunks 4G + b + LPR * jj of its run, or none has.
+  static constexpr bool even(int sub) {
+    for (int r = 0; r < NG / (KW * sub); r++)
+      for (int jj = 0; jj < G::NJ; jj++) {
+        const int lo = 4 * r * KW * sub + G::LPR * jj, hi = 4 * (r + 1) * KW * sub + G::LPR * jj;
+        if (lo < G::NCH && hi > G::NCH) return false;
+      }
+    return true;
+  }
+  static constexpr int SUB = NG >= 2 * KW && even(2) ? 2 : 1;
+  static constexpr int ROUNDS = NG / (KW * SUB);
+  static constexpr int NN = NG / SUB;  // tree nodes of an output
+  static_assert(even(SUB), "a round's waves must have the same chunks");
+  static constexpr bool valid(int r, int jj) { return 4 * r * KW * SUB + G::LPR * jj < G::NCH; }
+  struct Step {
+    int r, u, jj, half;
+  };
+  static constexpr int steps() {
+    int n = 0;
+    for (int r = 0; r < ROUNDS; r++)
+      for (int jj = 0; jj < G::NJ; jj++) n += valid(r, jj) ? SUB * HPC : 0;
+    return n;
+  }
+  static constexpr int N = steps();
+  static constexpr Step step(int s) {
+    int n = 0;
+    for (int r = 0; r < ROUNDS; r++)
+      for (int u = 0; u < SUB; u++)
+        for (int jj = 0; jj < G::NJ; jj++)
+          for (int h = 0; h < HPC; h++)
+            if (valid(r, jj) && n++ == s) return Step{r, u, jj, h};
+    return Step{-1, -1, -1, -1};
+  }
 };
 
-template <int DT, int K, int P>
-__device__ __forceinline__ void deq_rows(const Rows<DT, K, P>& r, DeqRows<DT, K, P>& w) {
-  using G = Geo<DT, K>;
-#pragma unroll
-  for (int p = 0; p < P; p++)
-#pragma unroll
-    for (int jj = 0; jj < G::NJ; jj++)
-#pragma unroll
-      for (int i = 0; i < Fmt<DT>::kElems; i++) w.w[p][jj][i] = chunk_elem<DT>(r.c[p][jj], i);
-}
-
-// rows_fma over dequantised rows: per row, the lane's fma chain over its chunks' elements in index order, then the
-// tree over the row's lanes (the decode kernels' dot, fma_chunk + group_sum, bit for bit).
-template <int DT, int K, int P>
-__device__ __forceinline__ void deq_fma(const DeqRows<DT, K, P>& w, const bool (&ok)[P], const XReg<DT, K>& xr,
-                                        int sub, float (&out)[P]) {
-  using G = Geo<DT, K>;
-#pragma unroll
-  for (int p = 0; p < P; p++) {
-    float acc = 0.0f;
-#pragma unroll
-    for (int jj = 0; jj < G::NJ; jj++) {
-      const int j = sub + G::LPR * jj;
-      if (ok[p] && j < G::NCH)
-#pragma unroll
-        for (int i = 0; i < Fmt<DT>::kElems; i++) acc = __builtin_fmaf(w.w[p][jj][i], xr.v[jj][i], acc);
-    }
-    out[p] = group_sum<G::LPR>(acc);
-  }
-}
-
-// LDS layout of a staged activation row. Lane `sub` of a row reads whole weight chunks of x (16 floats for Q8_0,
-// 32 for Q4_0), so in a plain layout the lanes' 16-byte reads are 64 or 128 bytes apart and fall in the same banks.
-// The float4 slots of chunk j are therefore stored with their index xor-ed by sw(j) (slot q of chunk j at
-// NQ j + (q ^ sw(j))), which spreads the 8 or 16 lanes one LDS pass serves over distinct bank groups (32 or 64
-// banks). The values and the order they are used in do not change.
+// Element i of a chunk whose payload words and scale are in registers: q * d, exact, as fma_chunk forms it.
 template <int DT>
-__device__ __forceinline__ int xslot(int s) {
-  constexpr int NQ = Fmt<DT>::kElems / 4;  // float4 slots per chunk
-  if constexpr (NQ == 1) {
-    return s;
+__device__ __forceinline__ float xg_elem(const uint4& v, float d, int i) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  if (DT == DT_Q8_0) return (float)(int8_t)(w[i >> 2] >> (8 * (i & 3))) * d;
+  if (DT == DT_Q4_0) {
+    const int b = i & 15;
+    return (float)((int)((w[b >> 2] >> (8 * (b & 3) + (i >= 16 ? 4 : 0))) & 15u) - 8) * d;
+  }
+  return __uint_as_float(w[i]);
+}
+
+template <int DT, int K, int MT, int NT>
+struct XgRegs {
+  RawChunk a[2][MT];
+  float4 b[2][NT][XGeo<DT, K>::SE / 4];
+  xg_f16 acc[MT][NT];
+  float node[MT][NT][4];
+};
+
+template <int DT, int K, int MT, int NT, int S>
+__device__ __forceinline__ void xg_load(XgRegs<DT, K, MT, NT>& x, const DMat& m, const size_t (&row)[MT],
+                                        const float* const (&xp)[NT], int w, int gq) {
+  using X = XGeo<DT, K>;
+  using G = Geo<DT, K>;
+  constexpr typename X::Step st = X::step(S);
+  const int j = 4 * ((st.r * X::KW + w) * X::SUB + st.u) + gq + G::LPR * st.jj;
+  if constexpr (st.half == 0) {
+#pragma unroll
+    for (int t = 0; t < MT; t++) x.a[S / X::HPC & 1][t] = load_chunk<DT>(m, row[t], j);
+  }
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int e = 0; e < X::SE / 4; e++) x.b[S & 1][t][e] = gload_f4(xp[t] + j * G::CE + st.half * X::SE + 4 * e);
+}
+
+template <int DT, int K, int MT, int NT, int S>
+__device__ __forceinline__ void xg_steps(XgRegs<DT, K, MT, NT>& x, const DMat& m, const size_t (&row)[MT],
+                                         const float* const (&xp)[NT], float* nodes, int lane, int w) {
+  using X = XGeo<DT, K>;
+  if constexpr (S < X::N) {
+    constexpr typename X::Step st = X::step(S), nx = X::step(S + 1);
+    constexpr bool first = st.jj == 0 && st.half == 0;                          // of its group
+    constexpr bool last = S + 1 == X::N || nx.r != st.r || nx.u != st.u;        // of its group
+    if constexpr (S + 1 < X::N) {
+      xg_load<DT, K, MT, NT, S + 1>(x, m, row, xp, w, lane >> 4);
+      __builtin_amdgcn_sched_barrier(0);  // the next step's loads ahead of this step's products
+    }
+    if constexpr (first) {
+#pragma unroll
+      for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int n = 0; n < NT; n++) x.acc[t][n] = xg_f16{};
+    }
+    float d[MT];
+#pragma unroll
+    for (int t = 0; t < MT; t++) d[t] = chunk_scale(x.a[S / X::HPC & 1][t]);
+#pragma unroll
+    for (int i = 0; i < X::SE; i++) {
+      float av[MT];
+#pragma unroll
+      for (int t = 0; t < MT; t++) av[t] = xg_elem<DT>(x.a[S / X::HPC & 1][t].v, d[t], st.half * X::SE + i);
+#pragma unroll
+      for (int n = 0; n < NT; n++) {
+        const float4 q = x.b[S & 1][n][i >> 2];
+        const float bv = (i & 3) == 0 ? q.x : (i & 3) == 1 ? q.y : (i & 3) == 2 ? q.z : q.w;
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+          x.acc[t][n] = __builtin_amdgcn_mfma_f32_16x16x1f32(av[t], bv, x.acc[t][n], 0, 0, 0);
+      }
+    }
+    if constexpr (last) {
+#pragma unroll
+      for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const xg_f16& c = x.acc[t][n];
+            const float f = (c[r] + c[4 + r]) + (c[8 + r] + c[12 + r]);
+            x.node[t][n][r] = st.u == 0 ? f : x.node[t][n][r] + f;
+            if (st.u == X::SUB - 1) nodes[(((st.r * X::KW + w) * MT + t) * NT + n) * 256 + 64 * r + lane] = x.node[t][n][r];
+          }
+    }
+    xg_steps<DT, K, MT, NT, S + 1>(x, m, row, xp, nodes, lane, w);
+  }
+}
+
+// The balanced pairwise tree over n nodes `stride` floats apart.
+template <int N>
+__device__ __forceinline__ float xg_tree(const float* p, int stride) {
+  if constexpr (N == 1) {
+    return p[0];
   } else {
-    const int j = s / NQ, q = s % NQ;
-    const int sw = NQ == 4 ? ((j >> 1) ^ (j >> 3)) & 3 : (j ^ (j >> 3)) & 7;
-    return NQ * j + (q ^ sw);
+    return xg_tree<N / 2>(p, stride) + xg_tree<N / 2>(p + N / 2 * stride, stride);
   }
 }
 
-// load_x over a row staged with xslot.
-template <int DT, int K>
-__device__ __forceinline__ void load_xs(XReg<DT, K>& xr, const float* x, int sub) {
-  using G = Geo<DT, K>;
-  constexpr int NQ = G::CE / 4;
-  const float4* x4 = reinterpret_cast<const float4*>(x);
+// Floats of LDS for the nodes of MT x NT tiles.
+template <int DT, int K, int MT, int NT>
+__host__ __device__ constexpr int xg_lds() {
+  return XGeo<DT, K>::NN * MT * NT * 256;
+}
+
+// MT x NT tiles: lane i = lane % 16 supplies rows row[t] (one of the 16 of tile t) and the activations at xp[n] (one
+// of the 16 positions of tile n). done(n, r, v) is called for every output of this thread: v[t] is row 4 (lane / 16)
+// + r of tile t against position lane % 16 of tile n.
+template <int DT, int K, int MT, int NT, class F>
+__device__ __forceinline__ void xg_run(const DMat& m, const size_t (&row)[MT], const float* const (&xp)[NT],
+                                       float* nodes, int lane, int w, const F& done) {
+  using X = XGeo<DT, K>;
+  XgRegs<DT, K, MT, NT> x;
+  xg_load<DT, K, MT, NT, 0>(x, m, row, xp, w, lane >> 4);
+  xg_steps<DT, K, MT, NT, 0>(x, m, row, xp, nodes, lane, w);
+  // runs without a chunk (a row that does not reach all 64 lanes) add +0
 #pragma unroll
-  for (int jj = 0; jj < G::NJ; jj++) {
-    const int j = sub + G::LPR * jj;
-    if (j < G::NCH) {
+  for (int r = 0; r < X::ROUNDS; r++)
+    if constexpr (!X::valid(X::ROUNDS - 1, 0)) {
+      if (!X::valid(r, 0))
 #pragma unroll
-      for (int e = 0; e < NQ; e++) {
-        const float4 t = x4[xslot<DT>(NQ * j + e)];
-        xr.v[jj][4 * e] = t.x;
-        xr.v[jj][4 * e + 1] = t.y;
-        xr.v[jj][4 * e + 2] = t.z;
-        xr.v[jj][4 * e + 3] = t.w;
-      }
+        for (int t = 0; t < MT * NT * 4; t++) nodes[(r * X::KW + w) * MT * NT * 256 + 64 * t + lane] = 0.0f;
     }
-  }
-}
-
-// Canonical rmsnorm scale of the K floats at x (LDS, staged with xslot): the sum of squares over 16-element chunks,
-// chunk j in lane j % 64, then the lane tree; r = 1 / sqrt(ss / K + eps). One wave.
-template <int DT, int K>
-__device__ __forceinline__ float wave_rms(const float* x, float eps, int lane) {
-  constexpr int NCH = K / 16;
-  const float4* x4 = reinterpret_cast<const float4*>(x);
-  float acc = 0.0f;
-#pragma unroll
-  for (int jj = 0; jj < (NCH + 63) / 64; jj++) {
-    const int j = lane + 64 * jj;
-    if (j < NCH) {
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const float4 t = x4[xslot<DT>(4 * j + e)];
-        acc = __builtin_fmaf(t.x, t.x, acc);
-        acc = __builtin_fmaf(t.y, t.y, acc);
-        acc = __builtin_fmaf(t.z, t.z, acc);
-        acc = __builtin_fmaf(t.w, t.w, acc);
-      }
-    }
-  }
-  const float ss = group_sum<64>(acc);
-  return 1.0f / sqrtf(ss / (float)K + eps);
-}
-
-// Stages positions [v0, v0 + n) of x ([*, K] rows, global) into xs ([kPfGroup][K], LDS, layout xslot); with lnw,
-// each is then normalised in place: xs = lnw * (x * r) (wave w normalises position w of the group). Ends with a
-// barrier.
-template <int DT, int K>
-__device__ __forceinline__ void stage_group(const float* __restrict__ x, int v0, int n, const float* __restrict__ lnw,
-                                            float eps, float (*xs)[K], float* rsv) {
-  constexpr int K4 = K / 4;
-  const float4* src = reinterpret_cast<const float4*>(x + (size_t)v0 * K);
-  for (int i = threadIdx.x; i < n * K4; i += kPfNT)
-    reinterpret_cast<float4*>(&xs[i / K4][0])[xslot<DT>(i % K4)] = src[i];
   __syncthreads();
-  if (!lnw) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (wave < n) {
-    const float r = wave_rms<DT, K>(&xs[wave][0], eps, lane);
-    if (lane == 0) rsv[wave] = r;
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < n * K4; i += kPfNT) {
-    const int v = i / K4, s = i % K4;
-    float4* p = reinterpret_cast<float4*>(&xs[v][0]) + xslot<DT>(s);
-    const float4 w = reinterpret_cast<const float4*>(lnw)[s];
-    const float r = rsv[v];
-    float4 t = *p;
-    t.x = w.x * (t.x * r);
-    t.y = w.y * (t.y * r);
-    t.z = w.z * (t.z * r);
-    t.w = w.w * (t.w * r);
-    *p = t;
-  }
-  __syncthreads();
-}
-
-// ------------------------------------------------------------------------------------------------------------
-// rmsnorm -> [q; k; v] -> RoPE -> q / KV cache, for positions pos0 .. pos0 + nv - 1 (k_qkv's arithmetic per
-// position). A wave owns NP row pairs (j, j + 32) of a head, as in k_qkv.
-template <int DT, int K, int NP>
-__global__ __launch_bounds__(kPfNT) void k_qkv_b(DMat m, const float* __restrict__ h, const float* __restrict__ lnw,
-                                                 float eps, int pos0, int nv, const float* __restrict__ rope,
-                                                 int heads, int kvh, int max_len, float* __restrict__ q,
-                                                 uint16_t* __restrict__ kc, uint16_t* __restrict__ vc) {
-  using G = Geo<DT, K>;
-  constexpr int P = 2 * NP;
-  __shared__ __align__(16) float xs[kPfGroup][K];
-  __shared__ float csv[kPfGroup][64];
-  __shared__ float rsv[kPfGroup];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int sub = lane % G::LPR, rw = lane / G::LPR;
-  const int npairs = m.rows / 2;
-  const int wbase = (blockIdx.x * kPfWaves + wave) * (NP * G::RPW);
-  size_t row[P];
-  bool ok[P];
-  int gp[NP];
+  constexpr int RPT = NT * 4 / X::KW;  // outputs of a thread: (n, r) = its RPT consecutive of NT x 4
 #pragma unroll
-  for (int a = 0; a < NP; a++) {
-    gp[a] = wbase + a * G::RPW + rw;
-    const bool v = gp[a] < npairs;
-    const int head = gp[a] / 32, jp = gp[a] % 32;
-    row[2 * a] = (size_t)head * 64 + jp;
-    row[2 * a + 1] = row[2 * a] + 32;
-    ok[2 * a] = ok[2 * a + 1] = v;
-  }
-  Rows<DT, K, P> rr;
-  rows_load<DT, K, P>(rr, m, row, ok, sub);
-  DeqRows<DT, K, P> dw;
-  deq_rows<DT, K, P>(rr, dw);
-  const int qd = heads * 64;
-  for (int v0 = 0; v0 < nv; v0 += kPfGroup) {
-    const int n = min(kPfGroup, nv - v0);
-    __syncthreads();  // the previous group's activations are no longer read
-    for (int i = threadIdx.x; i < n * 64; i += kPfNT) csv[i / 64][i % 64] = rope[(size_t)(pos0 + v0 + i / 64) * 64 + i % 64];
-    stage_group<DT, K>(h, v0, n, lnw, eps, xs, rsv);
-    for (int v = 0; v < n; v++) {
-      XReg<DT, K> xr;
-      load_xs<DT, K>(xr, &xs[v][0], sub);
-      float out[P];
-      deq_fma<DT, K, P>(dw, ok, xr, sub, out);
-      if (sub != 0) continue;
-      const int pos = pos0 + v0 + v;
+  for (int e = 0; e < RPT; e++) {
+    const int it = w * RPT + e;
+    float v[MT];
 #pragma unroll
-      for (int a = 0; a < NP; a++) {
-        if (!ok[2 * a]) continue;
-        const int head = gp[a] / 32, jp = gp[a] % 32;
-        const float x1 = out[2 * a], x2 = out[2 * a + 1];
-        const float c = csv[v][jp], sn = csv[v][32 + jp];
-        if (head < heads) {
-          float* qv = q + (size_t)(v0 + v) * qd;
-          qv[head * 64 + jp] = x1 * c - x2 * sn;
-          qv[head * 64 + jp + 32] = x2 * c + x1 * sn;
-        } else if (head < heads + kvh) {
-          uint16_t* kp = kc + ((size_t)(head - heads) * max_len + pos) * 64;
-          kp[jp] = f2h(x1 * c - x2 * sn);
-          kp[jp + 32] = f2h(x2 * c + x1 * sn);
-        } else {
-          uint16_t* vp = vc + ((size_t)(head - heads - kvh) * max_len + pos) * 64;
-          vp[jp] = f2h(x1);
-          vp[jp + 32] = f2h(x2);
-        }
-      }
-    }
+    for (int t = 0; t < MT; t++) v[t] = xg_tree<X::NN>(nodes + t * NT * 256 + it * 64 + lane, MT * NT * 256);
+    done(it >> 2, it & 3, v);
   }
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// h[v][r] = h[v][r] + res * (Wo att[v])[r] for every position v (k_oproj's arithmetic per position), then the
-// MoE-norm partials of each position's new rows into zp + v * kNormItems (k_oproj's epilogue per position).
-template <int DT, int K, int P>
-__global__ __launch_bounds__(kPfNT) void k_oproj_b(DMat m, const float* __restrict__ att, int nv, float res,
-                                                   float* __restrict__ h, DMat router, const float* __restrict__ lnw,
-                                                   float* __restrict__ zp) {
-  using G = Geo<DT, K>;
-  constexpr int RB = kPfWaves * P * G::RPW;  // rows of the workgroup: [r0, r0 + RB)
-  static_assert(RB % kNormBlk == 0, "the workgroup's rows must be whole partial blocks");
-  __shared__ __align__(16) float xs[kPfGroup][K];
-  __shared__ float hn[kPfGroup][RB];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int sub = lane % G::LPR, rw = lane / G::LPR;
-  const int r0 = blockIdx.x * RB;
-  const size_t base = ((size_t)blockIdx.x * kPfWaves + wave) * (P * G::RPW);
-  size_t row[P];
-  bool ok[P];
+// [q; k; v] rows (j, j + 32) of a head (tile pair 16 a .. +16 and 32 + 16 a .. +16) for NT tiles of positions, RoPE,
+// q and the KV rows (k_qkv's arithmetic per position). The first workgroup also empties the experts' member lists.
+template <int DT, int K, int NT>
+__global__ __launch_bounds__((XGeo<DT, K>::NT_), 2) void k_qkv_x(DMat m, const float* __restrict__ xn, int pos0, int nv,
+                                                               const float* __restrict__ rope, int heads, int kvh,
+                                                               int max_len, float* __restrict__ q,
+                                                               uint16_t* __restrict__ kc, uint16_t* __restrict__ vc,
+                                                               int* __restrict__ cnt) {
+  __shared__ float nodes[xg_lds<DT, K, 2, NT>()];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15;
+  const int head = blockIdx.x >> 1, a16 = 16 * (blockIdx.x & 1), p0 = blockIdx.y * 16 * NT;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 64) cnt[threadIdx.x] = 0;
+  const size_t row[2] = {(size_t)head * 64 + a16 + i, (size_t)head * 64 + a16 + i + 32};
+  const float* xp[NT];
 #pragma unroll
-  for (int p = 0; p < P; p++) {
-    row[p] = base + (size_t)p * G::RPW + rw;
-    ok[p] = row[p] < (size_t)m.rows;
-  }
-  Rows<DT, K, P> rr;
-  rows_load<DT, K, P>(rr, m, row, ok, sub);
-  __builtin_amdgcn_sched_barrier(0);
-  NormPart<RB, kPfNT> np;
-  norm_part_fetch<DT, RB, kPfNT>(router, lnw, r0, m.rows, np);
-  DeqRows<DT, K, P> dw;
-  deq_rows<DT, K, P>(rr, dw);
-  const int H = m.rows;
-  for (int v0 = 0; v0 < nv; v0 += kPfGroup) {
-    const int n = min(kPfGroup, nv - v0);
-    __syncthreads();
-    stage_group<DT, K>(att, v0, n, nullptr, 0.0f, xs, nullptr);
-    for (int v = 0; v < n; v++) {
-      XReg<DT, K> xr;
-      load_xs<DT, K>(xr, &xs[v][0], sub);
-      float out[P];
-      deq_fma<DT, K, P>(dw, ok, xr, sub, out);
-      if (sub != 0) continue;
-      float* hv = h + (size_t)(v0 + v) * H;
-#pragma unroll
-      for (int p = 0; p < P; p++)
-        if (ok[p]) {
-          const float hold = hv[row[p]];
-          const float hnew = hold + res * out[p];
-          hv[row[p]] = hnew;
-          hn[v][row[p] - r0] = hnew;
-        }
+  for (int n = 0; n < NT; n++) xp[n] = xn + (size_t)min(p0 + 16 * n + i, nv - 1) * K;
+  xg_run<DT, K, 2, NT>(m, row, xp, nodes, lane, w, [&](int n, int r, const float (&v)[2]) {
+    const int p = p0 + 16 * n + i, jp = a16 + 4 * (lane >> 4) + r;
+    if (p >= nv) return;
+    const int pos = pos0 + p;
+    const float x1 = v[0], x2 = v[1], c = rope[(size_t)pos * 64 + jp], sn = rope[(size_t)pos * 64 + 32 + jp];
+    if (head < heads) {
+      float* qv = q + ((size_t)p * heads + head) * 64;
+      qv[jp] = x1 * c - x2 * sn;
+      qv[jp + 32] = x2 * c + x1 * sn;
+    } else if (head < heads + kvh) {
+      uint16_t* kp = kc + ((size_t)(head - heads) * max_len + pos) * 64;
+      kp[jp] = f2h(x1 * c - x2 * sn);
+      kp[jp + 32] = f2h(x2 * c + x1 * sn);
+    } else {
+      uint16_t* vp = vc + ((size_t)(head - heads - kvh) * max_len + pos) * 64;
+      vp[jp] = f2h(x1);
+      vp[jp + 32] = f2h(x2);
     }
-    __syncthreads();
-    for (int v = 0; v < n; v++)
-      norm_part_finish<DT, RB, kPfNT>(np, &hn[v][0], router.rows, r0, H, zp + (size_t)(v0 + v) * kNormItems);
-  }
+  });
+}
+
+// h[v][r] = h[v][r] + res * (Wo att[v])[r] for 32 rows and NT tiles of positions (k_oproj's arithmetic per position).
+template <int DT, int K, int NT>
+__global__ __launch_bounds__((XGeo<DT, K>::NT_), 2) void k_oproj_x(DMat m, const float* __restrict__ att, int nv,
+                                                                 float res, float* __restrict__ h) {
+  __shared__ float nodes[xg_lds<DT, K, 2, NT>()];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15;
+  const int r0 = blockIdx.x * 32, p0 = blockIdx.y * 16 * NT, H = m.rows;
+  const size_t row[2] = {(size_t)r0 + i, (size_t)r0 + 16 + i};
+  const float* xp[NT];
+#pragma unroll
+  for (int n = 0; n < NT; n++) xp[n] = att + (size_t)min(p0 + 16 * n + i, nv - 1) * K;
+  xg_run<DT, K, 2, NT>(m, row, xp, nodes, lane, w, [&](int n, int r, const float (&v)[2]) {
+    const int p = p0 + 16 * n + i;
+    if (p >= nv) return;
+    float* hv = h + (size_t)p * H + r0 + 4 * (lane >> 4) + r;
+    const float h0 = hv[0], h1 = hv[16];
+    hv[0] = h0 + res * v[0];
+    hv[16] = h1 + res * v[1];
+  });
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// Router of position v = blockIdx.x: xn = rmsnorm(h[v]) (kept in xn[v] for the experts), logits = Wr xn (+ bias),
-// ranks, ids and weights in top-k order (k_route_up's router, arithmetic for arithmetic).
+// Position v = blockIdx.x: the MoE norm and the router in moe_norm.h's order. A wave takes whole experts (the last
+// item is the sum of squares): lane l forms the 8-column chains of blocks l, l + 64, .. itself and adds them in that
+// order, so no partials pass through memory. Then ranks, ids and weights in top-k order (the decode router), xn for
+// the experts, and slot v * k + rank into the member list of each expert chosen (the order of a list does not enter
+// any result: every member is a column of its own).
 // 16 waves, 8 for f32 rows (whose registers would not fit 16), as k_route_up
-__host__ __device__ constexpr int route_b_waves(int dt) { return dt == DT_F32 ? 8 : 16; }
+__host__ __device__ constexpr int route_x_waves(int dt) { return dt == DT_F32 ? 8 : 16; }
 
 template <int DT, int K>
-__global__ __launch_bounds__(route_b_waves(DT) * 64) void k_route_b(DMat router, const float* __restrict__ bias,
-                                                               const float* __restrict__ h,
-                                                               const float* __restrict__ lnw, float eps,
-                                                               const float* __restrict__ zp, int k,
-                                                               float* __restrict__ xn, int* __restrict__ ids,
-                                                               float* __restrict__ wts) {
-  constexpr int NW = route_b_waves(DT), NT = NW * 64;
-  constexpr int IPW = (64 + NW - 1) / NW;  // router items per wave
-  constexpr int XP = (K + NT - 1) / NT;    // elements of h per thread
+__global__ __launch_bounds__(route_x_waves(DT) * 64) void k_route_x(DMat router, const float* __restrict__ bias,
+                                                                  const float* __restrict__ h,
+                                                                  const float* __restrict__ lnw, float eps, int k,
+                                                                  int cap, float* __restrict__ xn,
+                                                                  float* __restrict__ wts, int* __restrict__ cnt,
+                                                                  int* __restrict__ list) {
+  constexpr int NW = route_x_waves(DT), NT = NW * 64;
+  constexpr int NB = K / kNormBlk, NQ = (NB + 63) / 64;  // column blocks, and those of a lane
+  constexpr int IPW = (65 + NW - 1) / NW;                // items of a wave
+  constexpr int XP = (K + NT - 1) / NT;                  // elements of xn per thread
   __shared__ __align__(16) float lg[64];
   __shared__ int part[NW][64];
+  __shared__ float rs;
+  __shared__ int sid[8];
   const int v = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int E = router.rows, nb = K / kNormBlk;
-  zp += (size_t)v * kNormItems;
-  NormItem ssi, it[IPW];
-  float bv[IPW], hv[XP], wv[XP];
-  norm_item_fetch(zp, E, lane, ssi);
+  const int E = router.rows;
+  const float* hv = h + (size_t)v * K;
+  float hb[NQ][8], ub[NQ][8];
 #pragma unroll
-  for (int i = 0; i < IPW; i++) {
-    const int e = wave + i * NW, ec = e < E ? e : 0;
-    norm_item_fetch(zp, ec, lane, it[i]);
-    bv[i] = bias ? bias[ec] : 0.0f;
-  }
+  for (int q = 0; q < NQ; q++) {
+    const int c0 = kNormBlk * min(lane + 64 * q, NB - 1);
+    const float4 a = gload_f4(hv + c0), b = gload_f4(hv + c0 + 4), la = gload_f4(lnw + c0), lb = gload_f4(lnw + c0 + 4);
+    const float ha[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}, lw[8] = {la.x, la.y, la.z, la.w, lb.x, lb.y, lb.z, lb.w};
 #pragma unroll
-  for (int e = 0; e < XP; e++) {
-    const int i = threadIdx.x + e * NT, ic = i < K ? i : 0;
-    hv[e] = h[(size_t)v * K + ic];
-    wv[e] = lnw[ic];
-  }
-  const float ss = norm_item_sum(ssi, nb, lane);
-  const float r = 1.0f / sqrtf(ss / (float)K + eps);
-#pragma unroll
-  for (int i = 0; i < IPW; i++) {
-    const int e = wave + i * NW;
-    if (e < E) {
-      const float z = norm_item_sum(it[i], nb, lane);
-      if (lane == 0) lg[e] = bias ? z * r + bv[i] : z * r;
+    for (int t = 0; t < 8; t++) {
+      hb[q][t] = ha[t];
+      ub[q][t] = lw[t] * ha[t];
     }
+  }
+  // item E (the sum of squares) is wave 0's first, so that r is known when the experts' sums are
+  float z[IPW];
+#pragma unroll
+  for (int it = 0; it < IPW; it++) {
+    const int item = wave + NW * it, e = item == 0 ? E : item - 1;
+    float acc = 0.0f;
+    if (e < E) {
+      Col8 c[NQ];
+#pragma unroll
+      for (int q = 0; q < NQ; q++) c[q] = load_col8<DT>(router, e, kNormBlk * min(lane + 64 * q, NB - 1));
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        const int c0 = kNormBlk * min(lane + 64 * q, NB - 1);
+        float a = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 8; t++) a = __builtin_fmaf(col8_elem<DT>(c[q], t, c0), ub[q][t], a);
+        if (lane + 64 * q < NB) acc = acc + a;
+      }
+    } else if (item == 0) {
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        float a = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 8; t++) a = __builtin_fmaf(hb[q][t], hb[q][t], a);
+        if (lane + 64 * q < NB) acc = acc + a;
+      }
+    }
+    z[it] = group_sum<64>(acc);
+  }
+  if (threadIdx.x == 0) rs = 1.0f / sqrtf(z[0] / (float)K + eps);
+  __syncthreads();
+  const float r = rs;
+#pragma unroll
+  for (int it = 0; it < IPW; it++) {
+    const int item = wave + NW * it, e = item - 1;
+    if (item > 0 && e < E && lane == 0) lg[e] = bias ? z[it] * r + bias[e] : z[it] * r;
   }
 #pragma unroll
   for (int e = 0; e < XP; e++) {
     const int i = threadIdx.x + e * NT;
-    if (i < K) xn[(size_t)v * K + i] = wv[e] * (hv[e] * r);
+    if (i < K) xn[(size_t)v * K + i] = lnw[i] * (hv[i] * r);
   }
   __syncthreads();
   int eid[8];
   const int rank = wg_rank<NW>(lg, E, lane, wave, part);
   const bool sel = lane < E && rank < k;
   ids_by_rank(sel, rank, k, eid);
-  if (wave == 0) route_weights(lg, sel, rank, k, lane, eid, ids + (size_t)v * k, wts + (size_t)v * k);
+  if (wave == 0) {
+    route_weights(lg, sel, rank, k, lane, eid, sid, wts + (size_t)v * k);
+    if (sel) list[(size_t)lane * cap + atomicAdd(&cnt[lane], 1)] = v * k + rank;
+  }
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// The experts routed by the nv positions, in LDS: the u-th expert of the step is the u-th set bit of the used mask
-// (ascending expert index; the order of the experts does not enter any sum, each position's combine runs in its
-// own top-k order). For expert e: the positions routed to it (bit mask) and, per position, the top-k rank of e.
-struct PfPlan {
-  unsigned bits[64];          // positions routed to expert e
-  unsigned long long used;    // experts routed by any position
-  signed char rank[64][kPfMaxPos];  // top-k rank of expert e at position v
-};
-
-__device__ __forceinline__ void pf_plan(const int* __restrict__ ids, int nv, int k, PfPlan& pl) {
-  const int t = threadIdx.x, n = nv * k;
-  if (t < 64) pl.bits[t] = 0u;
-  __syncthreads();
-  int e = 0;
-  if (t < n) {
-    e = ids[t];
-    atomicOr(&pl.bits[e], 1u << (t / k));
-    pl.rank[e][t / k] = (signed char)(t % k);
+// The tile-th tile of NP members over the experts in order: expert and first member, or expert -1 past the last.
+// Every wave computes it from the 64 member counts.
+template <int NP>
+__device__ __forceinline__ int member_tile(const int* __restrict__ cnt, int tile, int lane, int* first, int* members) {
+  const int c = cnt[lane], t = (c + NP - 1) / NP;
+  int sum = t;
+#pragma unroll
+  for (int s = 1; s < 64; s <<= 1) {
+    const int o = __shfl_up(sum, s);
+    sum += lane >= s ? o : 0;
   }
-  __syncthreads();
-  if (t < 64) {
-    const unsigned long long b = __ballot(pl.bits[t] != 0u);
-    if (t == 0) pl.used = b;
-  }
-  __syncthreads();
+  const unsigned long long hit = __ballot(tile >= sum - t && tile < sum);
+  if (!hit) return -1;
+  const int e = __ffsll((long long)hit) - 1;
+  *members = __builtin_amdgcn_readlane(c, e);
+  *first = (tile - __builtin_amdgcn_readlane(sum - t, e)) * NP;
+  return e;
 }
 
-__device__ __forceinline__ int nth_bit64(unsigned long long b, int u) {
-  for (int i = 0; i < u; i++) b &= b - 1ull;
-  return b ? __ffsll((long long)b) - 1 : -1;
-}
-
-// Gate/up of the u-th routed expert (u = blockIdx.y) for the positions routed to it: rows (r, I + r) of the
-// expert for the workgroup's pairs, act[v][j][r] = silu(gate_r . xn[v]) * (up_r . xn[v]) with j the expert's
-// rank at v (k_route_up's expert arithmetic per position).
-template <int DT, int K, int NP>
-__global__ __launch_bounds__(kPfNT) void k_moe_up_b(DMat gu, const float* __restrict__ xn, const int* __restrict__ ids,
-                                                    int nv, int k, int inter, float* __restrict__ act) {
-  using G = Geo<DT, K>;
-  constexpr int P = 2 * NP;
-  __shared__ PfPlan pl;
-  __shared__ __align__(16) float xs[kPfGroup][K];
-  pf_plan(ids, nv, k, pl);
-  const int e = nth_bit64(pl.used, blockIdx.y);
+// Gate/up rows (16 of each) of one expert for a tile of its members: act[slot][r] = silu(gate_r . xn) * (up_r . xn)
+// (k_route_up's expert arithmetic per position). A last tile of at most 16 members runs as one position tile.
+template <int DT, int K, int NT>
+__global__ __launch_bounds__((XGeo<DT, K>::NT_), 2) void k_moe_up_x(DMat gu, const float* __restrict__ xn,
+                                                                  const int* __restrict__ cnt,
+                                                                  const int* __restrict__ list, int cap, int k,
+                                                                  int inter, float* __restrict__ act) {
+  __shared__ float nodes[xg_lds<DT, K, 2, NT>()];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15;
+  int first = 0, members = 0;
+  const int e = member_tile<16 * NT>(cnt, blockIdx.y, lane, &first, &members);
   if (e < 0) return;
-  const unsigned members = pl.bits[e];
-  const int ne = __popc(members);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int sub = lane % G::LPR, rw = lane / G::LPR;
-  const int wbase = (blockIdx.x * kPfWaves + wave) * (NP * G::RPW);
-  size_t row[P];
-  bool ok[P];
-  int rr_[NP];
+  const int r0 = blockIdx.x * 16;
+  const size_t row[2] = {(size_t)e * 2 * inter + r0 + i, (size_t)e * 2 * inter + inter + r0 + i};
+  const float* xp[NT];
+  int slot[NT];
 #pragma unroll
-  for (int a = 0; a < NP; a++) {
-    rr_[a] = wbase + a * G::RPW + rw;
-    const bool v = rr_[a] < inter;
-    row[2 * a] = (size_t)e * 2 * inter + (v ? rr_[a] : 0);
-    row[2 * a + 1] = row[2 * a] + inter;
-    ok[2 * a] = ok[2 * a + 1] = v;
+  for (int n = 0; n < NT; n++) {
+    slot[n] = list[(size_t)e * cap + min(first + 16 * n + i, members - 1)];
+    xp[n] = xn + (size_t)(slot[n] / k) * K;
   }
-  Rows<DT, K, P> rr;
-  rows_load<DT, K, P>(rr, gu, row, ok, sub);
-  DeqRows<DT, K, P> dw;
-  deq_rows<DT, K, P>(rr, dw);
-  for (int c0 = 0; c0 < ne; c0 += kPfGroup) {
-    const int n = min(kPfGroup, ne - c0);
-    __syncthreads();
-    // members c0 .. c0 + n - 1 (the set bits of `members` in ascending position order) into LDS
-    for (int i = threadIdx.x; i < n * K / 4; i += kPfNT) {
-      const int c = i / (K / 4), w4 = i % (K / 4);
-      const int vpos = nth_bit64(members, c0 + c);
-      reinterpret_cast<float4*>(&xs[c][0])[xslot<DT>(w4)] = reinterpret_cast<const float4*>(xn + (size_t)vpos * K)[w4];
-    }
-    __syncthreads();
-    for (int c = 0; c < n; c++) {
-      XReg<DT, K> xr;
-      load_xs<DT, K>(xr, &xs[c][0], sub);
-      float out[P];
-      deq_fma<DT, K, P>(dw, ok, xr, sub, out);
-      if (sub != 0) continue;
-      const int vpos = nth_bit64(members, c0 + c);
-      float* av = act + ((size_t)vpos * k + pl.rank[e][vpos]) * inter;
-#pragma unroll
-      for (int a = 0; a < NP; a++)
-        if (ok[2 * a]) av[rr_[a]] = silu_mul(out[2 * a], out[2 * a + 1]);
-    }
+  auto done = [&](int n, int r, const float (&v)[2]) {
+    if (first + 16 * n + i >= members) return;
+    const int sl = NT == 1 || n == 0 ? slot[0] : slot[NT - 1];
+    act[(size_t)sl * inter + r0 + 4 * (lane >> 4) + r] = silu_mul(v[0], v[1]);
+  };
+  if (NT == 2 && first + 16 >= members) {
+    const float* const x1[1] = {xp[0]};
+    xg_run<DT, K, 2, 1>(gu, row, x1, nodes, lane, w, done);
+  } else {
+    xg_run<DT, K, 2, NT>(gu, row, xp, nodes, lane, w, done);
   }
 }
 
-// Down rows of the u-th routed expert for the positions routed to it: o[v][j][r] = down_r . act[v][j]
-// (k_expert_down's per-expert dot).
-template <int DT, int K, int P>
-__global__ __launch_bounds__(kPfNT) void k_moe_down_b(DMat dn, const float* __restrict__ act,
-                                                      const int* __restrict__ ids, int nv, int k, int hidden,
-                                                      float* __restrict__ o) {
-  using G = Geo<DT, K>;
-  __shared__ PfPlan pl;
-  __shared__ __align__(16) float xs[kPfMaxPos][K];
-  pf_plan(ids, nv, k, pl);
-  const int e = nth_bit64(pl.used, blockIdx.y);
+// 32 down rows of one expert for a tile of its members: o[slot][r] = down_r . act[slot] (k_expert_down's dot).
+template <int DT, int K, int NT>
+__global__ __launch_bounds__((XGeo<DT, K>::NT_), 2) void k_moe_down_x(DMat dn, const float* __restrict__ act,
+                                                                    const int* __restrict__ cnt,
+                                                                    const int* __restrict__ list, int cap, int hidden,
+                                                                    float* __restrict__ o) {
+  __shared__ float nodes[xg_lds<DT, K, 2, NT>()];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15;
+  int first = 0, members = 0;
+  const int e = member_tile<16 * NT>(cnt, blockIdx.y, lane, &first, &members);
   if (e < 0) return;
-  const unsigned members = pl.bits[e];
-  const int ne = __popc(members);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int sub = lane % G::LPR, rw = lane / G::LPR;
-  const size_t base = ((size_t)blockIdx.x * kPfWaves + wave) * (P * G::RPW);
-  size_t row[P];
-  bool ok[P];
+  const int r0 = blockIdx.x * 32;
+  const size_t row[2] = {(size_t)e * hidden + r0 + i, (size_t)e * hidden + r0 + 16 + i};
+  const float* xp[NT];
+  int slot[NT];
 #pragma unroll
-  for (int p = 0; p < P; p++) {
-    const size_t r = base + (size_t)p * G::RPW + rw;
-    ok[p] = r < (size_t)hidden;
-    row[p] = (size_t)e * hidden + (ok[p] ? r : 0);
+  for (int n = 0; n < NT; n++) {
+    slot[n] = list[(size_t)e * cap + min(first + 16 * n + i, members - 1)];
+    xp[n] = act + (size_t)slot[n] * K;
   }
-  Rows<DT, K, P> rr;
-  rows_load<DT, K, P>(rr, dn, row, ok, sub);
-  DeqRows<DT, K, P> dw;
-  deq_rows<DT, K, P>(rr, dw);
-  // every member's activation (K = I floats each) into LDS
-  for (int i = threadIdx.x; i < ne * K / 4; i += kPfNT) {
-    const int c = i / (K / 4), w4 = i % (K / 4);
-    const int vpos = nth_bit64(members, c);
-    reinterpret_cast<float4*>(&xs[c][0])[xslot<DT>(w4)] =
-        reinterpret_cast<const float4*>(act + ((size_t)vpos * k + pl.rank[e][vpos]) * K)[w4];
+  auto done = [&](int n, int r, const float (&v)[2]) {
+    if (first + 16 * n + i >= members) return;
+    const int sl = NT == 1 || n == 0 ? slot[0] : slot[NT - 1];
+    float* ov = o + (size_t)sl * hidden + r0 + 4 * (lane >> 4) + r;
+    ov[0] = v[0];
+    ov[16] = v[1];
+  };
+  if (NT == 2 && first + 16 >= members) {
+    const float* const x1[1] = {xp[0]};
+    xg_run<DT, K, 2, 1>(dn, row, x1, nodes, lane, w, done);
+  } else {
+    xg_run<DT, K, 2, NT>(dn, row, xp, nodes, lane, w, done);
+  }
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// Position blockIdx.x: h[r] = h[r] + res * y, y = sum over j = 0 .. k-1 in order of w[j] * o[j][r] (k_expert_down's
+// combine; k = 0: h stays), then with lnw the next layer's input xn = lnw * (h * rms scale) in the canonical order.
+template <int K>
+__global__ __launch_bounds__(256) void k_moe_comb_x(const float* __restrict__ o, const float* __restrict__ wts, int k,
+                                                    float res, float* __restrict__ h, const float* __restrict__ lnw,
+                                                    float eps, float* __restrict__ xn) {
+  constexpr int Q = K / 4, PER = (Q + 255) / 256;
+  __shared__ __align__(16) float hs[K];
+  __shared__ float rs;
+  const int v = blockIdx.x;
+  float4* hv = reinterpret_cast<float4*>(h + (size_t)v * K);
+  float4 hq[PER];
+#pragma unroll
+  for (int e = 0; e < PER; e++) {
+    const int q = threadIdx.x + 256 * e, qc = min(q, Q - 1);
+    float4 t = hv[qc];
+    if (k > 0) {
+      float4 y = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      for (int j = 0; j < k; j++) {
+        const float wj = wts[v * k + j];
+        const float4 x = reinterpret_cast<const float4*>(o + ((size_t)v * k + j) * K)[qc];
+        y.x = y.x + wj * x.x;
+        y.y = y.y + wj * x.y;
+        y.z = y.z + wj * x.z;
+        y.w = y.w + wj * x.w;
+      }
+      t.x = t.x + res * y.x;
+      t.y = t.y + res * y.y;
+      t.z = t.z + res * y.z;
+      t.w = t.w + res * y.w;
+      if (q < Q) hv[q] = t;
+    }
+    hq[e] = t;
+    if (q < Q) reinterpret_cast<float4*>(hs)[q] = t;
+  }
+  if (!lnw) return;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const float r = rms_scale<K>(hs, eps, threadIdx.x);
+    if (threadIdx.x == 0) rs = r;
   }
   __syncthreads();
-  for (int c = 0; c < ne; c++) {
-    XReg<DT, K> xr;
-    load_xs<DT, K>(xr, &xs[c][0], sub);
-    float out[P];
-    deq_fma<DT, K, P>(dw, ok, xr, sub, out);
-    if (sub != 0) continue;
-    const int vpos = nth_bit64(members, c);
-    float* ov = o + ((size_t)vpos * k + pl.rank[e][vpos]) * hidden;
+  const float r = rs;
 #pragma unroll
-    for (int p = 0; p < P; p++)
-      if (ok[p]) ov[base + (size_t)p * G::RPW + rw] = out[p];
+  for (int e = 0; e < PER; e++) {
+    const int q = threadIdx.x + 256 * e;
+    if (q >= Q) continue;
+    const float4 lw = reinterpret_cast<const float4*>(lnw)[q], t = hq[e];
+    reinterpret_cast<float4*>(xn + (size_t)v * K)[q] =
+        make_float4(lw.x * (t.x * r), lw.y * (t.y * r), lw.z * (t.z * r), lw.w * (t.w * r));
   }
-}
-
-// h[v][r] = h[v][r] + res * y, y = sum over j = 0 .. k-1 in order of w[v][j] * o[v][j][r] (k_expert_down's combine).
-__global__ __launch_bounds__(256) void k_moe_comb_b(const float* __restrict__ o, const float* __restrict__ wts, int k,
-                                                    int hidden, float res, float* __restrict__ h) {
-  const int v = blockIdx.y, r = blockIdx.x * 256 + threadIdx.x;
-  if (r >= hidden) return;
-  float y = 0.0f;
-  for (int j = 0; j < k; j++) y = y + wts[v * k + j] * o[((size_t)v * k + j) * hidden + r];
-  float* hv = h + (size_t)v * hidden;
-  const float hold = hv[r];
-  hv[r] = hold + res * y;
 }
 
 // Embedding rows of the nv tokens (k_embed per position).
@@ -533,10 +537,6 @@ __global__ __launch_bounds__(256) void k_embed_b(DMat e, const int* __restrict__
 // ------------------------------------------------------------------------------------------------------------
 // Launchers.
 static inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
-constexpr int kPfQkvNP = 1;    // row pairs per wave of k_qkv_b
-constexpr int kPfOprojP = 1;   // rows per wave of k_oproj_b
-constexpr int kPfUpNP = 1;     // row pairs per wave of k_moe_up_b
-constexpr int kPfDownP = 1;    // rows per wave of k_moe_down_b
 
 hipError_t launch_embed_b(hipStream_t s, const DMat& emb, const Dims& d, const PfBufs& p, int nv) {
   const dim3 grid((d.hidden + 255) / 256, nv);
@@ -549,54 +549,88 @@ hipError_t launch_embed_b(hipStream_t s, const DMat& emb, const Dims& d, const P
   return hipGetLastError();
 }
 
+// One or two position tiles per workgroup of the dense products: two halve the reads and the dequantisation of a row,
+// one gives twice the workgroups, which wins while those of two would leave compute units without one.
+static bool two_tiles(int row_groups, int nv) { return (long)row_groups * cdiv(nv, 32) >= 256; }
+
+static hipError_t comb_dispatch(hipStream_t s, const Dims& d, const PfBufs& p, int nv, int k, const float* lnw) {
+#define COMB(KK)                                                                                                 \
+  case KK: klaunch(k_moe_comb_x<KK>, nv, 256, 0, s, p.o, p.w, k, d.res_mult, p.h, lnw, d.eps, p.xn); break;
+  switch (d.hidden) {
+    MOERT_K_CASES(COMB)
+    default: return hipErrorInvalidValue;
+  }
+#undef COMB
+  return hipGetLastError();
+}
+
+hipError_t launch_norm_b(hipStream_t s, const Dims& d, const PfBufs& p, int nv, const float* lnw) {
+  return comb_dispatch(s, d, p, nv, 0, lnw);
+}
+
 hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* lenp, int pos0,
-                          int nv, const float* rope) {
-  if (nv < 1 || nv > kPfMaxPos || d.top_k > 8 || d.experts > 64 || d.head_dim != 64) return hipErrorInvalidValue;
-#define BODY(KK)                                                                                         \
-  case KK: {                                                                                             \
-    constexpr int PB = kPfWaves * kPfQkvNP * Geo<DTC, KK>::RPW;                                          \
-    klaunch(k_qkv_b<DTC, KK, kPfQkvNP>, cdiv(L.qkv.rows / 2, PB), kPfNT, 0, s, L.qkv, p.h, L.ln_attn, d.eps, \
-            pos0, nv, rope, d.heads, d.kv_heads, d.max_len, p.q, L.k_cache, L.v_cache);                  \
+                          int nv, const float* rope, const float* next_lnw) {
+  if (nv < 1 || nv > p.cap || d.top_k > 8 || d.experts > 64 || d.head_dim != 64) return hipErrorInvalidValue;
+  if (L.qkv.rows != (d.heads + 2 * d.kv_heads) * 64 || d.hidden % 32 || d.inter % 16) return hipErrorInvalidValue;
+#define QKV(KK, NN)                                                                                                 \
+  klaunch(k_qkv_x<DTC, KK, NN>, dim3(L.qkv.rows / 32, cdiv(nv, 16 * NN)), XGeo<DTC, KK>::NT_, 0, s, L.qkv, p.xn, pos0, \
+          nv, rope, d.heads, d.kv_heads, d.max_len, p.q, L.k_cache, L.v_cache, p.cnt)
+#define BODY(KK)                                        \
+  case KK: {                                            \
+    if (two_tiles(L.qkv.rows / 32, nv)) QKV(KK, 2);     \
+    else QKV(KK, 1);                                    \
   } break;
   MOERT_DISPATCH(L.qkv.dtype, L.qkv.cols, BODY)
 #undef BODY
+#undef QKV
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   // position v attends to pos0 + v + 1 positions: *lenp = pos0 on the device, len_add = 1
   if ((e = launch_attn_batched(s, L, d, lenp, 1, nv, p.q, p.part, p.att)) != hipSuccess) return e;
-#define BODY(KK)                                                                                         \
-  case KK: {                                                                                             \
-    constexpr int RB = kPfWaves * kPfOprojP * Geo<DTC, KK>::RPW;                                         \
-    klaunch(k_oproj_b<DTC, KK, kPfOprojP>, cdiv(L.o.rows, RB), kPfNT, 0, s, L.o, p.att, nv, d.res_mult, p.h, \
-            L.router, L.ln_moe, p.zpart);                                                                \
+#define OPROJ(KK, NN)                                                                                              \
+  klaunch(k_oproj_x<DTC, KK, NN>, dim3(L.o.rows / 32, cdiv(nv, 16 * NN)), XGeo<DTC, KK>::NT_, 0, s, L.o, p.att, nv, \
+          d.res_mult, p.h)
+#define BODY(KK)                                        \
+  case KK: {                                            \
+    if (two_tiles(L.o.rows / 32, nv)) OPROJ(KK, 2);     \
+    else OPROJ(KK, 1);                                  \
   } break;
   MOERT_DISPATCH(L.o.dtype, L.o.cols, BODY)
 #undef BODY
+#undef OPROJ
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (L.router.dtype != L.gate_up.dtype || L.router.cols != L.gate_up.cols) return hipErrorInvalidValue;
-#define BODY(KK)                                                                                         \
-  case KK: {                                                                                             \
-    klaunch(k_route_b<DTC, KK>, nv, route_b_waves(DTC) * 64, 0, s, L.router, L.router_bias, p.h, L.ln_moe, d.eps, \
-            p.zpart, d.top_k, p.xn, p.ids, p.w);                                                         \
+#define BODY(KK)                                                                                                    \
+  case KK: {                                                                                                        \
+    klaunch(k_route_x<DTC, KK>, nv, route_x_waves(DTC) * 64, 0, s, L.router, L.router_bias, p.h, L.ln_moe, d.eps,   \
+            d.top_k, p.cap, p.xn, p.w, p.cnt, p.list);                                                              \
   } break;
   MOERT_DISPATCH(L.router.dtype, L.router.cols, BODY)
 #undef BODY
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  const int U = std::min(nv * d.top_k, d.experts);
-#define BODY(KK)                                                                                         \
-  case KK: {                                                                                             \
-    constexpr int PB = kPfWaves * kPfUpNP * Geo<DTC, KK>::RPW;                                           \
-    klaunch(k_moe_up_b<DTC, KK, kPfUpNP>, dim3(cdiv(d.inter, PB), U), kPfNT, 0, s, L.gate_up, p.xn, p.ids, nv, \
-            d.top_k, d.inter, p.act);                                                                    \
+  // One position tile per workgroup while an expert has at most 16 members on average. The tiles of all experts are
+  // at most the members' over a tile and one more per expert used; a workgroup past the last ends at once.
+  const bool two = (long)nv * d.top_k > 16L * d.experts;
+  const int slots = nv * d.top_k, tiles = slots / (two ? 32 : 16) + std::min(slots, d.experts);
+#define UP(KK, NN)                                                                                                 \
+  klaunch(k_moe_up_x<DTC, KK, NN>, dim3(d.inter / 16, tiles), XGeo<DTC, KK>::NT_, 0, s, L.gate_up, p.xn, p.cnt, p.list, \
+          p.cap, d.top_k, d.inter, p.act)
+#define BODY(KK)               \
+  case KK: {                   \
+    if (two) UP(KK, 2);        \
+    else UP(KK, 1);            \
   } break;
   MOERT_DISPATCH(L.gate_up.dtype, L.gate_up.cols, BODY)
 #undef BODY
+#undef UP
   if ((e = hipGetLastError()) != hipSuccess) return e;
-#define BODY(KK)                                                                                         \
-  case KK: {                                                                                             \
-    constexpr int RB = kPfWaves * kPfDownP * Geo<DTC, KK>::RPW;                                          \
-    klaunch(k_moe_down_b<DTC, KK, kPfDownP>, dim3(cdiv(d.hidden, RB), U), kPfNT, 0, s, L.down, p.act, p.ids, nv, \
-            d.top_k, d.hidden, p.o);                                                                     \
+#define DOWN(KK, NN)                                                                                              \
+  klaunch(k_moe_down_x<DTC, KK, NN>, dim3(d.hidden / 32, tiles), XGeo<DTC, KK>::NT_, 0, s, L.down, p.act, p.cnt, p.list, \
+          p.cap, d.hidden, p.o)
+#define BODY(KK)               \
+  case KK: {                   \
+    if (two) DOWN(KK, 2);      \
+    else DOWN(KK, 1);          \
   } break;
   switch (L.down.dtype) {
     case DT_Q8_0: {
@@ -614,14 +648,14 @@ hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const
     default: return hipErrorInvalidValue;
   }
 #undef BODY
+#undef DOWN
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  klaunch(k_moe_comb_b, dim3((d.hidden + 255) / 256, nv), 256, 0, s, p.o, p.w, d.top_k, d.hidden, d.res_mult, p.h);
-  return hipGetLastError();
+  return comb_dispatch(s, d, p, nv, d.top_k, next_lnw);
 }
 
 hipError_t launch_layer_grouped(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* lenp,
                                 int pos0, int nv, const float* rope, const GroupBufs& g, const float* next_lnw) {
-  if (nv < 1 || nv > kPfMaxPos || d.top_k > 8 || d.experts > 64 || d.head_dim != 64) return hipErrorInvalidValue;
+  if (nv < 1 || nv > p.cap || nv > kGrpMaxPos || d.top_k > 8 || d.experts > 64 || d.head_dim != 64) return hipErrorInvalidValue;
   GroupBufs gg = g;
   gg.ids = p.ids;
   gg.w = p.w;
