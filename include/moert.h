@@ -196,10 +196,11 @@ int moert_generate(moert_model* m, const int* prompt, int n_prompt, int n_new, i
  * cuda_backend.rs:272-274. Resident models only (MOERT_E_CONFIG on a cached one). */
 int moert_step_batched(moert_model* m, const int* tokens, int n, float* logits, int* argmax);
 
-/* Reads n tokens from the current position in blocks of at most 32 positions (moert_step_batched each; the block
- * plan of plano_blocos, rust/moe-rt/src/motor/leitura.rs:53-60), as
+/* Reads n tokens from the current position in blocks of consecutive positions, as
  * le_ids (rust/moe-rt/src/motor/leitura.rs:79-85, validation leitura.rs:62-76): the tokens are checked and the
- * cache bound (MOERT_E_FULL) before any block runs; logits / argmax of the last position. */
+ * cache bound (MOERT_E_FULL) before any block runs; logits / argmax of the last position. In mode 0 a block holds up
+ * to 512 positions (every weight is read once per block), in mode 1 up to 32, the block plan of plano_blocos
+ * (rust/moe-rt/src/motor/leitura.rs:53-60); in mode 0 the result does not depend on the blocks. */
 int moert_prefill(moert_model* m, const int* tokens, int n, float* logits, int* argmax);
 
 /* Back to position 0 (old KV stays, masked by the length). Replaces GpuModel::reset

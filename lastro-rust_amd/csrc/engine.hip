@@ -525,23 +525,27 @@ struct moert_model {
     return MOERT_OK;
   }
 
-  // multi-position step buffers, allocated on first use
+  // Multi-position step buffers for at least n positions, allocated on first use. A longer prompt than any before
+  // replaces them (twice the positions at least, kPfBlock at most); they go with the model.
   PfBufs pf{};
-  int ensure_pf() {
-    if (pf.h) return MOERT_OK;
-    const int H = dims.hidden, qd = dims.heads * 64, I = dims.inter, M = kPfMaxPos, K8 = 8;
-    const size_t parts = (size_t)M * dims.heads * attn_splits_for(max_len, dims.tps) * 66;
-    pf.cap = M;
-    int rc;
-    if ((rc = zeros(arena, stream, (size_t)M, &pf.toks)) || (rc = zeros(arena, stream, (size_t)1, &pf.pos0)) ||
-        (rc = zeros(arena, stream, (size_t)M * qd, &pf.q)) || (rc = zeros(arena, stream, (size_t)M * qd, &pf.att)) ||
-        (rc = zeros(arena, stream, parts, &pf.part)) || (rc = zeros(arena, stream, (size_t)M * H, &pf.xn)) ||
-        (rc = zeros(arena, stream, (size_t)M * K8, &pf.ids)) || (rc = zeros(arena, stream, (size_t)M * K8, &pf.w)) ||
-        (rc = zeros(arena, stream, (size_t)64, &pf.cnt)) || (rc = zeros(arena, stream, (size_t)64 * M, &pf.list)) ||
-        (rc = zeros(arena, stream, (size_t)M * K8 * I, &pf.act)) ||
-        (rc = zeros(arena, stream, (size_t)M * K8 * H, &pf.o)) || (rc = zeros(arena, stream, (size_t)M * H, &pf.h)))
-      return rc;
+  Arena pf_arena;
+  int ensure_pf(int n) {
+    if (pf.cap >= n) return MOERT_OK;
     CHECK_HIP(hipStreamSynchronize(stream));
+    pf_arena.release();
+    pf = PfBufs{};
+    int M = kPfMaxPos;
+    while (M < n) M *= 2;
+    const int H = dims.hidden, qd = dims.heads * 64, I = dims.inter, K8 = 8;
+    const size_t parts = (size_t)M * dims.heads * attn_splits_for(max_len, dims.tps) * 66;
+    auto mem = [&](size_t words, auto** p) { return pf_arena.alloc((void**)p, words * 4); };  // written before it is read
+    int rc;
+    if ((rc = mem((size_t)M * qd, &pf.q)) || (rc = mem((size_t)M * qd, &pf.att)) || (rc = mem(parts, &pf.part)) ||
+        (rc = mem((size_t)M * H, &pf.xn)) || (rc = mem((size_t)M * K8, &pf.ids)) || (rc = mem((size_t)M * K8, &pf.w)) ||
+        (rc = mem(64, &pf.cnt)) || (rc = mem((size_t)64 * M, &pf.list)) || (rc = mem((size_t)M * K8 * I, &pf.act)) ||
+        (rc = mem((size_t)M * K8 * H, &pf.o)) || (rc = mem((size_t)M * H, &pf.h)))
+      return rc;
+    pf.cap = M;
     return MOERT_OK;
   }
 
@@ -585,11 +589,10 @@ struct moert_model {
     return MOERT_OK;
   }
 
-  // Positions pos0 .. pos0 + nv - 1 through every layer, then the final norm, head and argmax of the last one (the
-  // device state already holds pos = pos0 + nv - 1, fixed = pos0 + nv and *pf.pos0 = pos0); its hidden state is
-  // left in b.h, as after a decode step.
-  int enqueue_batched(int pos0, int nv) {
-    CHECK_HIP(launch_embed_b(stream, embed, dims, pf, nv));
+  // Positions pos0 .. pos0 + nv - 1 (tokens in b.seq) through every layer; with `head`, then the final norm, head and
+  // argmax of the last one, its hidden state left in b.h, as after a decode step.
+  int enqueue_batched(int pos0, int nv, bool head) {
+    CHECK_HIP(launch_embed_b(stream, embed, dims, pf, b.seq + pos0, nv, b.state, pos0 + nv - 1));
     if (batched_mode == 1)
       CHECK_HIP(launch_norm_codes(stream, dims.hidden, nv, pf.h, layers[0].ln_attn, dims.eps, mg));
     else
@@ -602,11 +605,12 @@ struct moert_model {
         g.dn = tiled[l].dn;
         g.qkv = tiled[l].qkv;
         g.oproj = tiled[l].o;
-        CHECK_HIP(launch_layer_grouped(stream, layers[l], dims, pf, pf.pos0, pos0, nv, b.rope, g, next));
+        CHECK_HIP(launch_layer_grouped(stream, layers[l], dims, pf, b.state, pos0, nv, b.rope, g, next));
       } else {
-        CHECK_HIP(launch_layer_b(stream, layers[l], dims, pf, pf.pos0, pos0, nv, b.rope, next));
+        CHECK_HIP(launch_layer_b(stream, layers[l], dims, pf, b.state, pos0, nv, b.rope, next));
       }
     }
+    if (!head) return MOERT_OK;
     StepBufs bl = b;
     bl.h = pf.h + (size_t)(nv - 1) * dims.hidden;
     CHECK_HIP(launch_head(stream, embed, norm, dims, bl));
@@ -734,6 +738,7 @@ struct moert_model {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
     if (tl_buf) (void)hipFree(tl_buf);
+    pf_arena.release();
     arena.release();
     if (host_store) (void)hipHostFree(host_store);
     for (hipEvent_t e : {ev_fork, ev_pred, ev_copy, mx_ev, mx_t[0], mx_t[1], mx_t[2]})
@@ -1467,6 +1472,24 @@ int moert_decode_step(moert_model* m, int token, float* logits, int* route_ids, 
   return MOERT_OK;
 }
 
+// n checked tokens at the current position, in equal blocks (a mode 1 block: at most kGrpMaxPos positions); logits and
+// argmax of the last one. One wait, at the end.
+static int read_tokens(moert_model* m, const int* tokens, int n, float* logits, int* argmax) {
+  const int most = m->batched_mode == 1 ? kGrpMaxPos : kPfBlock;
+  const int blocks = (n + most - 1) / most, per = std::min(most, ((n + blocks - 1) / blocks + 15) / 16 * 16);
+  const int pos0 = m->host_pos;
+  MTRY(m, m->ensure_pf(std::min(n, per)));
+  MTRY(m, model_copy_in(m, m->b.seq + pos0, tokens, (size_t)n * 4));
+  for (int i = 0; i < n; i += per) MTRY(m, m->enqueue_batched(pos0 + i, std::min(per, n - i), i + per >= n));
+  if (logits) MTRY(m, model_copy_out(m, logits, m->b.logits, (size_t)m->cfg.vocab * 4));
+  int am = 0;
+  MTRY(m, model_copy_out(m, &am, m->b.argmax_hist + pos0 + n - 1, 4));
+  MTRY(m, model_sync(m));
+  if (argmax) *argmax = am;
+  m->host_pos = pos0 + n;
+  return MOERT_OK;
+}
+
 int moert_step_batched(moert_model* m, const int* tokens, int n, float* logits, int* argmax) {
   MODEL_OK(m);
   CHECK_CFG(tokens && n >= 1 && n <= kPfMaxPos, "step_batched: %d positions outside [1, %d]", n, kPfMaxPos);
@@ -1480,21 +1503,7 @@ int moert_step_batched(moert_model* m, const int* tokens, int n, float* logits, 
       set_err("token %d outside the vocabulary (%d)", tokens[i], m->cfg.vocab);
       return MOERT_E_RANGE;
     }
-  MTRY(m, m->ensure_pf());
-  const int pos0 = m->host_pos;
-  int st[2] = {pos0 + n - 1, pos0 + n};
-  MTRY(m, model_copy_in(m, m->pf.toks, tokens, (size_t)n * 4));
-  MTRY(m, model_copy_in(m, m->b.seq + pos0, tokens, (size_t)n * 4));
-  MTRY(m, model_copy_in(m, m->pf.pos0, &pos0, 4));
-  MTRY(m, model_copy_in(m, m->b.state, st, sizeof st));
-  MTRY(m, m->enqueue_batched(pos0, n));
-  if (logits) MTRY(m, model_copy_out(m, logits, m->b.logits, (size_t)m->cfg.vocab * 4));
-  int am = 0;
-  MTRY(m, model_copy_out(m, &am, m->b.argmax_hist + pos0 + n - 1, 4));
-  MTRY(m, model_sync(m));
-  if (argmax) *argmax = am;
-  m->host_pos = pos0 + n;
-  return MOERT_OK;
+  return read_tokens(m, tokens, n, logits, argmax);
 }
 
 int moert_batched_mode(moert_model* m, int mode) {
@@ -1531,12 +1540,8 @@ int moert_prefill(moert_model* m, const int* tokens, int n, float* logits, int* 
     set_err("KV cache full: %d + %d positions > %d", m->host_pos, n, m->max_len);
     return MOERT_E_FULL;
   }
-  for (int i = 0; i < n; i += kPfMaxPos) {
-    const int nb = std::min(kPfMaxPos, n - i), last = i + nb == n;
-    const int rc = moert_step_batched(m, tokens + i, nb, last ? logits : nullptr, last ? argmax : nullptr);
-    if (rc) return rc;
-  }
-  return MOERT_OK;
+  CHECK_CFG(!m->cached, "step_batched: the multi-position step runs on a resident model");
+  return read_tokens(m, tokens, n, logits, argmax);
 }
 
 static int generate(moert_model* m, const int* prompt, int n_prompt, int n_new, int* out_tokens, float* gaps,

@@ -8,13 +8,16 @@
 
 namespace moert {
 
-constexpr int kPfMaxPos = 32;  // positions per step (the reference's block limit, cuda_backend.rs:272-274)
+constexpr int kPfMaxPos = 32;  // positions of one step call (the reference's block limit, cuda_backend.rs:272-274)
+// Positions per pass over the layers of a longer prompt. A pass reads every weight once, and its row products work on
+// tiles of 16 or 32 positions per expert: more positions fill more of a tile and hide more of the reads. 512 tokens
+// of the 3B shape, 4 layers: passes of 32 positions 7915 us, 128: 3015, 256: 2375, 512: 2000 (of which gate/up
+// 4 x 183); the buffers of a pass grow with it (512 positions: 0.2 GB at 64 splits).
+constexpr int kPfBlock = 512;
 
 // Device buffers of one multi-position step, sized for `cap` positions.
 struct PfBufs {
   int cap;       // positions
-  int* toks;     // [m] tokens of the positions
-  int* pos0;     // [1] first position of the step (the length every attention length is counted from)
   float* h;      // [m, H] residual streams
   float* q;      // [m, heads*d] queries
   float* att;    // [m, heads*d] attention outputs
@@ -28,18 +31,21 @@ struct PfBufs {
   int* ids;      // [m, k] routed experts, top-k order (grouped mode)
 };
 
-hipError_t launch_embed_b(hipStream_t s, const DMat& emb, const Dims& d, const PfBufs& p, int nv);
+// Embedding rows of the nv tokens at `toks` (device) into h; the step state becomes position `last` and first free
+// position last + 1.
+hipError_t launch_embed_b(hipStream_t s, const DMat& emb, const Dims& d, const PfBufs& p, const int* toks, int nv,
+                          int* state, int last);
 // xn = rmsnorm(h, lnw) of every position: the first layer's input.
 hipError_t launch_norm_b(hipStream_t s, const Dims& d, const PfBufs& p, int nv, const float* lnw);
-// One layer for positions pos0 .. pos0 + nv - 1 (*lenp == pos0 on the device), rope: the [max_len, 64] table; the
+// One layer for positions pos0 .. pos0 + nv - 1 (state[ST_POS] == pos0 + nv - 1 on the device), rope: the [max_len, 64] table; the
 // decode kernels' chains, so that the results equal nv decode steps bit for bit. On entry xn = rmsnorm(h, L.ln_attn);
 // with next_lnw the layer leaves rmsnorm(h, next_lnw) there for the next one.
-hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* lenp, int pos0,
+hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* state, int pos0,
                           int nv, const float* rope, const float* next_lnw);
 // The same layer in grouped mode: q/k/v, output projection and experts through the int8 MFMA kernels of grouped.h,
 // g holding the layer's tiled matrices. On entry g's codes are those of rmsnorm(h, L.ln_attn) (launch_norm_codes or
 // the previous layer's combine); with next_lnw the layer leaves the codes of rmsnorm(h, next_lnw) for the next one.
-hipError_t launch_layer_grouped(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* lenp,
+hipError_t launch_layer_grouped(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* state,
                                 int pos0, int nv, const float* rope, const GroupBufs& g, const float* next_lnw);
 
 }  // namespace moert

@@ -515,7 +515,11 @@ __global__ __launch_bounds__(256) void k_moe_comb_x(const float* __restrict__ o,
 // Embedding rows of the nv tokens (k_embed per position).
 template <int DT>
 __global__ __launch_bounds__(256) void k_embed_b(DMat e, const int* __restrict__ toks, float mult,
-                                                 float* __restrict__ h) {
+                                                 float* __restrict__ h, int* __restrict__ state, int last) {
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    state[ST_POS] = last;
+    state[ST_FIXED] = last + 1;
+  }
   const int v = blockIdx.y, tok = toks[v];
   const int H = e.cols;
   float* hv = h + (size_t)v * H;
@@ -538,12 +542,13 @@ __global__ __launch_bounds__(256) void k_embed_b(DMat e, const int* __restrict__
 // Launchers.
 static inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 
-hipError_t launch_embed_b(hipStream_t s, const DMat& emb, const Dims& d, const PfBufs& p, int nv) {
+hipError_t launch_embed_b(hipStream_t s, const DMat& emb, const Dims& d, const PfBufs& p, const int* toks, int nv,
+                          int* state, int last) {
   const dim3 grid((d.hidden + 255) / 256, nv);
   switch (emb.dtype) {
-    case DT_Q8_0: klaunch(k_embed_b<DT_Q8_0>, grid, 256, 0, s, emb, p.toks, d.emb_mult, p.h); break;
-    case DT_Q4_0: klaunch(k_embed_b<DT_Q4_0>, grid, 256, 0, s, emb, p.toks, d.emb_mult, p.h); break;
-    case DT_F32: klaunch(k_embed_b<DT_F32>, grid, 256, 0, s, emb, p.toks, d.emb_mult, p.h); break;
+    case DT_Q8_0: klaunch(k_embed_b<DT_Q8_0>, grid, 256, 0, s, emb, toks, d.emb_mult, p.h, state, last); break;
+    case DT_Q4_0: klaunch(k_embed_b<DT_Q4_0>, grid, 256, 0, s, emb, toks, d.emb_mult, p.h, state, last); break;
+    case DT_F32: klaunch(k_embed_b<DT_F32>, grid, 256, 0, s, emb, toks, d.emb_mult, p.h, state, last); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -568,7 +573,7 @@ hipError_t launch_norm_b(hipStream_t s, const Dims& d, const PfBufs& p, int nv, 
   return comb_dispatch(s, d, p, nv, 0, lnw);
 }
 
-hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* lenp, int pos0,
+hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* state, int pos0,
                           int nv, const float* rope, const float* next_lnw) {
   if (nv < 1 || nv > p.cap || d.top_k > 8 || d.experts > 64 || d.head_dim != 64) return hipErrorInvalidValue;
   if (L.qkv.rows != (d.heads + 2 * d.kv_heads) * 64 || d.hidden % 32 || d.inter % 16) return hipErrorInvalidValue;
@@ -585,8 +590,8 @@ hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const
 #undef QKV
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  // position v attends to pos0 + v + 1 positions: *lenp = pos0 on the device, len_add = 1
-  if ((e = launch_attn_batched(s, L, d, lenp, 1, nv, p.q, p.part, p.att)) != hipSuccess) return e;
+  // position v attends to pos0 + v + 1 positions: the length is counted from the last position on the device
+  if ((e = launch_attn_batched(s, L, d, state + ST_POS, 2 - nv, nv, p.q, p.part, p.att)) != hipSuccess) return e;
 #define OPROJ(KK, NN)                                                                                              \
   klaunch(k_oproj_x<DTC, KK, NN>, dim3(L.o.rows / 32, cdiv(nv, 16 * NN)), XGeo<DTC, KK>::NT_, 0, s, L.o, p.att, nv, \
           d.res_mult, p.h)
@@ -653,7 +658,7 @@ hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const
   return comb_dispatch(s, d, p, nv, d.top_k, next_lnw);
 }
 
-hipError_t launch_layer_grouped(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* lenp,
+hipError_t launch_layer_grouped(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* state,
                                 int pos0, int nv, const float* rope, const GroupBufs& g, const float* next_lnw) {
   if (nv < 1 || nv > p.cap || nv > kGrpMaxPos || d.top_k > 8 || d.experts > 64 || d.head_dim != 64) return hipErrorInvalidValue;
   GroupBufs gg = g;
@@ -661,8 +666,8 @@ hipError_t launch_layer_grouped(hipStream_t s, const LayerDev& L, const Dims& d,
   gg.w = p.w;
   hipError_t e;
   if ((e = launch_gd_qkv(s, d, nv, pos0, rope, p.q, L.k_cache, L.v_cache, gg)) != hipSuccess) return e;
-  // position v attends to pos0 + v + 1 positions: *lenp = pos0 on the device, len_add = 1
-  if ((e = launch_attn_batched(s, L, d, lenp, 1, nv, p.q, p.part, p.att)) != hipSuccess) return e;
+  // position v attends to pos0 + v + 1 positions: the length is counted from the last position on the device
+  if ((e = launch_attn_batched(s, L, d, state + ST_POS, 2 - nv, nv, p.q, p.part, p.att)) != hipSuccess) return e;
   if ((e = launch_grp_codes(s, d.heads * 64, nv, p.att, gg)) != hipSuccess) return e;
   if ((e = launch_gd_oproj(s, nv, d.res_mult, p.h, gg)) != hipSuccess) return e;
   if ((e = launch_grp_route_norm(s, L, nv, d.top_k, p.h, L.ln_moe, d.eps, gg)) != hipSuccess) return e;

@@ -522,7 +522,7 @@ class GpuModel:
         return lg, am.value
 
     def prefill(self, tokens, want_logits: bool = True):
-        """Any number of tokens in blocks of at most 32 positions (le_ids): (last logits, last argmax)."""
+        """Any number of tokens in blocks of positions (le_ids): (last logits, last argmax)."""
         t = np.ascontiguousarray(tokens, np.int32)
         lg = np.empty(self.cfg.vocab, np.float32) if want_logits else None
         am = ctypes.c_int(0)
