@@ -181,8 +181,9 @@ int moert_decode_step(moert_model* m, int token, float* logits, int* route_ids, 
  * (rust/moe-rt/src/cuda_dense.rs:236-288, motor/leitura.rs:79-85). */
 int moert_batched_mode(moert_model* m, int mode);
 
-/* Greedy generation with no host synchronisation between tokens: feeds the n_prompt tokens one position at a
- * time, then n_new tokens chosen by argmax (last index on ties). out_tokens receives the n_new generated ids;
+/* Greedy generation with no host synchronisation between tokens: feeds the n_prompt tokens (on a resident model in
+ * passes over several positions, as moert_prefill in mode 0, otherwise one position at a
+ * time), then n_new tokens chosen by argmax (last index on ties). out_tokens receives the n_new generated ids;
  * gaps (optional, n_new floats) receives top1 - top2 of the logits each generated token was chosen from.
  * Replaces the prompt + generation loop of rust/moe-rt/src/bin/m1b-gulosa.rs:85-105. */
 int moert_generate(moert_model* m, const int* prompt, int n_prompt, int n_new, int* out_tokens, float* gaps);

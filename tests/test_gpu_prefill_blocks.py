@@ -58,3 +58,35 @@ def test_mode_1_prompts_equal_steps_of_32(gpu):
     want = lg, am, g.hidden(), [tuple(a.copy() for a in g.read_kv(l, len(toks))) for l in range(cfg.layers)]
     same(got, want, "mode 1")
     g.close()
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_generate_equals_steps_for_every_prompt_length(gpu, mode):
+    """moert_generate reads a prompt of more than a few tokens in passes: the tokens and gaps of prompts of 1 to 6 and
+    of 40 tokens equal those of a loop of single steps, whatever the model's mode of its own multi-position steps."""
+    cfg = moert.Config(**{**moert.GRANITE_1B, "layers": 2, "vocab": 211})
+    m = moert.SynthModel(cfg, seed=19, std=0.05)
+    g = moert.GpuModel(m, 128, attn_splits=8)
+    g.batched_mode(mode)
+    rng = np.random.default_rng(6)
+    pos = 0
+    for n in (1, 2, 3, 4, 5, 6, 40):
+        prompt = rng.integers(0, cfg.vocab, n)
+        g.set_position(pos)
+        out, gaps = g.generate(prompt, 4, gaps=True)
+        end, lg = g.position(), g.read_logits()
+        g.set_position(pos)
+        want, feed = [], list(prompt)
+        for t in feed:
+            slg, _, _, am = g.step(int(t))
+        wgaps = []
+        for i in range(4):
+            s = np.sort(slg)
+            want.append(am)
+            wgaps.append(np.float32(s[-1] - s[-2]))
+            if i < 3:
+                slg, _, _, am = g.step(am)
+        assert out.tolist() == want and np.array_equal(gaps, np.array(wgaps, np.float32)), n
+        assert end == pos + n + 3 and np.array_equal(lg.view(np.uint32), slg.view(np.uint32)), n
+        pos += 3
+    g.close()
