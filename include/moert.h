@@ -200,8 +200,8 @@ int moert_step_batched(moert_model* m, const int* tokens, int n, float* logits, 
 /* Reads n tokens from the current position in blocks of consecutive positions, as
  * le_ids (rust/moe-rt/src/motor/leitura.rs:79-85, validation leitura.rs:62-76): the tokens are checked and the
  * cache bound (MOERT_E_FULL) before any block runs; logits / argmax of the last position. In mode 0 a block holds up
- * to 512 positions (every weight is read once per block), in mode 1 up to 32, the block plan of plano_blocos
- * (rust/moe-rt/src/motor/leitura.rs:53-60); in mode 0 the result does not depend on the blocks. */
+ * to 512 positions (every weight is read once per block) and the result does not depend on the blocks; in mode 1 the
+ * blocks are those of plano_blocos (rust/moe-rt/src/motor/leitura.rs:53-60), up to 32 positions, several to a launch. */
 int moert_prefill(moert_model* m, const int* tokens, int n, float* logits, int* argmax);
 
 /* Back to position 0 (old KV stays, masked by the length). Replaces GpuModel::reset

@@ -558,17 +558,29 @@ struct moert_model {
     TMat gu, dn, qkv, o;
   };
   std::vector<TiledLayer> tiled;
-  int ensure_grouped() {
-    if (mg.xh) return MOERT_OK;
-    const int H = dims.hidden, I = dims.inter, M = kGrpMaxPos, S = kGrpMaxPos * 8;
-    const int X = std::max(H, dims.heads * dims.head_dim);  // code rows: block inputs and attention outputs
+  Arena mg_arena;
+  int ensure_mg(int n) {  // buffers for at least n positions, replaced as those of ensure_pf
+    if (mg.cap >= n) return MOERT_OK;
+    CHECK_HIP(hipStreamSynchronize(stream));
+    mg_arena.release();
+    mg = GroupBufs{};
+    int M = kGrpMaxPos;
+    while (M < n) M *= 2;
+    const size_t H = dims.hidden, I = dims.inter, S = (size_t)M * 8;
+    const size_t X = std::max(dims.hidden, dims.heads * dims.head_dim);  // code rows: block inputs, attention outputs
+    auto mem = [&](size_t bytes, auto** p) { return mg_arena.alloc((void**)p, bytes); };  // written before it is read
     int rc;
-    if ((rc = zeros(arena, stream, (size_t)M * X, &mg.xh)) || (rc = zeros(arena, stream, (size_t)M * X, &mg.xl)) ||
-        (rc = zeros(arena, stream, (size_t)M * (X / 32), &mg.xd)) ||
-        (rc = zeros(arena, stream, (size_t)GRP_WORDS, &mg.grp)) || (rc = zeros(arena, stream, (size_t)S * I, &mg.ah)) ||
-        (rc = zeros(arena, stream, (size_t)S * I, &mg.al)) || (rc = zeros(arena, stream, (size_t)S * (I / 32), &mg.ad)) ||
-        (rc = zeros(arena, stream, (size_t)S * H, &mg.o)))
+    if ((rc = mem(M * X, &mg.xh)) || (rc = mem(M * X, &mg.xl)) || (rc = mem(M * (X / 32) * 4, &mg.xd)) ||
+        (rc = mem((size_t)M / kGrpMaxPos * GRP_WORDS * 4, &mg.grp)) || (rc = mem(S * I, &mg.ah)) ||
+        (rc = mem(S * I, &mg.al)) || (rc = mem(S * (I / 32) * 4, &mg.ad)) || (rc = mem(S * H * 4, &mg.o)))
       return rc;
+    mg.cap = M;
+    return MOERT_OK;
+  }
+  int ensure_grouped() {
+    if (!tiled.empty()) return MOERT_OK;
+    int rc;
+    std::vector<TiledLayer> made;
     auto tile = [&](const DMat& src, TMat* dst) -> int {
       uint8_t* q;
       uint16_t* d;
@@ -584,9 +596,10 @@ struct moert_model {
       if ((rc = tile(L.gate_up, &t.gu)) || (rc = tile(L.down, &t.dn)) || (rc = tile(L.qkv, &t.qkv)) ||
           (rc = tile(L.o, &t.o)))
         return rc;
-      tiled.push_back(t);
+      made.push_back(t);
     }
     CHECK_HIP(hipStreamSynchronize(stream));
+    tiled = std::move(made);
     return MOERT_OK;
   }
 
@@ -740,6 +753,7 @@ struct moert_model {
     if (graph) (void)hipGraphDestroy(graph);
     if (tl_buf) (void)hipFree(tl_buf);
     pf_arena.release();
+    mg_arena.release();
     arena.release();
     if (host_store) (void)hipHostFree(host_store);
     for (hipEvent_t e : {ev_fork, ev_pred, ev_copy, mx_ev, mx_t[0], mx_t[1], mx_t[2]})
@@ -1057,6 +1071,7 @@ struct moert_block {
         (rc = zeros(arena, stream, (size_t)S * I, &g.ah)) || (rc = zeros(arena, stream, (size_t)S * I, &g.al)) ||
         (rc = zeros(arena, stream, (size_t)S * (I / 32), &g.ad)) || (rc = zeros(arena, stream, (size_t)S * H, &g.o)))
       return rc;
+    g.cap = M;
     // the experts in the tiled layout of the MFMA kernels, copied once from the resident matrices
     auto tiled = [&](const DMat& src, TMat* dst) -> int {
       uint8_t* q;
@@ -1473,12 +1488,14 @@ int moert_decode_step(moert_model* m, int token, float* logits, int* route_ids, 
   return MOERT_OK;
 }
 
-// Positions pos0 .. pos0 + n - 1 (tokens in b.seq) in equal passes over the layers (mode 1: of at most kGrpMaxPos
-// positions), the last one with the head.
+// Positions pos0 .. pos0 + n - 1 (tokens in b.seq) in equal passes over the layers, of whole steps of kGrpMaxPos
+// positions (mode 1's results depend on its steps), the last one with the head.
 static int enqueue_blocks(moert_model* m, int pos0, int n, bool head) {
-  const int most = m->batched_mode == 1 ? kGrpMaxPos : kPfBlock;
-  const int blocks = (n + most - 1) / most, per = std::min(most, ((n + blocks - 1) / blocks + 15) / 16 * 16);
+  static_assert(kPfBlock % kGrpMaxPos == 0, "a pass is whole steps");
+  const int passes = (n + kPfBlock - 1) / kPfBlock, steps = grp_steps(n);
+  const int per = (steps + passes - 1) / passes * kGrpMaxPos;
   MTRY(m, m->ensure_pf(std::min(n, per)));
+  if (m->batched_mode == 1) MTRY(m, m->ensure_mg(std::min(n, per)));
   for (int i = 0; i < n; i += per) MTRY(m, m->enqueue_batched(pos0 + i, std::min(per, n - i), head && i + per >= n));
   return MOERT_OK;
 }

@@ -25,21 +25,40 @@ struct TMat {
   int rows, cols;
 };
 
-// Device buffers of one grouped step, sized for kGrpMaxPos positions, hidden H, inter I and top-k <= 8.
+// Device buffers of a grouped pass over `cap` positions, hidden H, inter I and top-k <= 8. A pass of more than
+// kGrpMaxPos positions is a run of steps of kGrpMaxPos (the last may be shorter) that share every launch: each has its
+// own plan and its own kGrpMaxPos * 8 member slots, so that its results are those of the step alone.
 struct GroupBufs {
+  int cap;       // positions the buffers hold
   int* ids;      // [m, k] routed experts, top-k order
   float* w;      // [m, k] routing weights
   int8_t* xh;    // [m, H] hi codes of the block inputs
   int8_t* xl;    // [m, H] lo codes
   float* xd;     // [m, H/32] their block scales
-  int* grp;      // [GRP_WORDS] the step plan (see GRP_*)
-  int8_t* ah;    // [m*k, I] hi codes of the SwiGLU activations, by member slot
-  int8_t* al;    // [m*k, I]
-  float* ad;     // [m*k, I/32]
-  float* o;      // [m*k, H] down outputs by member slot
+  int* grp;      // [steps, GRP_WORDS] the step plans (see GRP_*)
+  int8_t* ah;    // [steps * kGrpMaxPos * 8, I] hi codes of the SwiGLU activations, by member slot
+  int8_t* al;    // the same: lo codes
+  float* ad;     // [.., I/32] their block scales
+  float* o;      // [.., H] down outputs by member slot
   TMat gu, dn;   // gate_up [E*2I, H] and down [E*H, I] of the block in the tiled layout
   TMat qkv, oproj;  // the layer's q/k/v [(heads + 2 kv_heads) * 64, H] and output [H, heads * 64] projections, tiled
 };
+
+// Steps of a pass over m positions, and the buffers of step sb (its positions, its plan, its slots; H of the codes).
+inline int grp_steps(int m) { return (m + kGrpMaxPos - 1) / kGrpMaxPos; }
+__device__ __forceinline__ GroupBufs grp_step(GroupBufs g, int sb, int k, int H, int I) {
+  const size_t p0 = (size_t)sb * kGrpMaxPos, s0 = p0 * 8;
+  g.ids += p0 * k;
+  g.w += p0 * k;
+  g.xh += p0 * H;
+  g.xl += p0 * H;
+  g.xd += p0 * (H / 32);
+  g.grp += (size_t)sb * GRP_WORDS;
+  g.ah += s0 * I;
+  g.al += s0 * I;
+  g.ad += s0 * (I / 32);
+  return g;
+}
 
 // Exchange buffers of the one-launch block (launch_grp_fused), zeroed at allocation. Entries are (value bits,
 // epoch) 8-byte words; the input codes are plain bytes published by a per-position epoch flag.
@@ -78,7 +97,7 @@ hipError_t launch_tile_q8(hipStream_t s, const DMat& src, uint8_t* q, uint16_t* 
 // (route, up, down, combine) record their dispatch start/end into ev[2i], ev[2i+1].
 hipError_t launch_grouped_block(hipStream_t s, const LayerDev& L, int m, int k, int inter, const float* x,
                                 GroupBufs g, float* y, const hipEvent_t* ev = nullptr);
-// Pieces of a layer of the multi-position step in grouped mode (every projection an int8 MFMA GEMM), on m <= 32
+// Pieces of a layer of the multi-position step in grouped mode (every projection an int8 MFMA GEMM), on m <= g.cap
 // positions; the activation codes live in g.xh / g.xl / g.xd between kernels.
 //   launch_norm_codes     codes of rmsnorm(h[p], lnw) (H 1024 or 1536)
 //   launch_gd_qkv         q/k/v of the coded rows through g.qkv, RoPE at positions pos0 + p, q [m, heads*64] in f32,

@@ -16,6 +16,7 @@
 //                                    SwiGLU, hi/lo codes of act; workgroup (0, 0) publishes the plan
 //   k_grp_down    grid (H/64, U):    down MFMA of list expert u for its members -> o[member slot]
 //   k_grp_combine grid (m, H/256):   y[p] = sum over p's experts in list order of w * o
+#include <algorithm>
 #include <climits>
 
 #include "attn_dev.h"
@@ -234,8 +235,12 @@ hipError_t launch_tile_q8(hipStream_t s, const DMat& src, uint8_t* q, uint16_t* 
 // the cut of the members into groups of NM changes no result.
 constexpr int kGrpUpThreads = 512;
 
+//
+// A pass of several steps (nsb > 1) has the step inside blockIdx.x, tile + tiles * step, and blockIdx.y is the expert
+// itself: the workgroups of one weight tile follow each other, on the XCD of the tile where the tiles are a multiple
+// of 8, so that the steps share its read.
 template <int H, int NM, int NT>
-__global__ __launch_bounds__(NT) void k_grp_up(int m, int k, int inter, GroupBufs g) {
+__global__ __launch_bounds__(NT) void k_grp_up(int m, int k, int inter, int nsb, GroupBufs gp) {
   constexpr int NB = H / 32;
   constexpr int STR = H + 16;
   constexpr int WH = NT / 128;  // waves per half (gate or up)
@@ -248,11 +253,13 @@ __global__ __launch_bounds__(NT) void k_grp_up(int m, int k, int inter, GroupBuf
   __shared__ __align__(16) uint16_t sdt[NT / 64][NB * 16];
   __shared__ float gout[2][RT][NM + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int u = blockIdx.y, tile = blockIdx.x;
+  const int tiles = inter / RT, sb = blockIdx.x / tiles, tile = blockIdx.x % tiles;
+  const GroupBufs g = grp_step(gp, sb, k, H, inter);
+  m = min(m - kGrpMaxPos * sb, kGrpMaxPos);
   make_plan<NT>(g.ids, m, k, plan);
-  if (u >= plan.nu) return;
+  if (nsb == 1 && (int)blockIdx.y >= plan.nu) return;
   const int c0 = NM * blockIdx.z;  // this workgroup's first member
-  const int e = plan.list[u], off = plan.offe[e] + c0;
+  const int e = nsb == 1 ? plan.list[blockIdx.y] : (int)blockIdx.y, off = plan.offe[e] + c0;
   unsigned bits = plan.bits[e];
   if (__popc(bits) <= c0) return;
   for (int i = 0; i < c0; i++) bits &= bits - 1u;  // the members from c0 on
@@ -308,14 +315,14 @@ __global__ __launch_bounds__(NT) void k_grp_up(int m, int k, int inter, GroupBuf
       if (part == 0) g.ad[slotv * (inter / 32) + blk] = d;
     }
   }
-  if (u == 0 && tile == 0 && c0 == 0) publish_plan<NT>(plan, g.w, m, k, g.grp);
+  if (e == plan.list[0] && tile == 0 && c0 == 0) publish_plan<NT>(plan, g.w, m, k, g.grp);
 }
 
 // ------------------------------------------------------------------------------------------------------------
 // Down of list expert u = blockIdx.y for its members [NM z, NM z + NM) (z = blockIdx.z; a workgroup past the
 // expert's member count ends at once), output rows [64t, 64t+64): o[slot][row].
 template <int I, int NM>
-__global__ __launch_bounds__(256, NM == 16 ? 2 : 1) void k_grp_down(int hidden, GroupBufs g) {
+__global__ __launch_bounds__(256, NM == 16 ? 2 : 1) void k_grp_down(int hidden, int nsb, GroupBufs gp) {
   constexpr int NB = I / 32;
   constexpr int STR = I + 16;
   __shared__ __align__(16) int8_t bh[NM * STR];
@@ -323,8 +330,20 @@ __global__ __launch_bounds__(256, NM == 16 ? 2 : 1) void k_grp_down(int hidden, 
   __shared__ float dx[NM * NB];
   __shared__ __align__(16) uint16_t sdt[4][NB * 16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int u = blockIdx.y, tile = blockIdx.x;
-  if (u >= g.grp[GRP_NU]) return;
+  const int tiles = hidden / 64, sb = blockIdx.x / tiles, tile = blockIdx.x % tiles;  // steps as in k_grp_up
+  GroupBufs g = gp;
+  g.grp += (size_t)sb * GRP_WORDS;
+  g.ah += (size_t)sb * kGrpMaxPos * 8 * I;
+  g.al += (size_t)sb * kGrpMaxPos * 8 * I;
+  g.ad += (size_t)sb * kGrpMaxPos * 8 * NB;
+  g.o += (size_t)sb * kGrpMaxPos * 8 * hidden;
+  int u = blockIdx.y;
+  const int nu = g.grp[GRP_NU];
+  if (nsb > 1) {  // the list index of expert blockIdx.y (the list holds up to 64)
+    const unsigned long long at = __ballot(lane < nu && g.grp[GRP_LIST + lane] == u);
+    u = at ? __ffsll((long long)at) - 1 : nu;
+  }
+  if (u >= nu) return;
   const int c0 = NM * blockIdx.z;
   if (g.grp[GRP_CNT + u] <= c0) return;
   const int e = g.grp[GRP_LIST + u], ne = g.grp[GRP_CNT + u] - c0, off = g.grp[GRP_OFF + u] + c0;
@@ -410,7 +429,7 @@ hipError_t launch_grouped_block(hipStream_t s, const LayerDev& L, int m, int k, 
 }
 
 hipError_t launch_grp_codes(hipStream_t s, int K, int m, const float* x, const GroupBufs& g) {
-  if (m < 1 || m > kGrpMaxPos) return hipErrorInvalidValue;
+  if (m < 1 || m > g.cap) return hipErrorInvalidValue;
   switch (K) {
     case 1024: klaunch(k_grp_codes<1024>, m, 256, 0, s, x, g); break;
     case 1536: klaunch(k_grp_codes<1536>, m, 256, 0, s, x, g); break;
@@ -422,7 +441,7 @@ hipError_t launch_grp_codes(hipStream_t s, int K, int m, const float* x, const G
 hipError_t launch_grp_route_norm(hipStream_t s, const LayerDev& L, int m, int k, const float* h, const float* lnw,
                                  float eps, const GroupBufs& g) {
   const int H = L.router.cols;
-  if (m < 1 || m > kGrpMaxPos || k < 1 || k > 8 || L.router.rows > 64 || L.router.dtype != DT_Q8_0 || !lnw)
+  if (m < 1 || m > g.cap || k < 1 || k > 8 || L.router.rows > 64 || L.router.dtype != DT_Q8_0 || !lnw)
     return hipErrorInvalidValue;
   switch (H) {
     case 1024:
@@ -441,29 +460,30 @@ hipError_t launch_grp_experts(hipStream_t s, int H, int E, int m, int k, int int
   auto arm = [&](int i) {
     if (ev) arm_launch_events(ev[2 * i], ev[2 * i + 1]);
   };
-  if (m < 1 || m > kGrpMaxPos || k < 1 || k > 8 || E > 64 || (H != 1024 && H != 1536) || !g.gu.q || !g.dn.q ||
+  if (m < 1 || m > g.cap || k < 1 || k > 8 || E > 64 || (H != 1024 && H != 1536) || !g.gu.q || !g.dn.q ||
       g.gu.cols != H || g.gu.rows != E * 2 * inter || g.dn.cols != inter || g.dn.rows != E * H)
     return hipErrorInvalidValue;
   hipError_t e;
-  const int U = m * k < E ? m * k : E;
-  const int CH = (m + 15) / 16;  // member groups of 16: a step's expert has at most m members
+  const int nsb = grp_steps(m);
+  const int U = nsb == 1 && m * k < E ? m * k : E;
+  const int CH = (std::min(m, kGrpMaxPos) + 15) / 16;  // member groups of 16: a step's expert has at most m members
   // u is the slow grid index, so the workgroups of list indices past the step's expert count (which end at once)
   // are dispatched last
   constexpr int NT = kGrpUpThreads, RT = 16 * NT / 128;
-  const dim3 gu_grid(inter / RT, U, CH);
+  const dim3 gu_grid(inter / RT * nsb, U, CH);
   arm(1);
   if (H == 1024) {
-    klaunch(k_grp_up<1024, 16, NT>, gu_grid, NT, 0, s, m, k, inter, g);
+    klaunch(k_grp_up<1024, 16, NT>, gu_grid, NT, 0, s, m, k, inter, nsb, g);
   } else {
-    klaunch(k_grp_up<1536, 16, NT>, gu_grid, NT, 0, s, m, k, inter, g);
+    klaunch(k_grp_up<1536, 16, NT>, gu_grid, NT, 0, s, m, k, inter, nsb, g);
   }
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  const dim3 dn_grid(H / 64, U, CH);
+  const dim3 dn_grid(H / 64 * nsb, U, CH);
   arm(2);
   switch (inter) {
 #define DOWN_CASE(II)                                                                               \
   case II:                                                                                          \
-    klaunch(k_grp_down<II, 16>, dn_grid, 256, 0, s, H, g);                                      \
+    klaunch(k_grp_down<II, 16>, dn_grid, 256, 0, s, H, nsb, g);                                      \
     break;
     DOWN_CASE(128)
     DOWN_CASE(256)

@@ -1,4 +1,4 @@
-// Dense half of the multi-position step in grouped mode: the q/k/v and output projections of m <= 32 positions as
+// Dense half of the multi-position step in grouped mode: the q/k/v and output projections of the positions as
 // int8 MFMA GEMMs over the tiled Q8_0 weights (the dense kernels of the reference's block prefill,
 // rust/moe-rt/src/cuda_dense.rs:236-288, whose per-position GEMVs this replaces by one pass over each weight row),
 // the RMSNorms and 15-bit activation codes that feed them, and the experts' combine with the residual.
@@ -10,6 +10,7 @@
 // largest element.
 //
 // Kernels:
+// (grids for up to 32 positions; the dense kernels take a longer pass in groups of 32)
 //   k_gd_dense<K, NM, GD_QKV>  grid 2 * rows/64:  rows 16h..16h+15 and 32+16h..32+16h+15 of one head (h = half),
 //                                                 RoPE on the (j, j+32) pairs, q in f32, K and V into the fp16 cache
 //   k_gd_dense<K, NM, GD_RES>  grid rows/32:      32 rows of the output projection, h += res * (Wo att)
@@ -41,6 +42,9 @@ template <int K, int NM, int EPI>
 __global__ __launch_bounds__(kGdThreads) void k_gd_dense(TMat w, int m, const int8_t* __restrict__ xh,
                                                          const int8_t* __restrict__ xl, const float* __restrict__ xd,
                                                          GdEpi ep) {
+  // the positions of a longer pass NM at a time: blockIdx.x = row tile + row tiles * group
+  const int tiles = w.rows / 32, tile = blockIdx.x % tiles, c0 = blockIdx.x / tiles * NM;
+  m = min(m - c0, NM);
   constexpr int NB = K / 32, NBW = NB / 4, STR = K + 16;
   static_assert(NB % 8 == 0, "each K quarter is whole pairs of blocks");
   __shared__ __align__(16) int8_t bh[NM * STR];
@@ -50,12 +54,12 @@ __global__ __launch_bounds__(kGdThreads) void k_gd_dense(TMat w, int m, const in
   __shared__ float red[4][32][NM + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int p = wave & 1, kq = wave >> 1;
-  const int row0 = EPI == GD_QKV ? (blockIdx.x >> 1) * 64 + 16 * (blockIdx.x & 1) + 32 * p : 32 * blockIdx.x + 16 * p;
+  const int row0 = EPI == GD_QKV ? (tile >> 1) * 64 + 16 * (tile & 1) + 32 * p : 32 * tile + 16 * p;
   const size_t t16 = (size_t)row0 / 16;
   TileScales<NBW> sc;
   fetch_scales<NBW>(w, t16, NB, kq * NBW, sc);
   Members<K, NM, kGdThreads> mb;
-  fetch_members<K, NM, kGdThreads, true>(xh, xl, xd, 0u, 0, m, mb);
+  fetch_members<K, NM, kGdThreads, true>(xh, xl, xd, 0u, c0, m, mb);
   uint4 a[NBW / 2];
   fetch_tile_q8<NBW>(w, t16, NB, kq * NBW, a);
   store_scales<NBW>(sc, sdt[wave]);
@@ -75,11 +79,11 @@ __global__ __launch_bounds__(kGdThreads) void k_gd_dense(TMat w, int m, const in
     const int jj = threadIdx.x & 15, c = threadIdx.x >> 4;
     if (c >= NM || c >= m) return;
     const float x1 = sum(jj, c), x2 = sum(16 + jj, c);
-    const int head = blockIdx.x >> 1, jp = 16 * (blockIdx.x & 1) + jj;
-    const int pos = ep.pos0 + c;
+    const int head = tile >> 1, jp = 16 * (tile & 1) + jj;
+    const int pos = ep.pos0 + c0 + c;
     const float cs = ep.rope[(size_t)pos * 64 + jp], sn = ep.rope[(size_t)pos * 64 + 32 + jp];
     if (head < ep.heads) {
-      float* qv = ep.q + (size_t)c * ep.heads * 64 + head * 64;
+      float* qv = ep.q + (size_t)(c0 + c) * ep.heads * 64 + head * 64;
       qv[jp] = x1 * cs - x2 * sn;
       qv[jp + 32] = x2 * cs + x1 * sn;
     } else if (head < ep.heads + ep.kvh) {
@@ -95,7 +99,7 @@ __global__ __launch_bounds__(kGdThreads) void k_gd_dense(TMat w, int m, const in
     for (int it = threadIdx.x; it < 32 * NM; it += kGdThreads) {
       const int r = it & 31, c = it >> 5;
       if (c < m) {
-        float* hp = ep.h + (size_t)c * w.rows + 32 * blockIdx.x + r;
+        float* hp = ep.h + (size_t)(c0 + c) * w.rows + 32 * tile + r;
         *hp = *hp + ep.res * sum(r, c);
       }
     }
@@ -152,12 +156,15 @@ __global__ __launch_bounds__(256) void k_gd_combine(int k, float res, float* __r
                                                     const float* __restrict__ lnw, float eps, GroupBufs g) {
   constexpr int NP = (H + 1023) / 1024;
   const int p = blockIdx.x, t = threadIdx.x;
+  const int sb = p / kGrpMaxPos, pl = p % kGrpMaxPos;  // the step of the pass and its position
+  const int* plan = g.grp + (size_t)sb * GRP_WORDS;
+  const float* o = g.o + (size_t)sb * kGrpMaxPos * 8 * H;
   int sl[8];
   float wt[8];
 #pragma unroll
   for (int j = 0; j < 8; j++) {
-    sl[j] = j < k ? g.grp[GRP_ORD_SLOT + p * 8 + j] : 0;
-    wt[j] = j < k ? __int_as_float(g.grp[GRP_ORD_W + p * 8 + j]) : 0.0f;
+    sl[j] = j < k ? plan[GRP_ORD_SLOT + pl * 8 + j] : 0;
+    wt[j] = j < k ? __int_as_float(plan[GRP_ORD_W + pl * 8 + j]) : 0.0f;
   }
   float hv[NP][4];
   float ss = 0.0f;
@@ -169,7 +176,7 @@ __global__ __launch_bounds__(256) void k_gd_combine(int k, float res, float* __r
     float4 ov[8];
 #pragma unroll
     for (int u = 0; u < 8; u++)
-      ov[u] = u < k ? *reinterpret_cast<const float4*>(g.o + (size_t)sl[u] * H + ec) : make_float4(0, 0, 0, 0);
+      ov[u] = u < k ? *reinterpret_cast<const float4*>(o + (size_t)sl[u] * H + ec) : make_float4(0, 0, 0, 0);
     float4* hp = reinterpret_cast<float4*>(h + (size_t)p * H + ec);
     const float4 ho = *hp;
     float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -198,7 +205,7 @@ __global__ __launch_bounds__(256) void k_gd_combine(int k, float res, float* __r
 template <int K, int EPI>
 static void dense_launch(hipStream_t s, int grid, const TMat& w, int m, const GroupBufs& g, const GdEpi& ep) {
   if (m > 16)
-    klaunch(k_gd_dense<K, 32, EPI>, grid, kGdThreads, 0, s, w, m, g.xh, g.xl, g.xd, ep);
+    klaunch(k_gd_dense<K, 32, EPI>, grid * ((m + 31) / 32), kGdThreads, 0, s, w, m, g.xh, g.xl, g.xd, ep);
   else
     klaunch(k_gd_dense<K, 16, EPI>, grid, kGdThreads, 0, s, w, m, g.xh, g.xl, g.xd, ep);
 }
@@ -206,7 +213,7 @@ static void dense_launch(hipStream_t s, int grid, const TMat& w, int m, const Gr
 hipError_t launch_gd_qkv(hipStream_t s, const Dims& d, int m, int pos0, const float* rope, float* q, uint16_t* kc,
                          uint16_t* vc, const GroupBufs& g) {
   const TMat& w = g.qkv;
-  if (m < 1 || m > kGrpMaxPos || !w.q || d.head_dim != 64 || w.rows != (d.heads + 2 * d.kv_heads) * 64 ||
+  if (m < 1 || m > g.cap || !w.q || d.head_dim != 64 || w.rows != (d.heads + 2 * d.kv_heads) * 64 ||
       w.cols != d.hidden || pos0 < 0 || pos0 + m > d.max_len)
     return hipErrorInvalidValue;
   GdEpi ep{rope, pos0, d.heads, d.kv_heads, d.max_len, q, kc, vc, nullptr, 0.0f};
@@ -221,7 +228,7 @@ hipError_t launch_gd_qkv(hipStream_t s, const Dims& d, int m, int pos0, const fl
 
 hipError_t launch_gd_oproj(hipStream_t s, int m, float res, float* h, const GroupBufs& g) {
   const TMat& w = g.oproj;
-  if (m < 1 || m > kGrpMaxPos || !w.q || w.rows % 32) return hipErrorInvalidValue;
+  if (m < 1 || m > g.cap || !w.q || w.rows % 32) return hipErrorInvalidValue;
   GdEpi ep{nullptr, 0, 0, 0, 0, nullptr, nullptr, nullptr, h, res};
   switch (w.cols) {
     case 1024: dense_launch<1024, GD_RES>(s, w.rows / 32, w, m, g, ep); break;
@@ -233,7 +240,7 @@ hipError_t launch_gd_oproj(hipStream_t s, int m, float res, float* h, const Grou
 
 hipError_t launch_norm_codes(hipStream_t s, int H, int m, const float* h, const float* lnw, float eps,
                              const GroupBufs& g) {
-  if (m < 1 || m > kGrpMaxPos || !lnw) return hipErrorInvalidValue;
+  if (m < 1 || m > g.cap || !lnw) return hipErrorInvalidValue;
   switch (H) {
     case 1024: klaunch(k_gd_norm_codes<1024>, m, 256, 0, s, h, lnw, eps, g); break;
     case 1536: klaunch(k_gd_norm_codes<1536>, m, 256, 0, s, h, lnw, eps, g); break;
@@ -244,7 +251,7 @@ hipError_t launch_norm_codes(hipStream_t s, int H, int m, const float* h, const 
 
 hipError_t launch_gd_combine(hipStream_t s, int H, int m, int k, float res, float* h, const float* lnw, float eps,
                              const GroupBufs& g) {
-  if (m < 1 || m > kGrpMaxPos || k < 1 || k > 8) return hipErrorInvalidValue;
+  if (m < 1 || m > g.cap || k < 1 || k > 8) return hipErrorInvalidValue;
   switch (H) {
     case 1024: klaunch(k_gd_combine<1024>, m, 256, 0, s, k, res, h, lnw, eps, g); break;
     case 1536: klaunch(k_gd_combine<1536>, m, 256, 0, s, k, res, h, lnw, eps, g); break;

@@ -660,7 +660,7 @@ hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const
 
 hipError_t launch_layer_grouped(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* state,
                                 int pos0, int nv, const float* rope, const GroupBufs& g, const float* next_lnw) {
-  if (nv < 1 || nv > p.cap || nv > kGrpMaxPos || d.top_k > 8 || d.experts > 64 || d.head_dim != 64) return hipErrorInvalidValue;
+  if (nv < 1 || nv > p.cap || nv > g.cap || d.top_k > 8 || d.experts > 64 || d.head_dim != 64) return hipErrorInvalidValue;
   GroupBufs gg = g;
   gg.ids = p.ids;
   gg.w = p.w;
