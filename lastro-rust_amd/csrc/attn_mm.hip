@@ -44,7 +44,7 @@ __global__ __launch_bounds__(T * 64, 4) void k_attn_mm(const float* __restrict__
                                                    const uint16_t* __restrict__ vc, const int* __restrict__ lenp,
                                                    int len_add, int max_len, float scale, int tps, int kvh, int splits,
                                                    int ny, float* __restrict__ part) {
-  constexpr int NA = (4 + T - 1) / T;  // dim blocks of a wave in the combine: w, w + T, ...
+  constexpr int NR = (4 + T - 1) / T;  // quads of dims of a wave in the combine: w, w + T, ... of a lane's four
   __shared__ __align__(16) mm_f4 Pv[T][4][64];
   __shared__ __align__(16) float Qs[kMmUnits][68];  // rows 4 banks apart: a lane group's 16-byte reads do not collide
   __shared__ float Tm[T][16], Al[T][16], Ts[T][16];
@@ -67,9 +67,9 @@ __global__ __launch_bounds__(T * 64, 4) void k_attn_mm(const float* __restrict__
         gload_f4(q + ((size_t)(fu / G) * nh + g * G + fu % G) * 64 + 4 * (f & 15));
   }
   float m = NEG_INF, l = 0.0f;
-  mm_f4 acc[NA];
+  mm_f4 acc[NR];
 #pragma unroll
-  for (int a = 0; a < NA; a++) acc[a] = mm_f4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int a = 0; a < NR; a++) acc[a] = mm_f4{0.0f, 0.0f, 0.0f, 0.0f};
   for (int tr = t0; tr < t1; tr += T) {
     // a wave past the split's tiles goes through its last tile with no row valid and nothing of it is used: a branch
     // around the loads would keep their registers live through the whole loop (129 spilled at 128 registers)
@@ -194,14 +194,15 @@ __global__ __launch_bounds__(T * 64, 4) void k_attn_mm(const float* __restrict__
         }
       }
     }
+    // quad r of the lane: dims 16 gq + 4 r .. +3 of its unit, element r of the four dim blocks
     if constexpr (T == 1) {
       if (nv > 0) {
         l = __builtin_fmaf(l, alpha, ts);
         m = mn;
 #pragma unroll
-        for (int a = 0; a < NA; a++)
+        for (int r = 0; r < 4; r++)
 #pragma unroll
-          for (int r = 0; r < 4; r++) acc[a][r] = __builtin_fmaf(acc[a][r], alpha, pv[a][r]);
+          for (int a = 0; a < 4; a++) acc[r][a] = __builtin_fmaf(acc[r][a], alpha, pv[a][r]);
       }
     } else {
       if (gq == 0) {
@@ -209,7 +210,7 @@ __global__ __launch_bounds__(T * 64, 4) void k_attn_mm(const float* __restrict__
         Ts[w][i] = ts;
       }
 #pragma unroll
-      for (int a = 0; a < 4; a++) Pv[w][a][lane] = pv[a];
+      for (int r = 0; r < 4; r++) Pv[w][r][lane] = mm_f4{pv[0][r], pv[1][r], pv[2][r], pv[3][r]};
       __syncthreads();  // p.v, alpha and sums of every tile of the round
 #pragma unroll
       for (int v = 0; v < T; v++) {
@@ -218,11 +219,11 @@ __global__ __launch_bounds__(T * 64, 4) void k_attn_mm(const float* __restrict__
           l = __builtin_fmaf(l, a1, Ts[v][i]);
           m = m > Tm[v][i] ? m : Tm[v][i];
 #pragma unroll
-          for (int a = 0; a < NA; a++) {
-            if (w + T * a < 4) {
-              const mm_f4 x = Pv[v][w + T * a][lane];
+          for (int r = 0; r < NR; r++) {
+            if (w + T * r < 4) {
+              const mm_f4 x = Pv[v][w + T * r][lane];
 #pragma unroll
-              for (int r = 0; r < 4; r++) acc[a][r] = __builtin_fmaf(acc[a][r], a1, x[r]);
+              for (int a = 0; a < 4; a++) acc[r][a] = __builtin_fmaf(acc[r][a], a1, x[a]);
             }
           }
         }
@@ -233,11 +234,15 @@ __global__ __launch_bounds__(T * 64, 4) void k_attn_mm(const float* __restrict__
   if (u >= units || t0 * 64 >= len0 + y) return;
   float* pp = part + (head * splits + s) * 66;
   if (w == 0 && gq == 0) *reinterpret_cast<float2*>(pp) = make_float2(m, l);
+  // 8-byte stores of consecutive dims (one dword at a time, 16 lines to a store, took 62 us where this takes 42: 300
+  // positions after 1000, 3B shape, one tile per split)
+  float2* po = reinterpret_cast<float2*>(pp + 2 + 16 * gq);
 #pragma unroll
-  for (int a = 0; a < NA; a++)
-    if (w + T * a < 4)
-#pragma unroll
-      for (int r = 0; r < 4; r++) pp[2 + 16 * gq + 4 * r + w + T * a] = acc[a][r];
+  for (int r = 0; r < NR; r++)
+    if (w + T * r < 4) {
+      po[2 * (w + T * r)] = make_float2(acc[r][0], acc[r][1]);
+      po[2 * (w + T * r) + 1] = make_float2(acc[r][2], acc[r][3]);
+    }
 }
 
 hipError_t launch_attn_mm(hipStream_t s, int G, int kvh, int tps, const float* q, const uint16_t* kc,
