@@ -26,6 +26,7 @@
 #include "placement.h"
 #include "cache.h"
 #include "grouped.h"
+#include "hostio.h"
 #include "kernels.h"
 #include "layers.h"
 #include "moe_norm.h"
@@ -193,12 +194,19 @@ bool k_supported(int k) { return k == 128 || k == 256 || k == 512 || k == 1024 |
 
 // ------------------------------------------------------------------------------------------------------------
 // GpuModel (rust/moe-rt/src/gpu_model.rs:180-445).
+// The step state {pos, fixed, 0, 0}, and with seq the token of position pos.
+__global__ static void k_set_state(int* state, int pos, int fixed, int* seq, int token) {
+  if (threadIdx.x < ST_WORDS) state[threadIdx.x] = threadIdx.x == ST_POS ? pos : threadIdx.x == ST_FIXED ? fixed : 0;
+  if (seq && threadIdx.x == 0) seq[pos] = token;
+}
+
 struct moert_model {
   moert_config cfg{};
   Dims dims{};
   int max_len = 0, splits = 0, host_pos = 0;
   bool poisoned = false;
   hipStream_t stream = nullptr;
+  HostIo io;
   Arena arena;
   std::vector<LayerDev> layers;
   DMat embed{};
@@ -510,6 +518,7 @@ struct moert_model {
     if (rc == MOERT_E_DEVICE) {
       poisoned = true;
       (void)hipStreamSynchronize(stream);
+      io.finish(false);
     }
     return rc;
   }
@@ -633,10 +642,15 @@ struct moert_model {
     return MOERT_OK;
   }
 
+  // In stream order: nothing waits for it.
+  int set_state(int pos, int fixed, int* seq, int token) {
+    hipLaunchKernelGGL(k_set_state, 1, 64, 0, stream, b.state, pos, fixed, seq, token);
+    CHECK_HIP(hipGetLastError());
+    return MOERT_OK;
+  }
   int write_state(int pos, int fixed) {
-    int st[ST_WORDS] = {pos, fixed, 0, 0};
-    CHECK_HIP(hipMemcpyAsync(b.state, st, sizeof st, hipMemcpyHostToDevice, stream));
-    CHECK_HIP(hipStreamSynchronize(stream));
+    const int rc = set_state(pos, fixed, nullptr, 0);
+    if (rc) return rc;
     host_pos = pos;
     return MOERT_OK;
   }
@@ -884,6 +898,11 @@ static int model_create(const moert_config* c, const moert_model_weights* w, int
     set_err("hipStreamCreate failed");
     return bail(MOERT_E_DEVICE);
   }
+  // results of a step: the logits, routing and error words; tokens in, K/V rows out
+  if (m->io.create((size_t)c->vocab * 4 + (1u << 20)) != hipSuccess) {
+    set_err("pinned buffer for the results");
+    return bail(MOERT_E_DEVICE);
+  }
   hipStream_t s = m->stream;
   Arena& a = m->arena;
   int rc;
@@ -988,6 +1007,7 @@ static int model_create(const moert_config* c, const moert_model_weights* w, int
 struct moert_block {
   Dims dims{};
   hipStream_t stream = nullptr;
+  HostIo io;
   Arena arena;
   LayerDev L{};
   StepBufs b{};
@@ -1252,11 +1272,11 @@ int moert_model_destroy(moert_model* m) {
   } while (0)
 
 static int model_copy_in(moert_model* m, void* dst, const void* src, size_t bytes) {
-  CHECK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, m->stream));
+  CHECK_HIP(m->io.in(m->stream, dst, src, bytes));
   return MOERT_OK;
 }
 static int model_copy_out(moert_model* m, void* dst, const void* src, size_t bytes) {
-  CHECK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, m->stream));
+  CHECK_HIP(m->io.out(m->stream, dst, src, bytes));
   return MOERT_OK;
 }
 // MOERT_GRAPH=0 launches the step's kernels one by one instead of replaying the captured graph (for tracing
@@ -1299,18 +1319,11 @@ static int model_launch(moert_model* m) {
 // or the new K/V row of a KV head, 4 = the split partials of a merge, 8 = the act vector of an expert; k_layer only:
 // 32 = the merged heads (device-wide), 64 = h' (device-wide), 128 = the merged heads or h' in the XCD's L2, or the
 // router items.
-static int ab_check(moert_model* m) {
-  if (m->hybrid && m->hy_err) {
-    unsigned he = 0;
-    CHECK_HIP(hipMemcpy(&he, m->hy_err, 4, hipMemcpyDeviceToHost));
-    if (he) {
-      set_err("hybrid step: a layer's doorbell was not rung in time (error bits %#x)", he);
-      return MOERT_E_DEVICE;
-    }
+static int ab_report(unsigned he, unsigned e) {
+  if (he) {
+    set_err("hybrid step: a layer's doorbell was not rung in time (error bits %#x)", he);
+    return MOERT_E_DEVICE;
   }
-  if (!m->use_ab) return MOERT_OK;
-  unsigned e = 0;
-  CHECK_HIP(hipMemcpy(&e, m->ab.err, 4, hipMemcpyDeviceToHost));
   if (e) {
     set_err("%s%s%s%s%s%s%sgave up (error bits %#x): the launch's workgroups were not dispatched round-robin over the "
             "XCDs or not all resident at once",
@@ -1325,9 +1338,21 @@ static int ab_check(moert_model* m) {
   }
   return MOERT_OK;
 }
+static int ab_check(moert_model* m) {
+  unsigned he = 0, e = 0;
+  if (m->hybrid && m->hy_err) CHECK_HIP(hipMemcpy(&he, m->hy_err, 4, hipMemcpyDeviceToHost));
+  if (!he && m->use_ab) CHECK_HIP(hipMemcpy(&e, m->ab.err, 4, hipMemcpyDeviceToHost));
+  return ab_report(he, e);
+}
+// Waits for the stream, with the registered results and the error words behind it.
 static int model_sync(moert_model* m) {
+  unsigned he = 0, e = 0;
+  if (m->hybrid && m->hy_err) CHECK_HIP(m->io.out(m->stream, &he, m->hy_err, 4));
+  if (m->use_ab) CHECK_HIP(m->io.out(m->stream, &e, m->ab.err, 4));
+  CHECK_HIP(m->io.flush(m->stream));
   CHECK_HIP(hipStreamSynchronize(m->stream));
-  return ab_check(m);
+  m->io.finish(true);
+  return ab_report(he, e);
 }
 
 // ---- runtime metrics during moert_generate ----
@@ -1472,9 +1497,7 @@ int moert_decode_step(moert_model* m, int token, float* logits, int* route_ids, 
     return MOERT_E_RANGE;
   }
   int pos = m->host_pos;
-  int st[2] = {pos, pos + 1};
-  MTRY(m, model_copy_in(m, m->b.seq + pos, &token, 4));
-  MTRY(m, model_copy_in(m, m->b.state, st, sizeof st));
+  MTRY(m, m->set_state(pos, pos + 1, m->b.seq, token));
   MTRY(m, model_launch(m));
   const moert_config& c = m->cfg;
   if (logits) MTRY(m, model_copy_out(m, logits, m->b.logits, (size_t)c.vocab * 4));
@@ -2138,6 +2161,11 @@ int moert_block_create(int hidden, int inter, int experts, int top_k, const moer
     return bail(MOERT_E_DEVICE);
   }
   b->dims = Dims{hidden, inter, 1, 1, 64, hidden, experts, top_k, 64, 1, 0.0f, 1.0f, 1.0f, 1.0f, 1.0f};
+  // inputs and outputs of a step of kGrpMaxPos positions, routing and error word
+  if (b->io.create((size_t)kGrpMaxPos * (2 * hidden + 2 * 8) * 4 + 4096) != hipSuccess) {
+    set_err("pinned buffer for the results");
+    return bail(MOERT_E_DEVICE);
+  }
   hipStream_t s = b->stream;
   Arena& a = b->arena;
   int rc;
@@ -2171,12 +2199,15 @@ int moert_block_destroy(moert_block* b) {
 int moert_block_forward(moert_block* b, const float* x, float* y, int* ids, float* weights) {
   CHECK_CFG(b && x, "null argument");
   const Dims& d = b->dims;
-  CHECK_HIP(hipMemcpyAsync(b->x, x, (size_t)d.hidden * 4, hipMemcpyHostToDevice, b->stream));
+  CHECK_HIP(b->io.restart(b->stream));
+  CHECK_HIP(b->io.in(b->stream, b->x, x, (size_t)d.hidden * 4));
   TRY(b->enqueue());
-  if (y) CHECK_HIP(hipMemcpyAsync(y, b->b.logits, (size_t)d.hidden * 4, hipMemcpyDeviceToHost, b->stream));
-  if (ids) CHECK_HIP(hipMemcpyAsync(ids, b->b.route_ids, (size_t)d.top_k * 4, hipMemcpyDeviceToHost, b->stream));
-  if (weights) CHECK_HIP(hipMemcpyAsync(weights, b->b.route_w, (size_t)d.top_k * 4, hipMemcpyDeviceToHost, b->stream));
+  if (y) CHECK_HIP(b->io.out(b->stream, y, b->b.logits, (size_t)d.hidden * 4));
+  if (ids) CHECK_HIP(b->io.out(b->stream, ids, b->b.route_ids, (size_t)d.top_k * 4));
+  if (weights) CHECK_HIP(b->io.out(b->stream, weights, b->b.route_w, (size_t)d.top_k * 4));
+  CHECK_HIP(b->io.flush(b->stream));
   CHECK_HIP(hipStreamSynchronize(b->stream));
+  b->io.finish(true);
   return MOERT_OK;
 }
 
@@ -2212,12 +2243,15 @@ int moert_block_forward_batched(moert_block* b, int m, const float* x, float* y,
   TRY(check_grouped(b, m));
   const Dims& d = b->dims;
   CHECK_CFG(!b->fused || m <= kFbPos, "batched step: the one-launch kernel takes at most %d positions", kFbPos);
-  CHECK_HIP(hipMemcpyAsync(b->gx, x, (size_t)m * d.hidden * 4, hipMemcpyHostToDevice, b->stream));
+  CHECK_HIP(b->io.restart(b->stream));
+  CHECK_HIP(b->io.in(b->stream, b->gx, x, (size_t)m * d.hidden * 4));
   TRY(b->launch_batched(b->stream, m, nullptr));
-  if (y) CHECK_HIP(hipMemcpyAsync(y, b->gy, (size_t)m * d.hidden * 4, hipMemcpyDeviceToHost, b->stream));
-  if (ids) CHECK_HIP(hipMemcpyAsync(ids, b->g.ids, (size_t)m * d.top_k * 4, hipMemcpyDeviceToHost, b->stream));
-  if (weights) CHECK_HIP(hipMemcpyAsync(weights, b->g.w, (size_t)m * d.top_k * 4, hipMemcpyDeviceToHost, b->stream));
+  if (y) CHECK_HIP(b->io.out(b->stream, y, b->gy, (size_t)m * d.hidden * 4));
+  if (ids) CHECK_HIP(b->io.out(b->stream, ids, b->g.ids, (size_t)m * d.top_k * 4));
+  if (weights) CHECK_HIP(b->io.out(b->stream, weights, b->g.w, (size_t)m * d.top_k * 4));
+  CHECK_HIP(b->io.flush(b->stream));
   CHECK_HIP(hipStreamSynchronize(b->stream));
+  b->io.finish(true);
   return b->fused_check();
 }
 
