@@ -2442,15 +2442,13 @@ int moert_attn_decode(const float* q, const uint16_t* k_cache, const uint16_t* v
   TRY(sc.init());
   float *dq, *part, *dout;
   uint16_t *dk, *dv;
-  int* dlen;
   size_t kvn = (size_t)kv_heads * max_len * 64;
   TRY(sc.dev(&dq, (size_t)heads * 64, q));
   TRY(sc.dev(&dk, kvn, k_cache));
   TRY(sc.dev(&dv, kvn, v_cache));
   TRY(sc.dev(&part, (size_t)heads * attn_splits_for(max_len, tiles_per_split) * 66));
-  TRY(sc.dev(&dlen, 1, &len));
   TRY(sc.dev(&dout, (size_t)heads * 64));
-  CHECK_HIP(launch_attn_unit(sc.s, dq, dk, dv, heads, kv_heads, max_len, dlen, scale, tiles_per_split, part, dout));
+  CHECK_HIP(launch_attn_unit(sc.s, dq, dk, dv, heads, kv_heads, max_len, len, scale, tiles_per_split, part, dout));
   TRY(sc.get(out, dout, (size_t)heads * 64 * 4));
   return MOERT_OK;
 }
@@ -2472,10 +2470,8 @@ int moert_attn_decode_noalloc(const float* q_dev, const uint16_t* k_cache_dev, c
   uint8_t* base = (uint8_t*)noalloc_scratch(&e);
   CHECK_HIP(e);
   hipStream_t s = (hipStream_t)stream;
-  int* lenp = (int*)base;
   float* part = (float*)(base + kNoallocHeader);
-  CHECK_HIP(launch_set_int(s, lenp, len));
-  CHECK_HIP(launch_attn_unit(s, q_dev, k_cache_dev, v_cache_dev, heads, kv_heads, max_len, lenp, scale,
+  CHECK_HIP(launch_attn_unit(s, q_dev, k_cache_dev, v_cache_dev, heads, kv_heads, max_len, len, scale,
                              tiles_per_split, part, out_dev));
   return MOERT_OK;
 }

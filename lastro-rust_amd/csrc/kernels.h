@@ -156,8 +156,7 @@ hipError_t launch_copy(hipStream_t s, const void* src, void* dst, size_t bytes);
 hipError_t launch_read(hipStream_t s, const void* src, size_t bytes, unsigned* out);
 int read_probe_blocks(size_t bytes);
 hipError_t launch_attn_unit(hipStream_t s, const float* q, const uint16_t* kc, const uint16_t* vc, int heads,
-                            int kv_heads, int max_len, const int* len_dev, float scale, int tps, float* part,
-                            float* out);
+                            int kv_heads, int max_len, int len, float scale, int tps, float* part, float* out);
 // Splits of a cache of max_len positions with tps 64-position tiles per split.
 int attn_splits_for(int max_len, int tps);
 

@@ -215,7 +215,7 @@ __global__ __launch_bounds__(256) void k_attn_split(const float* __restrict__ q,
   const int t0 = s * tps;
   // q and the length first (loads complete in issue order), then the first tile's K rows and V shares
   const float qv = q[h * 64 + lane];
-  const int len = *lenp + len_add;
+  const int len = (lenp ? *lenp : 0) + len_add;
   __builtin_amdgcn_sched_barrier(0);
   Row8 kn;
   kn.load(reinterpret_cast<const uint4*>(K + (size_t)(t0 * 64 + lane) * 64));
@@ -297,21 +297,27 @@ __global__ __launch_bounds__(256) void k_attn_split(const float* __restrict__ q,
 // alpha_t = exp(m_{t-1} - m_t), p_t = exp(s - m_t), the tile sum and p.v are formed in parallel; the first wave of
 // each head then applies l = fma(l, alpha_t, sum_t) and acc = fma(acc, alpha_t, pv_t) over the tiles in order.
 // Every operation and its order are those of the sequential kernel, so the partials are the same bit for bit.
-template <int G, int T>
+// The tiles stay in fp16 in LDS (K by rows, V transposed, converted at their use): two workgroups of 3 heads x 4 tiles
+// fit a compute unit, where f32 tiles took 152 KB, so that the 512 of a 16384-position cache run in one round (a whole
+// call over 16001 positions of 24 heads 19.2 -> 14.1 us, with the length as an argument).
+//
+// ALL: the workgroup has every tile of the length (at most T) and forms all splits of `tps` tiles and their combine
+// (k_attn_combine's operations), writing the output row itself: one launch for a short context.
+template <int G, int T, bool ALL = false>
 __global__ __launch_bounds__(G * T * 64) void k_attn_tiles(const float* __restrict__ q, const uint16_t* __restrict__ kc,
                                                           const uint16_t* __restrict__ vc, const int* __restrict__ lenp,
-                                                          int len_add, int max_len, float scale, int splits,
+                                                          int len_add, int max_len, float scale, int splits, int tps,
                                                           float* __restrict__ part, Tl tl) {
   TL_START(tl);
   constexpr int TR = 8 % G == 0 ? 64 : 72;  // tile rows (64..71: padding for VShare when G does not divide 8)
-  constexpr int KS = 68;                     // K row stride in floats: 16-byte rows, conflict-free row reads
-  __shared__ __align__(16) float Vs[T][TR][64];  // V tiles in f32, row i = position
-  __shared__ __align__(16) float Ks[T][TR][KS];  // K tiles in f32, row i = position
-  __shared__ float Qs[G][64];
-  __shared__ float Ps[G][T][64];
+  constexpr int KS = 72;                    // K row stride in halves: 16-byte rows, conflict-free row reads
+  __shared__ __align__(16) uint16_t Vs[T][64 * 64];  // V tiles transposed (VShare::store_ht)
+  __shared__ __align__(16) uint16_t Ks[T][TR][KS];   // K tiles, row i = position
+  __shared__ __align__(16) float Qs[G][64];
+  __shared__ __align__(16) float Ps[G][T][64];
   __shared__ float Pv[G][T][64];
   __shared__ float Tm[G][T], Al[G][T], Ts[G][T];
-  const int g = blockIdx.x / splits, s = blockIdx.x % splits;
+  const int g = ALL ? blockIdx.x : blockIdx.x / splits, s = ALL ? 0 : blockIdx.x % splits;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int wh = wid % G, wt = wid / G;
   const int h = g * G + wh;
@@ -323,9 +329,9 @@ __global__ __launch_bounds__(G * T * 64) void k_attn_tiles(const float* __restri
   // T does not divide the tile count) reads the cache's last tile instead and is never used
   const int tc = min(t, max_len / 64 - 1);
   // q and the length first (loads complete in issue order), then this wave's shares of the tile's K and V (the G
-  // waves of a tile move it together, each element is loaded and converted once)
+  // waves of a tile move it together, each element is loaded once)
   const float qv = q[h * 64 + lane];
-  const int len = *lenp + len_add;
+  const int len = (lenp ? *lenp : 0) + len_add;
   __builtin_amdgcn_sched_barrier(0);
   VShare<G> ksh;
   ksh.load(K, tc, lane, wh);
@@ -337,33 +343,38 @@ __global__ __launch_bounds__(G * T * 64) void k_attn_tiles(const float* __restri
   const int used = min(T, nb - t0);  // tiles of this split inside the length (>= 1 when the split is used)
   const bool active = wt < used;
   const int nv = active ? min(64, len - t * 64) : 0;
-  ksh.template store<KS>(&Ks[wt][0][0], lane, wh, nv);
+  ksh.template store_h<KS>(&Ks[wt][0][0], lane, wh, nv);
   __syncthreads();  // Qs, K tiles
   TL_PHASE(tl, 2);
   // scores: lane = position, chain over the 64 dims in order (an inactive tile's scores are discarded)
   float sc;
   {
     float dt = 0.0f;
-    const float* krow = &Ks[wt][lane][0];
+    const uint16_t* krow = &Ks[wt][lane][0];
 #pragma unroll
-    for (int d4 = 0; d4 < 16; d4++) {
-      const float4 kk = *reinterpret_cast<const float4*>(krow + 4 * d4);
-      const float4 qq = *reinterpret_cast<const float4*>(&Qs[wh][4 * d4]);
-      dt = __builtin_fmaf(qq.x, kk.x, dt);
-      dt = __builtin_fmaf(qq.y, kk.y, dt);
-      dt = __builtin_fmaf(qq.z, kk.z, dt);
-      dt = __builtin_fmaf(qq.w, kk.w, dt);
+    for (int e = 0; e < 8; e++) {
+      const uint4 ke = *reinterpret_cast<const uint4*>(krow + 8 * e);
+      const uint32_t wv[4] = {ke.x, ke.y, ke.z, ke.w};
+#pragma unroll
+      for (int hh = 0; hh < 2; hh++) {
+        const float4 qq = *reinterpret_cast<const float4*>(&Qs[wh][8 * e + 4 * hh]);
+        const float qa[4] = {qq.x, qq.y, qq.z, qq.w};
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+          dt = __builtin_fmaf(qa[c], h2f((uint16_t)(wv[2 * hh + (c >> 1)] >> (16 * (c & 1)))), dt);
+      }
     }
     sc = lane < nv ? dt * scale : NEG_INF;  // nv = 0 for an inactive tile
   }
   const float tmax = group_max<64>(sc);
   if (lane == 0) Tm[wh][wt] = tmax;
-  __syncthreads();  // tile maxima
+  vsh.store_ht(&Vs[wt][0], lane, wh, nv);
+  __syncthreads();  // tile maxima; every share of every V tile stored
   TL_PHASE(tl, 3);
   float pv = 0.0f;
   if (active) {
     float mprev = NEG_INF;
-    for (int u = 0; u < wt; u++) mprev = mprev > Tm[wh][u] ? mprev : Tm[wh][u];
+    for (int u = ALL ? wt / tps * tps : 0; u < wt; u++) mprev = mprev > Tm[wh][u] ? mprev : Tm[wh][u];
     const float mn = mprev > tmax ? mprev : tmax;
     const float alpha = dexp(mprev - mn);
     const float p = dexp(sc - mn);
@@ -373,40 +384,23 @@ __global__ __launch_bounds__(G * T * 64) void k_attn_tiles(const float* __restri
       Al[wh][wt] = alpha;
       Ts[wh][wt] = ts;
     }
-  }
-  vsh.template store<64>(&Vs[wt][0][0], lane, wh, nv);
-  __syncthreads();  // every share of every V tile stored; P written
-  TL_PHASE(tl, 4);
-  if (active) {
+    wave_lds_sync();
+    TL_PHASE(tl, 4);
     // p.v: lane = dim, chain over the positions in order, without branches so that every LDS read can be issued
     // ahead of the chain. A position past the length has p = exp(-inf) = 0 and its V element is stored as 0, so
     // its step fma(0, 0, pv) returns pv unchanged (pv starts at +0 and an exact zero sum is +0, so pv is never -0):
     // the chain equals the one over the valid positions only, bit for bit.
-    const float* vcol = &Vs[wt][0][lane];
-    if constexpr (G * T < 16) {
+    const uint16_t* vrow = &Vs[wt][lane * 64];
+    const int key = (lane ^ (lane >> 3)) & 7;  // VShare::vt_col's permutation of the 8-position chunks of a dim
 #pragma unroll
-      for (int i0 = 0; i0 < 64; i0 += 4) {
-        const float4 p4 = *reinterpret_cast<const float4*>(&Ps[wh][wt][i0]);
-        const float pa[4] = {p4.x, p4.y, p4.z, p4.w};
+    for (int c = 0; c < 8; c++) {
+      const uint4 ve = *reinterpret_cast<const uint4*>(vrow + 8 * (c ^ key));
+      const uint32_t wv[4] = {ve.x, ve.y, ve.z, ve.w};
+      const float4 p0 = *reinterpret_cast<const float4*>(&Ps[wh][wt][8 * c]);
+      const float4 p1 = *reinterpret_cast<const float4*>(&Ps[wh][wt][8 * c + 4]);
+      const float pa[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
 #pragma unroll
-        for (int u = 0; u < 4; u++) pv = __builtin_fmaf(pa[u], vcol[(i0 + u) * 64], pv);
-      }
-    } else {
-      // 16 waves leave 128 VGPRs a lane, too few to hoist every read: batches of 8 positions, valid ones only
-#pragma unroll
-      for (int i0 = 0; i0 < 64; i0 += 8) {
-        if (i0 < nv) {
-          float vf[8];
-#pragma unroll
-          for (int u = 0; u < 8; u++) vf[u] = vcol[(i0 + u) * 64];
-          const float4 p0 = *reinterpret_cast<const float4*>(&Ps[wh][wt][i0]);
-          const float4 p1 = *reinterpret_cast<const float4*>(&Ps[wh][wt][i0 + 4]);
-          const float pa[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-#pragma unroll
-          for (int u = 0; u < 8; u++)
-            if (i0 + u < nv) pv = __builtin_fmaf(pa[u], vf[u], pv);
-        }
-      }
+      for (int u = 0; u < 8; u++) pv = __builtin_fmaf(pa[u], h2f((uint16_t)(wv[u >> 1] >> (16 * (u & 1)))), pv);
     }
     if (wt > 0) Pv[wh][wt][lane] = pv;
   }
@@ -417,18 +411,58 @@ __global__ __launch_bounds__(G * T * 64) void k_attn_tiles(const float* __restri
     return;
   }
   float m = NEG_INF, l = 0.0f, acc = 0.0f;
-  for (int u = 0; u < used; u++) {
+  auto add = [&](int u) {
     const float a = Al[wh][u];
     l = __builtin_fmaf(l, a, Ts[wh][u]);
     acc = __builtin_fmaf(acc, a, u == 0 ? pv : Pv[wh][u][lane]);
     m = m > Tm[wh][u] ? m : Tm[wh][u];
+  };
+  if constexpr (ALL) {
+    float ms[T], ls[T], av[T], M = NEG_INF;
+    int n = 0;  // splits
+#pragma unroll
+    for (int u = 0; u < T; u++) {
+      ms[u] = NEG_INF;
+      ls[u] = av[u] = 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < T; u++) {
+      if (u < used) {
+        add(u);
+        if ((u + 1) % tps == 0 || u + 1 == used) {  // the split's last tile
+#pragma unroll
+          for (int i = 0; i < T; i++)
+            if (i == n) {
+              ms[i] = m;
+              ls[i] = l;
+              av[i] = acc;
+            }
+          M = M > m ? M : m;
+          n++;
+          m = NEG_INF;
+          l = acc = 0.0f;
+        }
+      }
+    }
+    float den = 0.0f, num = 0.0f;
+#pragma unroll
+    for (int i = 0; i < T; i++) {
+      if (i < n) {
+        const float ws = dexp(ms[i] - M);
+        den = __builtin_fmaf(ws, ls[i], den);
+        num = __builtin_fmaf(ws, av[i], num);
+      }
+    }
+    part[h * 64 + lane] = num / den;
+  } else {
+    for (int u = 0; u < used; u++) add(u);
+    float* pp = part + ((size_t)h * splits + s) * 66;
+    if (lane == 0) {
+      pp[0] = m;
+      pp[1] = l;
+    }
+    pp[2 + lane] = acc;
   }
-  float* pp = part + ((size_t)h * splits + s) * 66;
-  if (lane == 0) {
-    pp[0] = m;
-    pp[1] = l;
-  }
-  pp[2 + lane] = acc;
   TL_END(tl);
 }
 
@@ -453,7 +487,7 @@ __global__ __launch_bounds__(64) void k_attn_combine(const float* __restrict__ p
   const int sl = min(lane, splits - 1);
   float ms = base[(size_t)sl * 66];
   float ls = base[(size_t)sl * 66 + 1];
-  const int len = *lenp + len_add;
+  const int len = (lenp ? *lenp : 0) + len_add;
   const int nb = (len + 63) / 64, used = (nb + tps - 1) / tps;
   if (lane >= used) {
     ms = NEG_INF;
@@ -1167,7 +1201,7 @@ static hipError_t attn_split_dispatch(hipStream_t s, int G, int kvh, int tps, co
   const dim3 blocks(kvh * splits);
 #define TILES_CASE(GG, TT)                                                                                   \
   if (G == GG && tps == TT) {                                                                                \
-    klaunch(k_attn_tiles<GG, TT>, blocks, GG * TT * 64, 0, s, q, kc, vc, lenp, len_add, max_len, scale, splits, part, tl); \
+    klaunch(k_attn_tiles<GG, TT>, blocks, GG * TT * 64, 0, s, q, kc, vc, lenp, len_add, max_len, scale, splits, tps, part, tl); \
     return hipGetLastError();                                                                                \
   }
   TILES_CASE(1, 1) TILES_CASE(2, 1) TILES_CASE(3, 1) TILES_CASE(4, 1)
@@ -1219,11 +1253,25 @@ hipError_t launch_attn_combine(hipStream_t s, const Dims& d, const StepBufs& b, 
 }
 
 hipError_t launch_attn_unit(hipStream_t s, const float* q, const uint16_t* kc, const uint16_t* vc, int heads,
-                            int kv_heads, int max_len, const int* len_dev, float scale, int tps, float* part,
-                            float* out) {
-  hipError_t e = attn_split_dispatch(s, heads / kv_heads, kv_heads, tps, q, kc, vc, len_dev, 0, max_len, scale, part);
+                            int kv_heads, int max_len, int len, float scale, int tps, float* part, float* out) {
+  // A length of at most 4 tiles in one launch, a workgroup per KV head: the second launch costs more than the tiles
+  // (100 positions, 16 heads, a call among others: 13.9 us as length, splits and combine, 7.2 as one).
+  const int G = heads / kv_heads, nb = (len + 63) / 64;
+  if (max_len % 64) return hipErrorInvalidValue;
+#define ALL_CASE(GG, TT)                                                                                         \
+  if (G == GG && nb == TT) {                                                                                     \
+    klaunch(k_attn_tiles<GG, TT, true>, kv_heads, GG * TT * 64, 0, s, q, kc, vc, (const int*)nullptr, len, max_len, \
+            scale, 1, tps, out, Tl{});                                                                           \
+    return hipGetLastError();                                                                                    \
+  }
+  ALL_CASE(1, 1) ALL_CASE(2, 1) ALL_CASE(3, 1) ALL_CASE(4, 1)
+  ALL_CASE(1, 2) ALL_CASE(2, 2) ALL_CASE(3, 2) ALL_CASE(4, 2)
+  ALL_CASE(1, 3) ALL_CASE(2, 3) ALL_CASE(3, 3) ALL_CASE(4, 3)
+  ALL_CASE(1, 4) ALL_CASE(2, 4) ALL_CASE(3, 4) ALL_CASE(4, 4)
+#undef ALL_CASE
+  hipError_t e = attn_split_dispatch(s, G, kv_heads, tps, q, kc, vc, nullptr, len, max_len, scale, part);
   if (e != hipSuccess) return e;
-  return attn_combine_dispatch(s, heads, tps, max_len, len_dev, 0, part, out);
+  return attn_combine_dispatch(s, heads, tps, max_len, nullptr, len, part, out);
 }
 
 hipError_t launch_oproj(hipStream_t s, const LayerDev& L, const Dims& d, const StepBufs& b, Tl tl, bool from_hc) {

@@ -5,8 +5,8 @@
 // stand-in, never passed to a kernel or a copy), and that address is what the kernels get.
 //
 // Every call on a GPU uses that GPU's one array: calls that overlap on one GPU (other streams, other threads) race
-// on it. Nothing in it has to start at zero: the length word is written by k_set_int on every call, and the attention
-// kernels read only the partials of the splits they wrote in the same call.
+// on it. Nothing in it has to start at zero: the attention kernels read only the partials of the splits they wrote in
+// the same call.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -22,10 +22,6 @@ namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
 void* g_ptr[kMaxDevices] = {};
-
-__global__ void k_set_int(int* p, int v) {
-  if (threadIdx.x == 0) *p = v;
-}
 
 }  // namespace
 
@@ -46,11 +42,6 @@ void* noalloc_scratch(hipError_t* err) {
   }
   *err = hipSuccess;
   return g_ptr[dev];
-}
-
-hipError_t launch_set_int(hipStream_t s, int* p, int v) {
-  hipLaunchKernelGGL(k_set_int, 1, 64, 0, s, p, v);
-  return hipGetLastError();
 }
 
 }  // namespace moert
