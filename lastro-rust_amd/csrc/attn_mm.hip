@@ -1,5 +1,5 @@
 // Split-KV attention of a multi-position step on the f32 matrix cores, bit for bit equal to the decode kernels
-// (k_attn_split / k_attn_tiles, kernels.hip).
+// (k_attn_tiles, kernels.hip).
 //
 // The f32 MFMAs are fused multiply-add chains: v_mfma_f32_16x16x1 adds one product to every element of its four
 // 16x16 blocks, and v_mfma_f32_16x16x4 adds its four products in the order of k, each step rounded as fmaf rounds it

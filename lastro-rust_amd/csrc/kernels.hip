@@ -170,140 +170,26 @@ __global__ __launch_bounds__(kQkvWaves * 64) void k_qkv(DMat m, const float* __r
 
 // ------------------------------------------------------------------------------------------------------------
 // Split-KV GQA decode attention over the fp16 cache, two kernels (attn_split + attn_combine, gpu.rs:205-292).
-// k_attn_split: one wave per (KV head g, split s) serves all G query heads of g, so each K/V byte is read once.
-// Lane i holds the K row of position i of a tile in registers (scores: lane = position); V goes straight from HBM
-// to the wave's LDS (p.v: lane = dim), double buffered: the next tile's K and V are requested before the current
-// tile's scores are computed. Partials (m, l, acc[64]) per (head, split).
+// k_attn_tiles: one workgroup per (KV head g, split s) serves all G query heads of g, so each K/V byte is read once;
+// partials (m, l, acc[64]) per (head, split).
 // k_attn_combine: one wave per query head merges the used splits in split order, all partials loaded at once.
 
-// A 128-byte row held in named registers (an array copied to LDS in a loop is turned into a memcpy from a stack
-// slot by the compiler).
-struct Row8 {
-  uint4 a, b, c, d, e, f, g, h;
-  __device__ __forceinline__ void load(const uint4* p) {
-    a = p[0]; b = p[1]; c = p[2]; d = p[3]; e = p[4]; f = p[5]; g = p[6]; h = p[7];
-  }
-  // member i for a compile-time i (unrolled loops)
-  __device__ __forceinline__ uint4 at(int i) const {
-    return i == 0 ? a : i == 1 ? b : i == 2 ? c : i == 3 ? d : i == 4 ? e : i == 5 ? f : i == 6 ? g : h;
-  }
-};
-
-template <int G>
-__global__ __launch_bounds__(256) void k_attn_split(const float* __restrict__ q, const uint16_t* __restrict__ kc,
-                                                   const uint16_t* __restrict__ vc, const int* __restrict__ lenp,
-                                                   int len_add, int max_len, float scale, int tps, int splits,
-                                                   float* __restrict__ part) {
-  // workgroup = G waves, wave w serves query head g*G + w; the K rows are read by every wave (L2 after the first),
-  // the V tile is moved into LDS once, each wave carrying a share of its rows
-  __shared__ uint4 Vs[2][64][8];  // fp16 V tiles, row i = position
-  __shared__ float Qs[G][64];
-  __shared__ float Ps[G][64];
-  const int g = blockIdx.x / splits, s = blockIdx.x % splits;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int h = g * G + w;
-  const float NEG_INF = __int_as_float(0xff800000);
-  const uint16_t* K = kc + (size_t)g * max_len * 64;
-  const uint16_t* V = vc + (size_t)g * max_len * 64;
-  auto v_share = [&](int t, int buf) {
-    const uint16_t* src = V + ((size_t)t * 64 + (lane >> 3)) * 64 + (lane & 7) * 8;
-    for (int e = w; e < 8; e += G)
-      __builtin_amdgcn_global_load_lds(src + (size_t)e * 8 * 64, &Vs[buf][8 * e][0], 16, 0, 0);
-  };
-  // split s covers tiles [s*tps, s*tps + tps); its first tile is requested before the length is known (the grid
-  // only covers tiles inside the cache)
-  const int t0 = s * tps;
-  // q and the length first (loads complete in issue order), then the first tile's K rows and V shares
-  const float qv = q[h * 64 + lane];
-  const int len = (lenp ? *lenp : 0) + len_add;
-  __builtin_amdgcn_sched_barrier(0);
-  Row8 kn;
-  kn.load(reinterpret_cast<const uint4*>(K + (size_t)(t0 * 64 + lane) * 64));
-  v_share(t0, 0);
-  Qs[w][lane] = qv;
-  const int nb = (len + 63) / 64;
-  if (t0 >= nb) {
-    __builtin_amdgcn_s_waitcnt(0);  // the tile copy into LDS has finished before the wave ends
-    return;
-  }
-  const int t1 = min(t0 + tps, nb);
-  float m = NEG_INF, l = 0.0f, acc = 0.0f;
-  for (int t = t0; t < t1; t++) {
-    const int nv = min(64, len - t * 64), buf = (t - t0) & 1;
-    const Row8 kr = kn;
-    __syncthreads();  // Qs written; every wave is done with the buffer the prefetch overwrites
-    if (t + 1 < t1) {
-      kn.load(reinterpret_cast<const uint4*>(K + (size_t)((t + 1) * 64 + lane) * 64));
-      v_share(t + 1, buf ^ 1);
-    }
-    // scores: lane = position, chain over the 64 dims in order
-    float dt = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const uint4 ke = kr.at(e);
-      const uint32_t wv[4] = {ke.x, ke.y, ke.z, ke.w};
-#pragma unroll
-      for (int hh = 0; hh < 2; hh++) {
-        const float4 qv = *reinterpret_cast<const float4*>(&Qs[w][8 * e + 4 * hh]);
-        const float qa[4] = {qv.x, qv.y, qv.z, qv.w};
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const uint32_t word = wv[2 * hh + (c >> 1)];
-          dt = __builtin_fmaf(qa[c], h2f((uint16_t)(word >> (16 * (c & 1)))), dt);
-        }
-      }
-    }
-    const float sc = lane < nv ? dt * scale : NEG_INF;
-    const float tmax = group_max<64>(sc);
-    const float mn = m > tmax ? m : tmax;
-    const float alpha = dexp(m - mn);
-    const float p = dexp(sc - mn);
-    const float ts = group_sum<64>(p);
-    l = __builtin_fmaf(l, alpha, ts);
-    Ps[w][lane] = p;
-    m = mn;
-    __builtin_amdgcn_s_waitcnt(0);  // this wave's share of the tile's V rows has landed in LDS
-    __syncthreads();                // every share has
-    // p.v: lane = dim, chain over the valid positions in order; LDS reads batched 8 positions at a time
-    const uint16_t* vcol = reinterpret_cast<const uint16_t*>(&Vs[buf][0][0]) + lane;
-    float pv = 0.0f;
-#pragma unroll
-    for (int i0 = 0; i0 < 64; i0 += 8) {
-      if (i0 < nv) {
-        float vf[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) vf[u] = h2f(vcol[(i0 + u) * 64]);
-        const float4 p0 = *reinterpret_cast<const float4*>(&Ps[w][i0]);
-        const float4 p1 = *reinterpret_cast<const float4*>(&Ps[w][i0 + 4]);
-        const float pa[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-          if (i0 + u < nv) pv = __builtin_fmaf(pa[u], vf[u], pv);
-      }
-    }
-    acc = __builtin_fmaf(acc, alpha, pv);
-  }
-  float* pp = part + ((size_t)h * splits + s) * 66;
-  if (lane == 0) {
-    pp[0] = m;
-    pp[1] = l;
-  }
-  pp[2 + lane] = acc;
-}
-
-// Tile-parallel form of k_attn_split for a split of exactly T tiles: workgroup = G x T waves, wave (wh, wt) takes
-// query head g*G + wh and tile t0 + wt. Every wave computes its tile's scores and tile max at once; the running max
+// Workgroup = G x T waves, wave (wh, wt) takes query head g*G + wh and tile t0 + wt of the split (T = its tiles; 4 and
+// rounds of 4 for a split of more: the 32 tiles of a split one after the other in one
+// wave per head took 66 us where this takes 25: 5000 positions, 16 heads, splits of 32 tiles).
+// Every wave computes its tile's scores and tile max at once; the running max
 // m_{t-1} each tile's online-softmax step needs is the max of the earlier tiles' maxima (exchanged through LDS), so
 // alpha_t = exp(m_{t-1} - m_t), p_t = exp(s - m_t), the tile sum and p.v are formed in parallel; the first wave of
-// each head then applies l = fma(l, alpha_t, sum_t) and acc = fma(acc, alpha_t, pv_t) over the tiles in order.
-// Every operation and its order are those of the sequential kernel, so the partials are the same bit for bit.
+// each head then applies l = fma(l, alpha_t, sum_t) and acc = fma(acc, alpha_t, pv_t) over the tiles in order:
+// the operations and the order of one tile after the other.
 // The tiles stay in fp16 in LDS (K by rows, V transposed, converted at their use): two workgroups of 3 heads x 4 tiles
 // fit a compute unit, where f32 tiles took 152 KB, so that the 512 of a 16384-position cache run in one round (a whole
 // call over 16001 positions of 24 heads 19.2 -> 14.1 us, with the length as an argument).
 //
-// ALL: the workgroup has every tile of the length (at most T) and forms all splits of `tps` tiles and their combine
+// TILES_ALL: the workgroup has every tile of the length (at most T) and forms all splits of `tps` tiles and their combine
 // (k_attn_combine's operations), writing the output row itself: one launch for a short context.
-template <int G, int T, bool ALL = false>
+enum { TILES_ONE, TILES_ROUNDS, TILES_ALL };  // the split has T tiles, or more; every split in one workgroup
+template <int G, int T, int FORM>
 __global__ __launch_bounds__(G * T * 64) void k_attn_tiles(const float* __restrict__ q, const uint16_t* __restrict__ kc,
                                                           const uint16_t* __restrict__ vc, const int* __restrict__ lenp,
                                                           int len_add, int max_len, float scale, int splits, int tps,
@@ -316,7 +202,8 @@ __global__ __launch_bounds__(G * T * 64) void k_attn_tiles(const float* __restri
   __shared__ __align__(16) float Qs[G][64];
   __shared__ __align__(16) float Ps[G][T][64];
   __shared__ float Pv[G][T][64];
-  __shared__ float Tm[G][T], Al[G][T], Ts[G][T];
+  __shared__ float Tm[G][T], Al[G][T], Ts[G][T], Mr[G];
+  constexpr bool ROUNDS = FORM == TILES_ROUNDS, ALL = FORM == TILES_ALL;
   const int g = ALL ? blockIdx.x : blockIdx.x / splits, s = ALL ? 0 : blockIdx.x % splits;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int wh = wid % G, wt = wid / G;
@@ -324,138 +211,152 @@ __global__ __launch_bounds__(G * T * 64) void k_attn_tiles(const float* __restri
   const float NEG_INF = __int_as_float(0xff800000);
   const uint16_t* K = kc + (size_t)g * max_len * 64;
   const uint16_t* V = vc + (size_t)g * max_len * 64;
-  const int t0 = s * T, t = t0 + wt;
+  const int t0 = s * (ROUNDS ? tps : T), last = max_len / 64 - 1;
   // the tile's rows are requested before the length is known; a tile past the end of the cache (last split, when
   // T does not divide the tile count) reads the cache's last tile instead and is never used
-  const int tc = min(t, max_len / 64 - 1);
   // q and the length first (loads complete in issue order), then this wave's shares of the tile's K and V (the G
   // waves of a tile move it together, each element is loaded once)
   const float qv = q[h * 64 + lane];
   const int len = (lenp ? *lenp : 0) + len_add;
   __builtin_amdgcn_sched_barrier(0);
   VShare<G> ksh;
-  ksh.load(K, tc, lane, wh);
+  ksh.load(K, min(t0 + wt, last), lane, wh);
   __builtin_amdgcn_sched_barrier(0);  // K (needed first) ahead of V
   VShare<G> vsh;
-  vsh.load(V, tc, lane, wh);
+  vsh.load(V, min(t0 + wt, last), lane, wh);
   Qs[wh][lane] = qv;  // every wave of head wh stores the same q (an unconditional store keeps the q load first)
-  const int nb = (len + 63) / 64;
-  const int used = min(T, nb - t0);  // tiles of this split inside the length (>= 1 when the split is used)
-  const bool active = wt < used;
-  const int nv = active ? min(64, len - t * 64) : 0;
-  ksh.template store_h<KS>(&Ks[wt][0][0], lane, wh, nv);
-  __syncthreads();  // Qs, K tiles
-  TL_PHASE(tl, 2);
-  // scores: lane = position, chain over the 64 dims in order (an inactive tile's scores are discarded)
-  float sc;
-  {
-    float dt = 0.0f;
-    const uint16_t* krow = &Ks[wt][lane][0];
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const uint4 ke = *reinterpret_cast<const uint4*>(krow + 8 * e);
-      const uint32_t wv[4] = {ke.x, ke.y, ke.z, ke.w};
-#pragma unroll
-      for (int hh = 0; hh < 2; hh++) {
-        const float4 qq = *reinterpret_cast<const float4*>(&Qs[wh][8 * e + 4 * hh]);
-        const float qa[4] = {qq.x, qq.y, qq.z, qq.w};
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-          dt = __builtin_fmaf(qa[c], h2f((uint16_t)(wv[2 * hh + (c >> 1)] >> (16 * (c & 1)))), dt);
-      }
-    }
-    sc = lane < nv ? dt * scale : NEG_INF;  // nv = 0 for an inactive tile
-  }
-  const float tmax = group_max<64>(sc);
-  if (lane == 0) Tm[wh][wt] = tmax;
-  vsh.store_ht(&Vs[wt][0], lane, wh, nv);
-  __syncthreads();  // tile maxima; every share of every V tile stored
-  TL_PHASE(tl, 3);
-  float pv = 0.0f;
-  if (active) {
-    float mprev = NEG_INF;
-    for (int u = ALL ? wt / tps * tps : 0; u < wt; u++) mprev = mprev > Tm[wh][u] ? mprev : Tm[wh][u];
-    const float mn = mprev > tmax ? mprev : tmax;
-    const float alpha = dexp(mprev - mn);
-    const float p = dexp(sc - mn);
-    const float ts = group_sum<64>(p);
-    Ps[wh][wt][lane] = p;
-    if (lane == 0) {
-      Al[wh][wt] = alpha;
-      Ts[wh][wt] = ts;
-    }
-    wave_lds_sync();
-    TL_PHASE(tl, 4);
-    // p.v: lane = dim, chain over the positions in order, without branches so that every LDS read can be issued
-    // ahead of the chain. A position past the length has p = exp(-inf) = 0 and its V element is stored as 0, so
-    // its step fma(0, 0, pv) returns pv unchanged (pv starts at +0 and an exact zero sum is +0, so pv is never -0):
-    // the chain equals the one over the valid positions only, bit for bit.
-    const uint16_t* vrow = &Vs[wt][lane * 64];
-    const int key = (lane ^ (lane >> 3)) & 7;  // VShare::vt_col's permutation of the 8-position chunks of a dim
-#pragma unroll
-    for (int c = 0; c < 8; c++) {
-      const uint4 ve = *reinterpret_cast<const uint4*>(vrow + 8 * (c ^ key));
-      const uint32_t wv[4] = {ve.x, ve.y, ve.z, ve.w};
-      const float4 p0 = *reinterpret_cast<const float4*>(&Ps[wh][wt][8 * c]);
-      const float4 p1 = *reinterpret_cast<const float4*>(&Ps[wh][wt][8 * c + 4]);
-      const float pa[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-#pragma unroll
-      for (int u = 0; u < 8; u++) pv = __builtin_fmaf(pa[u], h2f((uint16_t)(wv[u >> 1] >> (16 * (u & 1)))), pv);
-    }
-    if (wt > 0) Pv[wh][wt][lane] = pv;
-  }
-  __syncthreads();  // p.v of every tile
-  TL_PHASE(tl, 5);
-  if (wt != 0 || used <= 0) {
-    TL_END(tl);
-    return;
-  }
+  const int nb = (len + 63) / 64, t1 = ROUNDS ? min(t0 + tps, nb) : nb;  // tiles [t0, t1), at most T without rounds
   float m = NEG_INF, l = 0.0f, acc = 0.0f;
-  auto add = [&](int u) {
-    const float a = Al[wh][u];
-    l = __builtin_fmaf(l, a, Ts[wh][u]);
-    acc = __builtin_fmaf(acc, a, u == 0 ? pv : Pv[wh][u][lane]);
-    m = m > Tm[wh][u] ? m : Tm[wh][u];
-  };
-  if constexpr (ALL) {
-    float ms[T], ls[T], av[T], M = NEG_INF;
-    int n = 0;  // splits
+  for (int tr = t0;; tr += T) {
+    const int t = tr + wt;
+    const int used = min(T, t1 - tr);  // tiles of this round inside the split and the length (>= 1 when it is used)
+    const bool active = wt < used;
+    const int nv = active ? min(64, len - t * 64) : 0;
+    ksh.template store_h<KS>(&Ks[wt][0][0], lane, wh, nv);
+    __syncthreads();  // Qs, K tiles
+    TL_PHASE(tl, 2);
+    // scores: lane = position, chain over the 64 dims in order (an inactive tile's scores are discarded)
+    float sc;
+    {
+      float dt = 0.0f;
+      const uint16_t* krow = &Ks[wt][lane][0];
 #pragma unroll
-    for (int u = 0; u < T; u++) {
-      ms[u] = NEG_INF;
-      ls[u] = av[u] = 0.0f;
-    }
+      for (int e = 0; e < 8; e++) {
+        const uint4 ke = *reinterpret_cast<const uint4*>(krow + 8 * e);
+        const uint32_t wv[4] = {ke.x, ke.y, ke.z, ke.w};
 #pragma unroll
-    for (int u = 0; u < T; u++) {
-      if (u < used) {
-        add(u);
-        if ((u + 1) % tps == 0 || u + 1 == used) {  // the split's last tile
+        for (int hh = 0; hh < 2; hh++) {
+          const float4 qq = *reinterpret_cast<const float4*>(&Qs[wh][8 * e + 4 * hh]);
+          const float qa[4] = {qq.x, qq.y, qq.z, qq.w};
 #pragma unroll
-          for (int i = 0; i < T; i++)
-            if (i == n) {
-              ms[i] = m;
-              ls[i] = l;
-              av[i] = acc;
-            }
-          M = M > m ? M : m;
-          n++;
-          m = NEG_INF;
-          l = acc = 0.0f;
+          for (int c = 0; c < 4; c++)
+            dt = __builtin_fmaf(qa[c], h2f((uint16_t)(wv[2 * hh + (c >> 1)] >> (16 * (c & 1)))), dt);
         }
       }
+      sc = lane < nv ? dt * scale : NEG_INF;  // nv = 0 for an inactive tile
     }
-    float den = 0.0f, num = 0.0f;
-#pragma unroll
-    for (int i = 0; i < T; i++) {
-      if (i < n) {
-        const float ws = dexp(ms[i] - M);
-        den = __builtin_fmaf(ws, ls[i], den);
-        num = __builtin_fmaf(ws, av[i], num);
+    const float tmax = group_max<64>(sc);
+    if (lane == 0) Tm[wh][wt] = tmax;
+    if (ROUNDS && wt == 0 && lane == 0) Mr[wh] = m;  // the maximum of the rounds before
+    vsh.store_ht(&Vs[wt][0], lane, wh, nv);
+    if (ROUNDS && tr + T < t1) {  // the next round's tiles arrive behind this one's
+      ksh.load(K, min(t + T, last), lane, wh);
+      vsh.load(V, min(t + T, last), lane, wh);
+    }
+    __syncthreads();  // tile maxima; every share of every V tile stored
+    TL_PHASE(tl, 3);
+    float pv = 0.0f;
+    if (active) {
+      float mprev = ROUNDS ? Mr[wh] : NEG_INF;
+      for (int u = ALL ? wt / tps * tps : 0; u < wt; u++) mprev = mprev > Tm[wh][u] ? mprev : Tm[wh][u];
+      const float mn = mprev > tmax ? mprev : tmax;
+      const float alpha = dexp(mprev - mn);
+      const float p = dexp(sc - mn);
+      const float ts = group_sum<64>(p);
+      Ps[wh][wt][lane] = p;
+      if (lane == 0) {
+        Al[wh][wt] = alpha;
+        Ts[wh][wt] = ts;
       }
+      wave_lds_sync();
+      TL_PHASE(tl, 4);
+      // p.v: lane = dim, chain over the positions in order, without branches so that every LDS read can be issued
+      // ahead of the chain. A position past the length has p = exp(-inf) = 0 and its V element is stored as 0, so
+      // its step fma(0, 0, pv) returns pv unchanged (pv starts at +0 and an exact zero sum is +0, so pv is never -0):
+      // the chain equals the one over the valid positions only, bit for bit.
+      const uint16_t* vrow = &Vs[wt][lane * 64];
+      const int key = (lane ^ (lane >> 3)) & 7;  // VShare::vt_col's permutation of the 8-position chunks of a dim
+#pragma unroll
+      for (int c = 0; c < 8; c++) {
+        const uint4 ve = *reinterpret_cast<const uint4*>(vrow + 8 * (c ^ key));
+        const uint32_t wv[4] = {ve.x, ve.y, ve.z, ve.w};
+        const float4 p0 = *reinterpret_cast<const float4*>(&Ps[wh][wt][8 * c]);
+        const float4 p1 = *reinterpret_cast<const float4*>(&Ps[wh][wt][8 * c + 4]);
+        const float pa[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+#pragma unroll
+        for (int u = 0; u < 8; u++) pv = __builtin_fmaf(pa[u], h2f((uint16_t)(wv[u >> 1] >> (16 * (u & 1)))), pv);
+      }
+      if (wt > 0) Pv[wh][wt][lane] = pv;
     }
-    part[h * 64 + lane] = num / den;
-  } else {
-    for (int u = 0; u < used; u++) add(u);
+    __syncthreads();  // p.v of every tile
+    TL_PHASE(tl, 5);
+    if constexpr (!ALL) {
+      if (wt == 0) {
+        for (int u = 0; u < used; u++) {
+          const float a = Al[wh][u];
+          l = __builtin_fmaf(l, a, Ts[wh][u]);
+          acc = __builtin_fmaf(acc, a, u == 0 ? pv : Pv[wh][u][lane]);
+          m = m > Tm[wh][u] ? m : Tm[wh][u];
+        }
+      }
+      if (ROUNDS && tr + T < t1) {
+        __syncthreads();  // the round's entries are read
+        continue;
+      }
+    } else if (wt == 0) {
+      float ms[T], ls[T], av[T], M = NEG_INF;
+      int n = 0;  // splits
+#pragma unroll
+      for (int u = 0; u < T; u++) {
+        ms[u] = NEG_INF;
+        ls[u] = av[u] = 0.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < T; u++) {
+        if (u < used) {
+          const float a = Al[wh][u];
+          l = __builtin_fmaf(l, a, Ts[wh][u]);
+          acc = __builtin_fmaf(acc, a, u == 0 ? pv : Pv[wh][u][lane]);
+          m = m > Tm[wh][u] ? m : Tm[wh][u];
+          if ((u + 1) % tps == 0 || u + 1 == used) {  // the split's last tile
+#pragma unroll
+            for (int i = 0; i < T; i++)
+              if (i == n) {
+                ms[i] = m;
+                ls[i] = l;
+                av[i] = acc;
+              }
+            M = M > m ? M : m;
+            n++;
+            m = NEG_INF;
+            l = acc = 0.0f;
+          }
+        }
+      }
+      float den = 0.0f, num = 0.0f;
+#pragma unroll
+      for (int i = 0; i < T; i++) {
+        if (i < n) {
+          const float ws = dexp(ms[i] - M);
+          den = __builtin_fmaf(ws, ls[i], den);
+          num = __builtin_fmaf(ws, av[i], num);
+        }
+      }
+      part[h * 64 + lane] = num / den;
+    }
+    break;
+  }
+  if (wt == 0 && !ALL && t0 < t1) {
     float* pp = part + ((size_t)h * splits + s) * 66;
     if (lane == 0) {
       pp[0] = m;
@@ -1200,8 +1101,9 @@ static hipError_t attn_split_dispatch(hipStream_t s, int G, int kvh, int tps, co
   if (splits > 64 || max_len % 64) return hipErrorInvalidValue;
   const dim3 blocks(kvh * splits);
 #define TILES_CASE(GG, TT)                                                                                   \
-  if (G == GG && tps == TT) {                                                                                \
-    klaunch(k_attn_tiles<GG, TT>, blocks, GG * TT * 64, 0, s, q, kc, vc, lenp, len_add, max_len, scale, splits, tps, part, tl); \
+  if (G == GG && std::min(tps, 4) == TT) {                                                                   \
+    auto kernel = tps > TT ? k_attn_tiles<GG, TT, TT == 4 ? TILES_ROUNDS : TILES_ONE> : k_attn_tiles<GG, TT, TILES_ONE>; \
+    klaunch(kernel, blocks, GG * TT * 64, 0, s, q, kc, vc, lenp, len_add, max_len, scale, splits, tps, part, tl); \
     return hipGetLastError();                                                                                \
   }
   TILES_CASE(1, 1) TILES_CASE(2, 1) TILES_CASE(3, 1) TILES_CASE(4, 1)
@@ -1209,14 +1111,7 @@ static hipError_t attn_split_dispatch(hipStream_t s, int G, int kvh, int tps, co
   TILES_CASE(1, 3) TILES_CASE(2, 3) TILES_CASE(3, 3) TILES_CASE(4, 3)
   TILES_CASE(1, 4) TILES_CASE(2, 4) TILES_CASE(3, 4) TILES_CASE(4, 4)
 #undef TILES_CASE
-  switch (G) {
-    case 1: klaunch(k_attn_split<1>, blocks, 64, 0, s, q, kc, vc, lenp, len_add, max_len, scale, tps, splits, part); break;
-    case 2: klaunch(k_attn_split<2>, blocks, 128, 0, s, q, kc, vc, lenp, len_add, max_len, scale, tps, splits, part); break;
-    case 3: klaunch(k_attn_split<3>, blocks, 192, 0, s, q, kc, vc, lenp, len_add, max_len, scale, tps, splits, part); break;
-    case 4: klaunch(k_attn_split<4>, blocks, 256, 0, s, q, kc, vc, lenp, len_add, max_len, scale, tps, splits, part); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
 static hipError_t attn_combine_dispatch(hipStream_t s, int heads, int tps, int max_len, const int* lenp, int len_add,
@@ -1260,7 +1155,7 @@ hipError_t launch_attn_unit(hipStream_t s, const float* q, const uint16_t* kc, c
   if (max_len % 64) return hipErrorInvalidValue;
 #define ALL_CASE(GG, TT)                                                                                         \
   if (G == GG && nb == TT) {                                                                                     \
-    klaunch(k_attn_tiles<GG, TT, true>, kv_heads, GG * TT * 64, 0, s, q, kc, vc, (const int*)nullptr, len, max_len, \
+    klaunch(k_attn_tiles<GG, TT, TILES_ALL>, kv_heads, GG * TT * 64, 0, s, q, kc, vc, (const int*)nullptr, len, max_len, \
             scale, 1, tps, out, Tl{});                                                                           \
     return hipGetLastError();                                                                                    \
   }
