@@ -100,8 +100,14 @@ __global__ __launch_bounds__(T * 64, 4) void k_attn_mm(const float* __restrict__
 #pragma unroll
     for (int e = 0; e < 16; e++) vr[e] = gload_u2(vp + 4 * 64 * e);
     __builtin_amdgcn_sched_barrier(0);
+    // lo, hi: rows of the tile that the first and the last position see; whole tiles are not masked
+    const int lo = tw < t1 ? len0 + y_lo - t * 64 : 0, hi = len0 + y_hi - t * 64;
 #pragma unroll
-    for (int v = 0; v < 16; v++) p[v] = 4 * v < nv - gq ? sa[v] * scale : NEG_INF;
+    for (int v = 0; v < 16; v++) p[v] = sa[v] * scale;
+    if (lo < 64) {
+#pragma unroll
+      for (int v = 0; v < 16; v++) p[v] = 4 * v < nv - gq ? p[v] : NEG_INF;
+    }
     float tm;
     {
       float x[8];
@@ -124,12 +130,12 @@ __global__ __launch_bounds__(T * 64, 4) void k_attn_mm(const float* __restrict__
         if (v < w) mprev = mprev > Tm[v][i] ? mprev : Tm[v][i];
     }
     const float mn = mprev > tm ? mprev : tm;
-    const float alpha = dexp_sel(mprev - mn);
+    const float alpha = dexp_neg(mprev - mn);
     float ts;
     mm_f4 pv[4];
 #pragma unroll
     for (int v = 0; v < 16; v++) {
-      p[v] = dexp_sel(p[v] - mn);
+      p[v] = dexp_neg(p[v] - mn);
       if ((v & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // four exps side by side
     }
     // the pairwise tree over the 64 positions: bits 0, 1 of a position are the lane group, bits 2, 3 the element
@@ -151,7 +157,6 @@ __global__ __launch_bounds__(T * 64, 4) void k_attn_mm(const float* __restrict__
     // Rows past a unit's length have p = 0 and must not reach its sum. Rows that no unit sees enter as +0. A row
     // that only the later positions see stays (fma(0, v, c) is c for a finite v), unless it holds an inf or NaN:
     // then the tile is taken once per position, each with its own rows.
-    const int lo = len0 + y_lo - t * 64, hi = len0 + y_hi - t * 64;
     bool apart = false;
     if (lo < 64) {
       uint32_t bad = 0u;
@@ -162,30 +167,36 @@ __global__ __launch_bounds__(T * 64, 4) void k_attn_mm(const float* __restrict__
       }
       apart = __ballot(bad != 0u) != 0;
     }
-    {
-      const int rows = (apart ? lo : hi) - gq;
-#pragma unroll
-      for (int a = 0; a < 4; a++) pv[a] = mm_f4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int rows = (apart ? lo : hi) - gq;
+    if (lo < 64) {
 #pragma unroll
       for (int e = 0; e < 16; e++) {
         const bool in = 4 * e < rows;
-        const uint32_t x = in ? vr[e].x : 0u, z = in ? vr[e].y : 0u;
-        pv[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(half_of(x, 0), p[e], pv[0], 0, 0, 0);
-        pv[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(half_of(x, 1), p[e], pv[1], 0, 0, 0);
-        pv[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(half_of(z, 0), p[e], pv[2], 0, 0, 0);
-        pv[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(half_of(z, 1), p[e], pv[3], 0, 0, 0);
-        if (e & 1) __builtin_amdgcn_sched_barrier(0);
+        vr[e].x = in ? vr[e].x : 0u;
+        vr[e].y = in ? vr[e].y : 0u;
       }
     }
+#pragma unroll
+    for (int a = 0; a < 4; a++) pv[a] = mm_f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      pv[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(half_of(vr[e].x, 0), p[e], pv[0], 0, 0, 0);
+      pv[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(half_of(vr[e].x, 1), p[e], pv[1], 0, 0, 0);
+      pv[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(half_of(vr[e].y, 0), p[e], pv[2], 0, 0, 0);
+      pv[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(half_of(vr[e].y, 1), p[e], pv[3], 0, 0, 0);
+      if (e & 1) __builtin_amdgcn_sched_barrier(0);
+    }
     if (apart) {
+#pragma unroll
+      for (int e = 0; e < 16; e++) vr[e] = gload_u2(vp + 4 * 64 * e);  // unmasked again
       for (int yy = y_lo + 1; yy <= y_hi; yy++) {
-        const int rows = len0 + yy - t * 64 - gq;
+        const int rows_y = len0 + yy - t * 64 - gq;
 #pragma unroll
         for (int a = 0; a < 4; a++) {  // one block of dims at a time: few registers
           mm_f4 o = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
           for (int e = 0; e < 16; e++) {
-            uint32_t x = 4 * e < rows ? (a < 2 ? vr[e].x : vr[e].y) : 0u;
+            uint32_t x = 4 * e < rows_y ? (a < 2 ? vr[e].x : vr[e].y) : 0u;
             asm("" : "+v"(x));  // converted here: not shared with the first product, at 64 registers more
             o = __builtin_amdgcn_mfma_f32_16x16x4f32(half_of(x, a & 1), p[e], o, 0, 0, 0);
             if (e & 1) __builtin_amdgcn_sched_barrier(0);
