@@ -581,7 +581,8 @@ struct moert_model {
     int rc;
     if ((rc = mem(M * X, &mg.xh)) || (rc = mem(M * X, &mg.xl)) || (rc = mem(M * (X / 32) * 4, &mg.xd)) ||
         (rc = mem((size_t)M / kGrpMaxPos * GRP_WORDS * 4, &mg.grp)) || (rc = mem(S * I, &mg.ah)) ||
-        (rc = mem(S * I, &mg.al)) || (rc = mem(S * (I / 32) * 4, &mg.ad)) || (rc = mem(S * H * 4, &mg.o)))
+        (rc = mem(S * I, &mg.al)) || (rc = mem(S * (I / 32) * 4, &mg.ad)) || (rc = mem(S * H * 4, &mg.o)) ||
+        (rc = mem(64 * 4, &mg.cnt)) || (rc = mem((size_t)64 * M * 4, &mg.list)))
       return rc;
     mg.cap = M;
     return MOERT_OK;

@@ -40,25 +40,14 @@ struct GroupBufs {
   int8_t* al;    // the same: lo codes
   float* ad;     // [.., I/32] their block scales
   float* o;      // [.., H] down outputs by member slot
+  int* cnt;      // [64] members of each expert over the steps of a pass
+  int* list;     // [64, cap] the members: slot << 16 | position
   TMat gu, dn;   // gate_up [E*2I, H] and down [E*H, I] of the block in the tiled layout
   TMat qkv, oproj;  // the layer's q/k/v [(heads + 2 kv_heads) * 64, H] and output [H, heads * 64] projections, tiled
 };
 
-// Steps of a pass over m positions, and the buffers of step sb (its positions, its plan, its slots; H of the codes).
+// Steps of a pass over m positions.
 inline int grp_steps(int m) { return (m + kGrpMaxPos - 1) / kGrpMaxPos; }
-__device__ __forceinline__ GroupBufs grp_step(GroupBufs g, int sb, int k, int H, int I) {
-  const size_t p0 = (size_t)sb * kGrpMaxPos, s0 = p0 * 8;
-  g.ids += p0 * k;
-  g.w += p0 * k;
-  g.xh += p0 * H;
-  g.xl += p0 * H;
-  g.xd += p0 * (H / 32);
-  g.grp += (size_t)sb * GRP_WORDS;
-  g.ah += s0 * I;
-  g.al += s0 * I;
-  g.ad += s0 * (I / 32);
-  return g;
-}
 
 // Exchange buffers of the one-launch block (launch_grp_fused), zeroed at allocation. Entries are (value bits,
 // epoch) 8-byte words; the input codes are plain bytes published by a per-position epoch flag.

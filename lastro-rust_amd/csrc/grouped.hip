@@ -35,6 +35,7 @@ template <int H>
 __global__ __launch_bounds__(256) void k_grp_codes(const float* __restrict__ x, GroupBufs g) {
   constexpr int NB = H / 32;
   const int p = blockIdx.x;
+  if (p == 0 && g.cnt && threadIdx.x < 64) g.cnt[threadIdx.x] = 0;  // for k_grp_plan, behind this kernel
   for (int base = 0; base < NB; base += 256 / 8) {
     const int b = base + (threadIdx.x >> 3), part = threadIdx.x & 7;
     const bool valid = b < NB;
@@ -201,6 +202,23 @@ __device__ __forceinline__ void publish_plan(const Plan& s, const float* __restr
   }
 }
 
+// The plans of a pass of several steps: workgroup sb makes and publishes the plan of step sb and enters its members in
+// the experts' lists (their order in a list enters no result). The counts start at zero (k_grp_codes).
+__global__ __launch_bounds__(256) void k_grp_plan(int m, int k, GroupBufs g) {
+  __shared__ Plan plan;
+  __shared__ int base[64];
+  const int sb = blockIdx.x, p0 = sb * kGrpMaxPos, t = threadIdx.x;
+  m = min(m - p0, kGrpMaxPos);
+  make_plan<256>(g.ids + (size_t)p0 * k, m, k, plan);
+  publish_plan<256>(plan, g.w + (size_t)p0 * k, m, k, g.grp + (size_t)sb * GRP_WORDS);
+  if (t < 64) base[t] = plan.bits[t] ? atomicAdd(&g.cnt[t], __popc(plan.bits[t])) : 0;
+  __syncthreads();
+  if (t < m * k) {
+    const int e = plan.se[t], p = t / k, c = __popc(plan.bits[e] & ((1u << p) - 1u));
+    g.list[(size_t)e * g.cap + base[e] + c] = (sb * kGrpMaxPos * 8 + plan.offe[e] + c) << 16 | (p0 + p);
+  }
+}
+
 // ------------------------------------------------------------------------------------------------------------
 // Tiled copy of a Q8_0 matrix (TMat layout): thread i writes the 16-byte piece i = (tile, span, lane) and, for
 // lanes below 32, the scale of row lane%16 in block 2*span + lane/16.
@@ -236,11 +254,11 @@ hipError_t launch_tile_q8(hipStream_t s, const DMat& src, uint8_t* q, uint16_t* 
 constexpr int kGrpUpThreads = 512;
 
 //
-// A pass of several steps (nsb > 1) has the step inside blockIdx.x, tile + tiles * step, and blockIdx.y is the expert
-// itself: the workgroups of one weight tile follow each other, on the XCD of the tile where the tiles are a multiple
-// of 8, so that the steps share its read.
-template <int H, int NM, int NT>
-__global__ __launch_bounds__(NT) void k_grp_up(int m, int k, int inter, int nsb, GroupBufs gp) {
+// PASS: a pass of several steps, whose plans k_grp_plan made. The members of an expert over all steps stand in a list,
+// blockIdx.y is a tile of 16 of them (member_tile): an expert of a step of 32 positions fills 6 or 7 of the 16 columns
+// on average and ran in a workgroup per step (300 positions, 3B shape: gate/up 143 -> 65 us, down 55 -> 32).
+template <int H, int NM, int NT, bool PASS>
+__global__ __launch_bounds__(NT) void k_grp_up(int m, int k, int inter, GroupBufs g) {
   constexpr int NB = H / 32;
   constexpr int STR = H + 16;
   constexpr int WH = NT / 128;  // waves per half (gate or up)
@@ -253,23 +271,35 @@ __global__ __launch_bounds__(NT) void k_grp_up(int m, int k, int inter, int nsb,
   __shared__ __align__(16) uint16_t sdt[NT / 64][NB * 16];
   __shared__ float gout[2][RT][NM + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int tiles = inter / RT, sb = blockIdx.x / tiles, tile = blockIdx.x % tiles;
-  const GroupBufs g = grp_step(gp, sb, k, H, inter);
-  m = min(m - kGrpMaxPos * sb, kGrpMaxPos);
-  make_plan<NT>(g.ids, m, k, plan);
-  if (nsb == 1 && (int)blockIdx.y >= plan.nu) return;
-  const int c0 = NM * blockIdx.z;  // this workgroup's first member
-  const int e = nsb == 1 ? plan.list[blockIdx.y] : (int)blockIdx.y, off = plan.offe[e] + c0;
-  unsigned bits = plan.bits[e];
-  if (__popc(bits) <= c0) return;
-  for (int i = 0; i < c0; i++) bits &= bits - 1u;  // the members from c0 on
-  const int ne = __popc(bits);
+  const int tile = blockIdx.x;
+  int c0 = 0, ne = 0, e, off = 0;
+  unsigned bits = 0u;
+  const int* entry = nullptr;
+  if constexpr (PASS) {
+    int members = 0;
+    e = member_tile<NM>(g.cnt, blockIdx.y, lane, &c0, &members);
+    if (e < 0) return;
+    ne = min(members - c0, NM);
+    entry = g.list + (size_t)e * g.cap + c0;
+  } else {
+    make_plan<NT>(g.ids, m, k, plan);
+    if ((int)blockIdx.y >= plan.nu) return;
+    c0 = NM * blockIdx.z;  // this workgroup's first member
+    e = plan.list[blockIdx.y];
+    off = plan.offe[e] + c0;
+    bits = plan.bits[e];
+    if (__popc(bits) <= c0) return;
+    for (int i = 0; i < c0; i++) bits &= bits - 1u;  // the members from c0 on
+    ne = __popc(bits);
+  }
+  auto position = [&](int c) { return PASS ? entry[c] & 0xffff : nth_set_bit(bits, c); };
+  auto slot = [&](int c) { return PASS ? entry[c] >> 16 : off + c; };
   // this wave's 16 rows: gate (first half) or up (second half) rows [RT tile + 16 (wave % WH), +16) of expert e
   const size_t t16 = ((size_t)e * 2 * inter + (size_t)(wave / WH) * inter + RT * tile + 16 * (wave % WH)) / 16;
   TileScales<NB> sc;
   fetch_scales<NB>(g.gu, t16, NB, 0, sc);
   Members<H, NM, NT> mb;
-  fetch_members<H, NM, NT, false>(g.xh, g.xl, g.xd, bits, 0, ne, mb);
+  fetch_members<H, NM, NT>(g.xh, g.xl, g.xd, position, ne, mb);
   uint4 a[NB / 2];
   fetch_tile_q8<NB>(g.gu, t16, NB, 0, a);
   store_scales<NB>(sc, sdt[wave]);
@@ -308,21 +338,21 @@ __global__ __launch_bounds__(NT) void k_grp_up(int m, int k, int inter, int nsb,
       lw |= (uint32_t)(uint8_t)(int8_t)(q - 256 * h) << (8 * i);
     }
     if (valid) {
-      const size_t slotv = (size_t)(off + j);
+      const size_t slotv = (size_t)slot(j);
       const int blk = RT / 32 * tile + bi;
       reinterpret_cast<uint32_t*>(g.ah + slotv * inter + 32 * blk)[part] = hw;
       reinterpret_cast<uint32_t*>(g.al + slotv * inter + 32 * blk)[part] = lw;
       if (part == 0) g.ad[slotv * (inter / 32) + blk] = d;
     }
   }
-  if (e == plan.list[0] && tile == 0 && c0 == 0) publish_plan<NT>(plan, g.w, m, k, g.grp);
+  if (!PASS && blockIdx.y == 0 && tile == 0 && c0 == 0) publish_plan<NT>(plan, g.w, m, k, g.grp);
 }
 
 // ------------------------------------------------------------------------------------------------------------
 // Down of list expert u = blockIdx.y for its members [NM z, NM z + NM) (z = blockIdx.z; a workgroup past the
 // expert's member count ends at once), output rows [64t, 64t+64): o[slot][row].
-template <int I, int NM>
-__global__ __launch_bounds__(256, NM == 16 ? 2 : 1) void k_grp_down(int hidden, int nsb, GroupBufs gp) {
+template <int I, int NM, bool PASS>
+__global__ __launch_bounds__(256, NM == 16 ? 2 : 1) void k_grp_down(int hidden, GroupBufs g) {
   constexpr int NB = I / 32;
   constexpr int STR = I + 16;
   __shared__ __align__(16) int8_t bh[NM * STR];
@@ -330,28 +360,28 @@ __global__ __launch_bounds__(256, NM == 16 ? 2 : 1) void k_grp_down(int hidden, 
   __shared__ float dx[NM * NB];
   __shared__ __align__(16) uint16_t sdt[4][NB * 16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int tiles = hidden / 64, sb = blockIdx.x / tiles, tile = blockIdx.x % tiles;  // steps as in k_grp_up
-  GroupBufs g = gp;
-  g.grp += (size_t)sb * GRP_WORDS;
-  g.ah += (size_t)sb * kGrpMaxPos * 8 * I;
-  g.al += (size_t)sb * kGrpMaxPos * 8 * I;
-  g.ad += (size_t)sb * kGrpMaxPos * 8 * NB;
-  g.o += (size_t)sb * kGrpMaxPos * 8 * hidden;
-  int u = blockIdx.y;
-  const int nu = g.grp[GRP_NU];
-  if (nsb > 1) {  // the list index of expert blockIdx.y (the list holds up to 64)
-    const unsigned long long at = __ballot(lane < nu && g.grp[GRP_LIST + lane] == u);
-    u = at ? __ffsll((long long)at) - 1 : nu;
+  const int tile = blockIdx.x;
+  int e, ne, off = 0;
+  const int* entry = nullptr;
+  if constexpr (PASS) {  // members as in k_grp_up
+    int c0 = 0, members = 0;
+    e = member_tile<NM>(g.cnt, blockIdx.y, lane, &c0, &members);
+    if (e < 0) return;
+    ne = min(members - c0, NM);
+    entry = g.list + (size_t)e * g.cap + c0;
+  } else {
+    const int u = blockIdx.y, c0 = NM * blockIdx.z;
+    if (u >= g.grp[GRP_NU] || g.grp[GRP_CNT + u] <= c0) return;
+    e = g.grp[GRP_LIST + u];
+    ne = g.grp[GRP_CNT + u] - c0;
+    off = g.grp[GRP_OFF + u] + c0;
   }
-  if (u >= nu) return;
-  const int c0 = NM * blockIdx.z;
-  if (g.grp[GRP_CNT + u] <= c0) return;
-  const int e = g.grp[GRP_LIST + u], ne = g.grp[GRP_CNT + u] - c0, off = g.grp[GRP_OFF + u] + c0;
+  auto slot = [&](int c) { return PASS ? entry[c] >> 16 : off + c; };
   const size_t t16 = ((size_t)e * hidden + 64 * tile + 16 * wave) / 16;  // this wave's 16 output rows
   TileScales<NB> sc;
   fetch_scales<NB>(g.dn, t16, NB, 0, sc);
   Members<I, NM, 256> mb;
-  fetch_members<I, NM, 256, true>(g.ah, g.al, g.ad, 0u, off, ne, mb);
+  fetch_members<I, NM, 256>(g.ah, g.al, g.ad, slot, ne, mb);
   uint4 a[NB / 2];
   fetch_tile_q8<NB>(g.dn, t16, NB, 0, a);
   store_scales<NB>(sc, sdt[wave]);
@@ -365,7 +395,7 @@ __global__ __launch_bounds__(256, NM == 16 ? 2 : 1) void k_grp_down(int hidden, 
     const int c = 16 * ct + (lane & 15);
     if (c < ne) {
       const int r0 = 64 * tile + 16 * wave + 4 * grp;
-      *reinterpret_cast<float4*>(g.o + (size_t)(off + c) * hidden + r0) =
+      *reinterpret_cast<float4*>(g.o + (size_t)slot(c) * hidden + r0) =
           make_float4(acc[ct][0], acc[ct][1], acc[ct][2], acc[ct][3]);
     }
   }
@@ -464,33 +494,38 @@ hipError_t launch_grp_experts(hipStream_t s, int H, int E, int m, int k, int int
       g.gu.cols != H || g.gu.rows != E * 2 * inter || g.dn.cols != inter || g.dn.rows != E * H)
     return hipErrorInvalidValue;
   hipError_t e;
-  const int nsb = grp_steps(m);
-  const int U = nsb == 1 && m * k < E ? m * k : E;
-  const int CH = (std::min(m, kGrpMaxPos) + 15) / 16;  // member groups of 16: a step's expert has at most m members
+  constexpr int NT = kGrpUpThreads, RT = 16 * NT / 128;
+#define UP(PASS, GRID)                                                                       \
+  if (H == 1024) klaunch(k_grp_up<1024, 16, NT, PASS>, GRID, NT, 0, s, m, k, inter, g);      \
+  else klaunch(k_grp_up<1536, 16, NT, PASS>, GRID, NT, 0, s, m, k, inter, g)
+#define DOWN(PASS, GRID)                                                                     \
+  switch (inter) {                                                                           \
+    case 128: klaunch(k_grp_down<128, 16, PASS>, GRID, 256, 0, s, H, g); break;              \
+    case 256: klaunch(k_grp_down<256, 16, PASS>, GRID, 256, 0, s, H, g); break;              \
+    case 512: klaunch(k_grp_down<512, 16, PASS>, GRID, 256, 0, s, H, g); break;              \
+    default: return hipErrorInvalidValue;                                                    \
+  }
+  if (m > kGrpMaxPos) {
+    if (!g.cnt || !g.list || ev) return hipErrorInvalidValue;
+    klaunch(k_grp_plan, grp_steps(m), 256, 0, s, m, k, g);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    const int tiles = m * k / 16 + std::min(m * k, E);  // full tiles, and a partial one per expert
+    UP(true, dim3(inter / RT, tiles));
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    DOWN(true, dim3(H / 64, tiles));
+    return hipGetLastError();
+  }
+  const int U = m * k < E ? m * k : E;
+  const int CH = (m + 15) / 16;  // member groups of 16: a step's expert has at most m members
   // u is the slow grid index, so the workgroups of list indices past the step's expert count (which end at once)
   // are dispatched last
-  constexpr int NT = kGrpUpThreads, RT = 16 * NT / 128;
-  const dim3 gu_grid(inter / RT * nsb, U, CH);
   arm(1);
-  if (H == 1024) {
-    klaunch(k_grp_up<1024, 16, NT>, gu_grid, NT, 0, s, m, k, inter, nsb, g);
-  } else {
-    klaunch(k_grp_up<1536, 16, NT>, gu_grid, NT, 0, s, m, k, inter, nsb, g);
-  }
+  UP(false, dim3(inter / RT, U, CH));
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  const dim3 dn_grid(H / 64 * nsb, U, CH);
   arm(2);
-  switch (inter) {
-#define DOWN_CASE(II)                                                                               \
-  case II:                                                                                          \
-    klaunch(k_grp_down<II, 16>, dn_grid, 256, 0, s, H, nsb, g);                                      \
-    break;
-    DOWN_CASE(128)
-    DOWN_CASE(256)
-    DOWN_CASE(512)
-#undef DOWN_CASE
-    default: return hipErrorInvalidValue;
-  }
+  DOWN(false, dim3(H / 64, U, CH));
+#undef UP
+#undef DOWN
   return hipGetLastError();
 }
 

@@ -59,7 +59,7 @@ __global__ __launch_bounds__(kGdThreads) void k_gd_dense(TMat w, int m, const in
   TileScales<NBW> sc;
   fetch_scales<NBW>(w, t16, NB, kq * NBW, sc);
   Members<K, NM, kGdThreads> mb;
-  fetch_members<K, NM, kGdThreads, true>(xh, xl, xd, 0u, c0, m, mb);
+  fetch_members<K, NM, kGdThreads>(xh, xl, xd, [&](int c) { return c0 + c; }, m, mb);
   uint4 a[NBW / 2];
   fetch_tile_q8<NBW>(w, t16, NB, kq * NBW, a);
   store_scales<NBW>(sc, sdt[wave]);

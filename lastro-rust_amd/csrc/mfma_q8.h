@@ -123,8 +123,7 @@ __device__ __forceinline__ void fetch_tile_q8(const TMat& m, size_t t16, int NB,
   for (int q = 0; q < NBW / 2; q++) a[q] = p[q * 64];
 }
 
-// Member activations: rows row(c) for c in [0, ne) of the hi/lo planes (row length K) and their K/32 block scales;
-// row(c) = off + c (member slots, contiguous) or the c-th set bit of `bits` (member positions).
+// Member activations: rows row(c) for c in [0, ne) of the hi/lo planes (row length K) and their K/32 block scales.
 template <int K, int NM, int NT>
 struct Members {
   static constexpr int C16 = K / 16;
@@ -139,9 +138,9 @@ __device__ __forceinline__ int nth_set_bit(unsigned bits, int c) {
   return __ffs(bits) - 1;
 }
 
-template <int K, int NM, int NT, bool CONTIG>
+template <int K, int NM, int NT, class R>
 __device__ __forceinline__ void fetch_members(const int8_t* __restrict__ srch, const int8_t* __restrict__ srcl,
-                                              const float* __restrict__ srcd, unsigned bits, int off, int ne,
+                                              const float* __restrict__ srcd, const R& row, int ne,
                                               Members<K, NM, NT>& mb) {
   using M = Members<K, NM, NT>;
 #pragma unroll
@@ -150,7 +149,7 @@ __device__ __forceinline__ void fetch_members(const int8_t* __restrict__ srch, c
     mb.h[q] = make_uint4(0, 0, 0, 0);
     mb.l[q] = make_uint4(0, 0, 0, 0);
     if (i < NM * M::C16 && c < ne) {
-      const size_t r = CONTIG ? (size_t)(off + c) : (size_t)nth_set_bit(bits, c);
+      const size_t r = (size_t)row(c);
       mb.h[q] = reinterpret_cast<const uint4*>(srch + r * K)[j];
       mb.l[q] = reinterpret_cast<const uint4*>(srcl + r * K)[j];
     }
@@ -159,7 +158,7 @@ __device__ __forceinline__ void fetch_members(const int8_t* __restrict__ srch, c
   for (int q = 0; q < M::PERD; q++) {
     const int i = threadIdx.x + q * NT, c = i / (K / 32), b = i % (K / 32);
     mb.d[q] = 0.0f;
-    if (i < NM * (K / 32) && c < ne) mb.d[q] = srcd[(CONTIG ? (size_t)(off + c) : (size_t)nth_set_bit(bits, c)) * (K / 32) + b];
+    if (i < NM * (K / 32) && c < ne) mb.d[q] = srcd[(size_t)row(c) * (K / 32) + b];
   }
 }
 

@@ -370,25 +370,6 @@ __global__ __launch_bounds__(route_x_waves(DT) * 64) void k_route_x(DMat router,
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// The tile-th tile of NP members over the experts in order: expert and first member, or expert -1 past the last.
-// Every wave computes it from the 64 member counts.
-template <int NP>
-__device__ __forceinline__ int member_tile(const int* __restrict__ cnt, int tile, int lane, int* first, int* members) {
-  const int c = cnt[lane], t = (c + NP - 1) / NP;
-  int sum = t;
-#pragma unroll
-  for (int s = 1; s < 64; s <<= 1) {
-    const int o = __shfl_up(sum, s);
-    sum += lane >= s ? o : 0;
-  }
-  const unsigned long long hit = __ballot(tile >= sum - t && tile < sum);
-  if (!hit) return -1;
-  const int e = __ffsll((long long)hit) - 1;
-  *members = __builtin_amdgcn_readlane(c, e);
-  *first = (tile - __builtin_amdgcn_readlane(sum - t, e)) * NP;
-  return e;
-}
-
 // Gate/up rows (16 of each) of one expert for a tile of its members: act[slot][r] = silu(gate_r . xn) * (up_r . xn)
 // (k_route_up's expert arithmetic per position). A last tile of at most 16 members runs as one position tile.
 template <int DT, int K, int NT>
