@@ -35,8 +35,12 @@ namespace moert {
 // A workgroup holds MT x NT tiles of 16 rows x 16 positions. Its waves share the groups of four chains: wave w takes
 // the runs of SUB adjacent groups w, w + KW, ... (so that the chunks past the row's 64th, which only the first groups
 // have, spread over all waves), one tree node per run goes to LDS, and every thread adds the NN nodes of its outputs.
-// Bound: the matrix cores (127 TFLOP/s for this instruction on 256 CUs, 32 cycles for 1024 products) where the tiles
-// are full; a row's dequantisation, two vector instructions an element, serves NT tiles and hides behind them.
+// Bound: instruction issue. f32 MFMAs (32 cycles for 1024 products, 127 TFLOP/s on 256 CUs) do not overlap with vector
+// instructions, so that a row's dequantisation, two of them an element and row tile, counts in full and serves NT
+// position tiles. 512 positions of the 3B shape: gate/up 185 us under the trace, 75 TFLOP/s, 77% of its issue bound; down 105, q/k/v
+// 58, output projection 36. 32 positions: 31, 18.5, 10, 10 us, where one vector fma chain per lane with the activations
+// in LDS took 60, 47, 32, 28. Measured and not taken, all within 3%: activations laid out so that a B load takes 64
+// consecutive bytes per position, three waves to a SIMD without the register prefetch, K over two waves.
 typedef float xg_f16 __attribute__((ext_vector_type(16)));
 
 template <int DT, int K>
@@ -279,7 +283,8 @@ __global__ __launch_bounds__((XGeo<DT, K>::NT_), 2) void k_oproj_x(DMat m, const
 // ------------------------------------------------------------------------------------------------------------
 // Position v = blockIdx.x: the MoE norm and the router in moe_norm.h's order. A wave takes whole experts (the last
 // item is the sum of squares): lane l forms the 8-column chains of blocks l, l + 64, .. itself and adds them in that
-// order, so no partials pass through memory. Then ranks, ids and weights in top-k order (the decode router), xn for
+// order, so no partials pass through memory (8.8 us for 70 positions, 16.6 for 512, 3B shape; with the partials written
+// by the output projection's epilogue the router took 4.8 us for 32 and the epilogue 8). Then ranks, ids and weights in top-k order (the decode router), xn for
 // the experts, and slot v * k + rank into the member list of each expert chosen (the order of a list does not enter
 // any result: every member is a column of its own).
 // 16 waves, 8 for f32 rows (whose registers would not fit 16), as k_route_up
@@ -441,7 +446,9 @@ __global__ __launch_bounds__((XGeo<DT, K>::NT_), 2) void k_moe_down_x(DMat dn, c
 
 // ------------------------------------------------------------------------------------------------------------
 // Position blockIdx.x: h[r] = h[r] + res * y, y = sum over j = 0 .. k-1 in order of w[j] * o[j][r] (k_expert_down's
-// combine; k = 0: h stays), then with lnw the next layer's input xn = lnw * (h * rms scale) in the canonical order.
+// combine; k = 0: h stays), then with lnw the next layer's input xn = lnw * (h * rms scale) in the canonical order: one
+// pass over h where the q/k/v kernel normalised every position in every workgroup. Bound: latency (7 us for 70 positions,
+// 8.8 for 512: 27 MB of expert outputs at 3 TB/s).
 template <int K>
 __global__ __launch_bounds__(256) void k_moe_comb_x(const float* __restrict__ o, const float* __restrict__ wts, int k,
                                                     float res, float* __restrict__ h, const float* __restrict__ lnw,
