@@ -542,9 +542,15 @@ hipError_t launch_embed_b(hipStream_t s, const DMat& emb, const Dims& d, const P
   return hipGetLastError();
 }
 
-// One or two position tiles per workgroup of the dense products: two halve the reads and the dequantisation of a row,
-// one gives twice the workgroups, which wins while those of two would leave compute units without one.
-static bool two_tiles(int row_groups, int nv) { return (long)row_groups * cdiv(nv, 32) >= 256; }
+// One or two position tiles per workgroup of the dense products: two share a row's reads and dequantisation, one makes
+// twice the workgroups. With c workgroups on the fullest of 256 compute units one tile takes about 10.4 + 5.65 (c - 1)
+// us and two 14.4 + 9.6 (c - 1) (3B shape, q/k/v, one / two: 48 positions 10.6 / 14.4, 64 16.2 / 14.4, 128 22.2 / 24.0,
+// 192 28.2 / 24.3, 256 33.0 / 32.9, 512 61 / 53; output projection 64 10.0 / 14.0, 128 15.2 / 13.9, 256 21.4 / 22.6,
+// 512 38.6 / 32.8): two where 17 c2 < 10 c1, which takes the faster one at each of these.
+static bool two_tiles(int row_groups, int nv) {
+  const int c1 = cdiv((long)row_groups * cdiv(nv, 16), 256), c2 = cdiv((long)row_groups * cdiv(nv, 32), 256);
+  return 17 * c2 < 10 * c1;
+}
 
 static hipError_t comb_dispatch(hipStream_t s, const Dims& d, const PfBufs& p, int nv, int k, const float* lnw) {
 #define COMB(KK)                                                                                                 \
@@ -601,7 +607,8 @@ hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const
   MOERT_DISPATCH(L.router.dtype, L.router.cols, BODY)
 #undef BODY
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  // One position tile per workgroup while an expert has at most 16 members on average. The tiles of all experts are
+  // One position tile per workgroup while an expert has at most 16 members on average (3B shape, gate/up with one / two:
+  // 64 positions, 13 members, 38.0 / 43.0 us; 96, 19 members, 54.6 / 50.6; 512 189 / 166). The tiles of all experts are
   // at most the members' over a tile and one more per expert used; a workgroup past the last ends at once.
   const bool two = (long)nv * d.top_k > 16L * d.experts;
   const int slots = nv * d.top_k, tiles = slots / (two ? 32 : 16) + std::min(slots, d.experts);
