@@ -7,8 +7,8 @@ namespace moert {
 
 // One wave's share of a V tile moved into LDS through registers, by the G waves that serve the same tile: piece e
 // (e = wave, wave + G, ...) is rows 8e..8e+7, lane l carrying 16 bytes of row 8e + l/8, so each piece reads 1 KB of
-// consecutive cache rows. The LDS tile is row-major [64][64] f32, converted once for the G heads, with the rows at
-// and past the tile's valid length `nv` stored as +0. Plain loads (not LDS DMA) keep the wait for the tile separate
+// consecutive cache rows. The tile stays in fp16, with the rows at and past its valid length `nv` stored as +0, and is
+// converted at its use. Plain loads (not LDS DMA) keep the wait for the tile separate
 // from the waits for the kernel's other loads. A piece index past 7 (only for G = 3) loads piece 7 again and stores
 // it into rows 64..71 of the tile, which are padding and never read.
 template <int G>
@@ -26,28 +26,6 @@ struct VShare {
     if (N > 5) f = at(5);
     if (N > 6) g = at(6);
     if (N > 7) h = at(7);
-  }
-  template <int STRIDE>
-  __device__ __forceinline__ void store(float* dst, int lane, int wave, int nv) const {
-    auto put = [&](int i, const uint4& v) {
-      const int row = 8 * (wave + G * i) + (lane >> 3);
-      const bool z = row >= nv;
-      float4* o = reinterpret_cast<float4*>(dst + row * STRIDE + (lane & 7) * 8);
-      o[0] = z ? make_float4(0.0f, 0.0f, 0.0f, 0.0f)
-               : make_float4(h2f((uint16_t)(v.x & 0xffffu)), h2f((uint16_t)(v.x >> 16)), h2f((uint16_t)(v.y & 0xffffu)),
-                             h2f((uint16_t)(v.y >> 16)));
-      o[1] = z ? make_float4(0.0f, 0.0f, 0.0f, 0.0f)
-               : make_float4(h2f((uint16_t)(v.z & 0xffffu)), h2f((uint16_t)(v.z >> 16)), h2f((uint16_t)(v.w & 0xffffu)),
-                             h2f((uint16_t)(v.w >> 16)));
-    };
-    put(0, a);
-    if (N > 1) put(1, b);
-    if (N > 2) put(2, c);
-    if (N > 3) put(3, d);
-    if (N > 4) put(4, e);
-    if (N > 5) put(5, f);
-    if (N > 6) put(6, g);
-    if (N > 7) put(7, h);
   }
   // The tile kept in fp16, row-major with rows of RS halves, as loaded (rows at and past nv stored as +0).
   template <int RS>
