@@ -48,6 +48,7 @@ class HostIo {
 
   // dev[0, bytes) = src, in stream order; src is free on return
   hipError_t in(hipStream_t s, void* dev, const void* src, size_t bytes) {
+    if (!src && bytes) return hipErrorInvalidValue;
     if (!fits(bytes)) return hipMemcpyAsync(dev, src, bytes, hipMemcpyHostToDevice, s);
     uint8_t* p = buf_ + used_;
     std::memcpy(p, src, bytes);
@@ -56,6 +57,7 @@ class HostIo {
   }
   // dst[0, bytes) = dev, as it stands behind the work queued so far; there after finish()
   hipError_t out(hipStream_t s, void* dst, const void* dev, size_t bytes) {
+    if (!dst && bytes) return hipErrorInvalidValue;  // refused here: finish() would copy into it
     if (bytes % 4 || (reinterpret_cast<uintptr_t>(dev) & 3) || !fits(bytes))
       return hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s);
     segs_.src[n_] = dev;

@@ -1,0 +1,104 @@
+"""HostIo (csrc/hostio.h) on the CPU: the header compiled with g++ against a stand-in of the few runtime calls it makes
+(copies and the gather kernel run at once), so that the bookkeeping of a call's inputs and results is checked without a
+GPU: what is refused, what falls back to a plain copy, and what is left behind by a call that failed."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lastro-rust_amd", "csrc")
+
+RUNTIME = r"""
+#pragma once
+#include <cstdint>
+#include <cstdlib>
+#include <cstring>
+enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorLaunchFailure = 719 };
+typedef int* hipStream_t;
+enum { hipMemcpyHostToDevice, hipMemcpyDeviceToHost, hipHostMallocMapped };
+struct dim3 { unsigned x, y, z; dim3(unsigned a = 1, unsigned b = 1, unsigned c = 1) : x(a), y(b), z(c) {} };
+struct uint4 { unsigned x, y, z, w; };
+static dim3 blockIdx, threadIdx, gridDim;
+static int copies = 0, launches = 0;  // plain copies and gather launches so far
+#define __global__
+#define __launch_bounds__(n)
+static hipError_t hipHostMalloc(void** p, size_t n, int) { *p = aligned_alloc(64, (n + 63) / 64 * 64); return hipSuccess; }
+static hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
+static hipError_t hipHostGetDevicePointer(void** d, void* p, int) { *d = p; return hipSuccess; }
+static hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+static hipError_t hipGetLastError() { return hipSuccess; }
+static hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, hipStream_t) {
+  copies++;
+  if (n) memcpy(d, s, n);
+  return hipSuccess;
+}
+template <class K, class... A>
+static void hipLaunchKernelGGL(K k, dim3 g, int threads, int, hipStream_t, A... a) {
+  launches++;
+  gridDim = g;
+  for (blockIdx.y = 0; blockIdx.y < g.y; blockIdx.y++)
+    for (blockIdx.x = 0; blockIdx.x < g.x; blockIdx.x++)
+      for (threadIdx.x = 0; threadIdx.x < (unsigned)threads; threadIdx.x++) k(a...);
+}
+"""
+
+MAIN = r"""
+#include "hostio.h"
+#include <cstdio>
+#define NEED(c) do { if (!(c)) { std::printf("failed: %s (line %d)\n", #c, __LINE__); return 1; } } while (0)
+using namespace moert;
+int main(int, char** argv) {
+  const char* name = argv[1];
+  alignas(16) static uint32_t dev[24100];
+  for (unsigned i = 0; i < 24100; i++) dev[i] = i * 2654435761u;
+  HostIo io;
+  NEED(io.create(4096) == hipSuccess);
+  CASES
+  std::printf("no such case\n");
+  return 1;
+}
+"""
+
+CASES = {
+    # a null output or input of any size is refused, as the runtime's own copy refuses it; nothing is registered
+    "null": r"""
+      uint32_t got[4] = {};
+      NEED(io.out(0, nullptr, dev, 16) == hipErrorInvalidValue);
+      NEED(io.in(0, dev, nullptr, 16) == hipErrorInvalidValue);
+      NEED(io.out(0, got, dev + 1, 16) == hipSuccess);
+      NEED(io.out(0, nullptr, dev, 0) == hipSuccess && io.in(0, dev, nullptr, 0) == hipSuccess);
+      NEED(io.flush(0) == hipSuccess);
+      io.finish(true);
+      NEED(!memcmp(got, dev + 1, 16));""",
+    # every size and alignment of a source, more results than one launch gathers, and results past the buffer
+    "results": r"""
+      static uint32_t got[40][600];
+      for (int round = 0; round < 3; round++) {
+        memset(got, 0, sizeof got);
+        for (int i = 0; i < 40; i++) NEED(io.out(0, got[i], dev + 600 * i + i % 5, 4 * (i * 13 % 600)) == hipSuccess);
+        NEED(io.out(0, (char*)got[39] + 2300, (char*)dev + 2, 3) == hipSuccess);  // not whole words: a plain copy
+        NEED(io.flush(0) == hipSuccess);
+        io.finish(true);
+        for (int i = 0; i < 40; i++) NEED(!memcmp(got[i], dev + 600 * i + i % 5, 4 * (i * 13 % 600)));
+        NEED(!memcmp((char*)got[39] + 2300, (char*)dev + 2, 3));
+      }""",
+}
+
+
+@pytest.fixture(scope="session")
+def program(tmp_path_factory):
+    d = tmp_path_factory.mktemp("hostio")
+    (d / "hip").mkdir()
+    (d / "hip" / "hip_runtime.h").write_text(RUNTIME)
+    body = "".join(f'if (!strcmp(name, "{n}")) {{{c}\n      return 0;\n  }}\n' for n, c in CASES.items())
+    (d / "main.cpp").write_text(MAIN.replace("CASES", body))
+    exe = d / "hostio"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fsanitize=address,undefined", "-I", str(d), "-I", CSRC, "-o", str(exe),
+                    str(d / "main.cpp")], check=True)
+    return exe
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_host_io(program, name):
+    r = subprocess.run([str(program), name], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
