@@ -1469,6 +1469,12 @@ static void mx_publish(moert_model* m, moert_model::Clock::time_point now, bool 
   m->mx_last_pub = now;
 }
 
+// Timing mark i of the generate call (a failure must reach MTRY: the call's results may be registered with the model).
+static int mx_mark(moert_model* m, int i) {
+  CHECK_HIP(hipEventRecord(m->mx_t[i], m->stream));
+  return MOERT_OK;
+}
+
 // Between step launches: consumes a completed read-back, or queues the next one once the interval has passed.
 static int mx_poll(moert_model* m, const MxCall& c) {
   const auto now = moert_model::Clock::now();
@@ -1627,8 +1633,8 @@ static int generate(moert_model* m, const int* prompt, int n_prompt, int n_new, 
                                   (uint64_t)(n_prompt > 1 ? n_prompt : n_new), nullptr);
     (void)moert_metrics_set_context(m->mx, (uint64_t)pos0, (uint64_t)m->max_len);
     mx_publish(m, moert_model::Clock::now(), true);
-    CHECK_HIP(hipEventRecord(m->mx_t[0], m->stream));
-    if (n_prompt == 1) CHECK_HIP(hipEventRecord(m->mx_t[1], m->stream));
+    MTRY(m, mx_mark(m, 0));
+    if (n_prompt == 1) MTRY(m, mx_mark(m, 1));
   }
   std::vector<float> lg(gaps ? m->cfg.vocab : 0);
   int i0 = 0;  // tokens read in passes over several positions; the decode steps take it from there
@@ -1639,13 +1645,13 @@ static int generate(moert_model* m, const int* prompt, int n_prompt, int n_new, 
     m->batched_mode = mode;
     if (rc) return rc;
     st[0] = pos0 + i0;
-    if (mc) CHECK_HIP(hipEventRecord(m->mx_t[1], m->stream));
+    if (mc) MTRY(m, mx_mark(m, 1));
   }
   MTRY(m, model_copy_in(m, m->b.state, st, sizeof st));
   for (int i = i0; i < steps; i++) {
     MTRY(m, model_launch(m));
     if (mc) {
-      if (i == n_prompt - 2) CHECK_HIP(hipEventRecord(m->mx_t[1], m->stream));
+      if (i == n_prompt - 2) MTRY(m, mx_mark(m, 1));
       MTRY(m, mx_poll(m, *mc));
     }
     if (gaps && i >= n_prompt - 1) {
@@ -1667,7 +1673,7 @@ static int generate(moert_model* m, const int* prompt, int n_prompt, int n_new, 
   }
   // token i was chosen at position pos0 + n_prompt - 1 + i (the last one is never fed back)
   MTRY(m, model_copy_out(m, out_tokens, m->b.argmax_hist + pos0 + n_prompt - 1, (size_t)n_new * 4));
-  if (mc) CHECK_HIP(hipEventRecord(m->mx_t[2], m->stream));
+  if (mc) MTRY(m, mx_mark(m, 2));
   const auto w0 = moert_model::Clock::now();
   MTRY(m, model_sync(m));
   m->mx_wait_s += std::chrono::duration<double>(moert_model::Clock::now() - w0).count();

@@ -2,6 +2,7 @@
 (copies and the gather kernel run at once), so that the bookkeeping of a call's inputs and results is checked without a
 GPU: what is refused, what falls back to a plain copy, and what is left behind by a call that failed."""
 import os
+import re
 import subprocess
 
 import pytest
@@ -102,3 +103,22 @@ def program(tmp_path_factory):
 def test_host_io(program, name):
     r = subprocess.run([str(program), name], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_no_model_call_returns_between_registering_a_result_and_the_wait():
+    """A result registered with the model (model_copy_out) keeps the caller's pointer until model_sync has filled it or
+    a failure handled by MTRY has dropped it. A plain return in between would leave the pointer for a later call."""
+    src = open(os.path.join(CSRC, "engine.hip")).read()
+    src = re.sub(r"//[^\n]*", "", src)
+    seen = 0
+    for body in re.findall(r"^(?:static )?int \w+\([^;{]*\) \{\n(.*?)^\}", src, re.M | re.S):
+        open_at = None
+        for line in body.split("\n"):
+            if "model_copy_out(m" in line:
+                open_at, seen = line, seen + 1
+            if open_at:
+                assert not re.search(r"\b(CHECK_HIP|CHECK_CFG|TRY|return)\b", line.replace("MTRY", "")), (open_at, line)
+            if "model_sync(m)" in line:
+                open_at = None
+        assert open_at is None, open_at
+    assert seen > 10
