@@ -7,7 +7,6 @@
 #include <stdint.h>
 
 #include <cstring>
-#include <vector>
 
 namespace moert {
 
@@ -58,12 +57,12 @@ class HostIo {
   // dst[0, bytes) = dev, as it stands behind the work queued so far; there after finish()
   hipError_t out(hipStream_t s, void* dst, const void* dev, size_t bytes) {
     if (!dst && bytes) return hipErrorInvalidValue;  // refused here: finish() would copy into it
-    if (bytes % 4 || (reinterpret_cast<uintptr_t>(dev) & 3) || !fits(bytes))
+    if (bytes % 4 || (reinterpret_cast<uintptr_t>(dev) & 3) || !fits(bytes) || n_outs_ == kOuts)
       return hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s);
     segs_.src[n_] = dev;
     segs_.off[n_] = (unsigned)used_;
     segs_.words[n_] = (unsigned)(bytes / 4);
-    outs_.push_back({dst, used_, bytes});
+    outs_[n_outs_++] = Out{dst, used_, bytes};
     take(bytes);
     return ++n_ == HostSegs::kMax ? flush(s) : hipSuccess;
   }
@@ -80,8 +79,8 @@ class HostIo {
   // After the stream is idle: results to the caller's memory (dropped without `ok`), the buffer free again.
   void finish(bool ok) {
     if (ok)
-      for (const Out& o : outs_) std::memcpy(o.dst, buf_ + o.off, o.bytes);
-    outs_.clear();
+      for (int i = 0; i < n_outs_; i++) std::memcpy(outs_[i].dst, buf_ + outs_[i].off, outs_[i].bytes);
+    n_outs_ = 0;
     used_ = 0;
     n_ = 0;
   }
@@ -105,7 +104,9 @@ class HostIo {
   size_t cap_ = 0, used_ = 0;
   HostSegs segs_{};
   int n_ = 0;
-  std::vector<Out> outs_;
+  static constexpr int kOuts = 64;  // results of a call; a further one is a plain copy. Fixed: no call allocates
+  Out outs_[kOuts];
+  int n_outs_ = 0;
 };
 
 }  // namespace moert

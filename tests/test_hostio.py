@@ -46,6 +46,11 @@ static void hipLaunchKernelGGL(K k, dim3 g, int threads, int, hipStream_t, A... 
 MAIN = r"""
 #include "hostio.h"
 #include <cstdio>
+#include <new>
+static int news = 0;  // allocations so far
+void* operator new(size_t n) { news++; return malloc(n); }
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
 #define NEED(c) do { if (!(c)) { std::printf("failed: %s (line %d)\n", #c, __LINE__); return 1; } } while (0)
 using namespace moert;
 int main(int, char** argv) {
@@ -83,6 +88,27 @@ CASES = {
         for (int i = 0; i < 40; i++) NEED(!memcmp(got[i], dev + 600 * i + i % 5, 4 * (i * 13 % 600)));
         NEED(!memcmp((char*)got[39] + 2300, (char*)dev + 2, 3));
       }""",
+    # more results than the table holds: the rest are plain copies, and no call allocates (an allocation that fails
+    # would leave the C entry point as an exception)
+    "many": r"""
+      static uint32_t got[100][2];
+      HostIo big;
+      NEED(big.create(1 << 16) == hipSuccess);
+      news = 0;
+      for (int i = 0; i < 100; i++) NEED(big.out(0, got[i], dev + 2 * i, 8) == hipSuccess);
+      NEED(copies == 36 && big.flush(0) == hipSuccess);
+      big.finish(true);
+      NEED(news == 0 && !memcmp(got, dev, sizeof got));""",
+    # a call that failed between registering and the wait leaves nothing for the next one
+    "restart": r"""
+      uint32_t* gone = new uint32_t[4];
+      NEED(io.out(0, gone, dev, 16) == hipSuccess);
+      delete[] gone;
+      NEED(io.restart(0) == hipSuccess);
+      uint32_t got[4];
+      NEED(io.out(0, got, dev + 4, 16) == hipSuccess && io.flush(0) == hipSuccess);
+      io.finish(true);
+      NEED(!memcmp(got, dev + 4, 16));""",
 }
 
 
