@@ -201,7 +201,9 @@ int moert_step_batched(moert_model* m, const int* tokens, int n, float* logits, 
  * le_ids (rust/moe-rt/src/motor/leitura.rs:79-85, validation leitura.rs:62-76): the tokens are checked and the
  * cache bound (MOERT_E_FULL) before any block runs; logits / argmax of the last position. In mode 0 a block holds up
  * to 512 positions (every weight is read once per block) and the result does not depend on the blocks; in mode 1 the
- * blocks are those of plano_blocos (rust/moe-rt/src/motor/leitura.rs:53-60), up to 32 positions, several to a launch. */
+ * blocks are those of plano_blocos (rust/moe-rt/src/motor/leitura.rs:53-60), up to 32 positions, several to a launch.
+ * The buffers of a block are allocated by the first prompt that is long enough for it (here and in moert_generate) and
+ * kept; without device memory for them the blocks are smaller, down to single steps in mode 0. */
 int moert_prefill(moert_model* m, const int* tokens, int n, float* logits, int* argmax);
 
 /* Back to position 0 (old KV stays, masked by the length). Replaces GpuModel::reset
@@ -274,6 +276,10 @@ int moert_model_path(const moert_model* m, int* layer, int* attn_block, int* moe
  * the fused kernels. Bit 16 alone (the wait of the cache prefetch's copy workgroups for the layer's predicted misses)
  * applies to an expert-cache model whose prefetch runs inside the attention launch, and to no other. */
 int moert_fault_inject(moert_model* m, unsigned bits);
+/* Test hook for a device without memory for a prompt's passes: while it is set, buffers of passes of more than
+ * `positions` positions ask the device for 2^50 bytes, which it does not have (negative: no limit). Buffers that are
+ * there stay. No reference counterpart. */
+int moert_pass_limit_inject(moert_model* m, int positions);
 
 /* Phase timeline of one decode step (measurement build libmoert_tl.so only; MOERT_E_CONFIG otherwise): one graph
  * replay in which every workgroup of every launch stamps the 100 MHz real-time clock at its phase boundaries.

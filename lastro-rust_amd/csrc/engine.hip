@@ -10,6 +10,7 @@
 
 #include <atomic>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <memory>
 #include <cstdlib>
@@ -94,6 +95,14 @@ struct Arena {
     CHECK_HIP(hipMalloc(p, bytes));
     ptrs.push_back(*p);
     return MOERT_OK;
+  }
+  // As alloc, for memory that the caller can do without: running out leaves no error behind it.
+  hipError_t try_alloc(void** p, size_t bytes) {
+    *p = nullptr;
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) ptrs.push_back(*p);
+    else (void)hipGetLastError();
+    return e;
   }
   void release() {
     for (void* p : ptrs) (void)hipFree(p);
@@ -535,28 +544,48 @@ struct moert_model {
     return MOERT_OK;
   }
 
-  // Multi-position step buffers for at least n positions, allocated on first use. A longer prompt than any before
-  // replaces them (twice the positions at least, kPfBlock at most); they go with the model.
+  // Buffers of a pass over several positions, allocated on first use; a longer pass than any before replaces them (by a
+  // power of two of steps, kPfBlock positions at most) once the larger ones are there. They go with the model. `make`
+  // fills a set for M positions from an arena with try_alloc. Where memory is short the set stays smaller than asked
+  // for: `bufs.cap` positions, 0 if there is none.
+  template <class B, class F>
+  int grow_bufs(int n, B& bufs, Arena& mem, const F& make) {
+    int M = kPfMaxPos;
+    while (M < n) M *= 2;
+    for (; M >= kPfMaxPos && M > bufs.cap; M /= 2) {
+      B made{};
+      Arena a;
+      hipError_t e = make(M, made, a);
+      if (e == hipSuccess && (e = hipStreamSynchronize(stream)) == hipSuccess) {
+        mem.release();
+        mem.ptrs.swap(a.ptrs);
+        bufs = made;
+        bufs.cap = M;
+        return MOERT_OK;
+      }
+      a.release();
+      if (e != hipErrorOutOfMemory) CHECK_HIP(e);
+    }
+    return MOERT_OK;
+  }
+  int pass_limit = INT_MAX;  // moert_pass_limit_inject
+  size_t pass_bytes(int M, size_t bytes) const { return M > pass_limit ? (size_t)1 << 50 : bytes; }
+
+  // multi-position step buffers
   PfBufs pf{};
   Arena pf_arena;
   int ensure_pf(int n) {
-    if (pf.cap >= n) return MOERT_OK;
-    CHECK_HIP(hipStreamSynchronize(stream));
-    pf_arena.release();
-    pf = PfBufs{};
-    int M = kPfMaxPos;
-    while (M < n) M *= 2;
-    const int H = dims.hidden, qd = dims.heads * 64, I = dims.inter, K8 = 8;
-    const size_t parts = (size_t)M * dims.heads * attn_splits_for(max_len, dims.tps) * 66;
-    auto mem = [&](size_t words, auto** p) { return pf_arena.alloc((void**)p, words * 4); };  // written before it is read
-    int rc;
-    if ((rc = mem((size_t)M * qd, &pf.q)) || (rc = mem((size_t)M * qd, &pf.att)) || (rc = mem(parts, &pf.part)) ||
-        (rc = mem((size_t)M * H, &pf.xn)) || (rc = mem((size_t)M * K8, &pf.ids)) || (rc = mem((size_t)M * K8, &pf.w)) ||
-        (rc = mem(64, &pf.cnt)) || (rc = mem((size_t)64 * M, &pf.list)) || (rc = mem((size_t)M * K8 * I, &pf.act)) ||
-        (rc = mem((size_t)M * K8 * H, &pf.o)) || (rc = mem((size_t)M * H, &pf.h)))
-      return rc;
-    pf.cap = M;
-    return MOERT_OK;
+    return grow_bufs(n, pf, pf_arena, [&](int M, PfBufs& p, Arena& a) {
+      const int H = dims.hidden, qd = dims.heads * 64, I = dims.inter, K8 = 8;
+      const size_t parts = (size_t)M * dims.heads * attn_splits_for(max_len, dims.tps) * 66;
+      hipError_t e = hipSuccess;  // every buffer is written before it is read
+      auto mem = [&](size_t words, auto** q) { return (e = a.try_alloc((void**)q, pass_bytes(M, words * 4))) == hipSuccess; };
+      (void)(mem(parts, &p.part) && mem((size_t)M * qd, &p.q) && mem((size_t)M * qd, &p.att) &&
+             mem((size_t)M * H, &p.xn) && mem((size_t)M * K8, &p.ids) && mem((size_t)M * K8, &p.w) &&
+             mem(64, &p.cnt) && mem((size_t)64 * M, &p.list) && mem((size_t)M * K8 * I, &p.act) &&
+             mem((size_t)M * K8 * H, &p.o) && mem((size_t)M * H, &p.h));
+      return e;
+    });
   }
 
   // grouped mode of the multi-position step (moert_batched_mode): the grouped kernels' buffers and every layer's
@@ -568,24 +597,18 @@ struct moert_model {
   };
   std::vector<TiledLayer> tiled;
   Arena mg_arena;
-  int ensure_mg(int n) {  // buffers for at least n positions, replaced as those of ensure_pf
-    if (mg.cap >= n) return MOERT_OK;
-    CHECK_HIP(hipStreamSynchronize(stream));
-    mg_arena.release();
-    mg = GroupBufs{};
-    int M = kGrpMaxPos;
-    while (M < n) M *= 2;
-    const size_t H = dims.hidden, I = dims.inter, S = (size_t)M * 8;
-    const size_t X = std::max(dims.hidden, dims.heads * dims.head_dim);  // code rows: block inputs, attention outputs
-    auto mem = [&](size_t bytes, auto** p) { return mg_arena.alloc((void**)p, bytes); };  // written before it is read
-    int rc;
-    if ((rc = mem(M * X, &mg.xh)) || (rc = mem(M * X, &mg.xl)) || (rc = mem(M * (X / 32) * 4, &mg.xd)) ||
-        (rc = mem((size_t)M / kGrpMaxPos * GRP_WORDS * 4, &mg.grp)) || (rc = mem(S * I, &mg.ah)) ||
-        (rc = mem(S * I, &mg.al)) || (rc = mem(S * (I / 32) * 4, &mg.ad)) || (rc = mem(S * H * 4, &mg.o)) ||
-        (rc = mem(64 * 4, &mg.cnt)) || (rc = mem((size_t)64 * M * 4, &mg.list)))
-      return rc;
-    mg.cap = M;
-    return MOERT_OK;
+  int ensure_mg(int n) {
+    return grow_bufs(n, mg, mg_arena, [&](int M, GroupBufs& g, Arena& a) {
+      const size_t H = dims.hidden, I = dims.inter, S = (size_t)M * 8;
+      const size_t X = std::max(dims.hidden, dims.heads * dims.head_dim);  // code rows: block inputs, attention outputs
+      hipError_t e = hipSuccess;  // every buffer is written before it is read
+      auto mem = [&](size_t bytes, auto** q) { return (e = a.try_alloc((void**)q, pass_bytes(M, bytes))) == hipSuccess; };
+      (void)(mem(M * X, &g.xh) && mem(M * X, &g.xl) && mem(M * (X / 32) * 4, &g.xd) &&
+             mem((size_t)M / kGrpMaxPos * GRP_WORDS * 4, &g.grp) && mem(S * I, &g.ah) && mem(S * I, &g.al) &&
+             mem(S * (I / 32) * 4, &g.ad) && mem(S * H * 4, &g.o) && mem(64 * 4, &g.cnt) &&
+             mem((size_t)64 * M * 4, &g.list));
+      return e;
+    });
   }
   int ensure_grouped() {
     if (!tiled.empty()) return MOERT_OK;
@@ -1518,24 +1541,43 @@ int moert_decode_step(moert_model* m, int token, float* logits, int* route_ids, 
   return MOERT_OK;
 }
 
-// Positions pos0 .. pos0 + n - 1 (tokens in b.seq) in equal passes over the layers, of whole steps of kGrpMaxPos
-// positions (mode 1's results depend on its steps), the last one with the head.
-static int enqueue_blocks(moert_model* m, int pos0, int n, bool head) {
-  static_assert(kPfBlock % kGrpMaxPos == 0, "a pass is whole steps");
-  const int passes = (n + kPfBlock - 1) / kPfBlock, steps = grp_steps(n);
+// The buffers of a multi-position step's mode for n positions: the positions of a pass, 0 without memory for any.
+static int ensure_pass(moert_model* m, int mode, int n, int* cap) {
+  n = std::min(n, kPfBlock);
+  MTRY(m, m->ensure_pf(n));
+  if (mode == 1) MTRY(m, m->ensure_mg(n));
+  *cap = std::min(kPfBlock, mode == 1 ? std::min(m->pf.cap, m->mg.cap) : m->pf.cap);
+  return MOERT_OK;
+}
+
+// Positions pos0 .. pos0 + n - 1 (tokens in b.seq) in equal passes of at most cap positions over the layers, of whole
+// steps of kGrpMaxPos positions (mode 1's results depend on its steps), the last one with the head.
+static int enqueue_blocks(moert_model* m, int pos0, int n, int cap, bool head) {
+  static_assert(kPfBlock % kGrpMaxPos == 0 && kPfMaxPos % kGrpMaxPos == 0, "a pass is whole steps");
+  const int passes = (n + cap - 1) / cap, steps = grp_steps(n);
   const int per = (steps + passes - 1) / passes * kGrpMaxPos;
-  MTRY(m, m->ensure_pf(std::min(n, per)));
-  if (m->batched_mode == 1) MTRY(m, m->ensure_mg(std::min(n, per)));
   for (int i = 0; i < n; i += per) MTRY(m, m->enqueue_batched(pos0 + i, std::min(per, n - i), head && i + per >= n));
+  return MOERT_OK;
+}
+
+// The same positions as decode steps, bit for bit what mode 0's passes give: without memory for a pass.
+static int enqueue_steps(moert_model* m, int pos0, int n) {
+  MTRY(m, m->set_state(pos0, pos0 + n, nullptr, 0));
+  for (int i = 0; i < n; i++) MTRY(m, model_launch(m));
   return MOERT_OK;
 }
 
 // n checked tokens at the current position; logits and argmax of the last one. One wait, at the end.
 static int read_tokens(moert_model* m, const int* tokens, int n, float* logits, int* argmax) {
   const int pos0 = m->host_pos;
+  int rc, cap = 0;
+  if ((rc = ensure_pass(m, m->batched_mode, n, &cap))) return rc;
+  if (!cap && m->batched_mode == 1) {
+    set_err("multi-position step: no device memory for a step of %d positions", kGrpMaxPos);
+    return m->fail(MOERT_E_DEVICE);
+  }
   MTRY(m, model_copy_in(m, m->b.seq + pos0, tokens, (size_t)n * 4));
-  int rc = enqueue_blocks(m, pos0, n, true);
-  if (rc) return rc;
+  if ((rc = cap ? enqueue_blocks(m, pos0, n, cap, true) : enqueue_steps(m, pos0, n))) return rc;
   if (logits) MTRY(m, model_copy_out(m, logits, m->b.logits, (size_t)m->cfg.vocab * 4));
   int am = 0;
   MTRY(m, model_copy_out(m, &am, m->b.argmax_hist + pos0 + n - 1, 4));
@@ -1577,6 +1619,11 @@ int moert_batched_mode(moert_model* m, int mode) {
                     L.o.dtype == DT_Q8_0 && L.router.dtype == DT_Q8_0,
                 "grouped mode: Q8_0 weights only (q/k/v, output, router and experts)");
     MTRY(m, m->ensure_grouped());
+    MTRY(m, m->ensure_mg(kGrpMaxPos));
+    if (!m->mg.cap) {
+      set_err("grouped mode: no device memory for a step of %d positions", kGrpMaxPos);
+      return m->fail(MOERT_E_DEVICE);
+    }
   }
   m->batched_mode = mode;
   return MOERT_OK;
@@ -1637,11 +1684,15 @@ static int generate(moert_model* m, const int* prompt, int n_prompt, int n_new, 
     if (n_prompt == 1) MTRY(m, mx_mark(m, 1));
   }
   std::vector<float> lg(gaps ? m->cfg.vocab : 0);
-  int i0 = 0;  // tokens read in passes over several positions; the decode steps take it from there
+  int i0 = 0, cap = 0;  // i0: tokens read in passes over several positions; the decode steps take it from there
   if (!m->cached && n_prompt - 1 >= kPromptPass) {
+    const int rc = ensure_pass(m, 0, n_prompt - 1, &cap);
+    if (rc) return rc;
+  }
+  if (cap) {
     i0 = n_prompt - 1;
     const int mode = std::exchange(m->batched_mode, 0);  // the passes that equal decode steps
-    const int rc = enqueue_blocks(m, pos0, i0, false);
+    const int rc = enqueue_blocks(m, pos0, i0, cap, false);
     m->batched_mode = mode;
     if (rc) return rc;
     st[0] = pos0 + i0;
@@ -1964,6 +2015,12 @@ int moert_model_path(const moert_model* m, int* layer, int* attn_block, int* moe
   *layer = m->use_px ? 1 : 0;
   *attn_block = blk && !m->use_px ? 1 : 0;
   *moe_xcd = blk && m->use_mx && !m->use_px ? 1 : 0;
+  return MOERT_OK;
+}
+
+int moert_pass_limit_inject(moert_model* m, int positions) {
+  MODEL_OK(m);
+  m->pass_limit = positions < 0 ? INT_MAX : positions;
   return MOERT_OK;
 }
 

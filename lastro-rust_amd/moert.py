@@ -141,6 +141,7 @@ def lib() -> ctypes.CDLL:
             "moert_time_steps": (i, [vp, i, i, ctypes.POINTER(ctypes.c_double)]),
             "moert_time_kernel": (i, [vp, i, i, ctypes.POINTER(ctypes.c_double), ip]),
             "moert_fault_inject": (i, [vp, ctypes.c_uint]),
+            "moert_pass_limit_inject": (i, [vp, i]),
             "moert_model_path": (i, [vp, ip, ip, ip]),
             "moert_timeline_step": (i, [vp, vp, vp, vp, i, ip]),
             "moert_block_create": (i, [i, i, i, i, ctypes.POINTER(moert_tensor), vp, ctypes.POINTER(moert_tensor),
@@ -230,7 +231,7 @@ EXPORTED = ["moert_last_error", "moert_device_info", "moert_model_create", "moer
             "moert_decode_step", "moert_generate", "moert_step_batched", "moert_prefill", "moert_reset_sequence",
             "moert_kv_prefill_fp16",
             "moert_set_position", "moert_get_position", "moert_read_kv_fp16", "moert_read_hidden", "moert_read_logits",
-            "moert_time_steps", "moert_time_kernel", "moert_fault_inject", "moert_model_path", "moert_timeline_step", "moert_block_create", "moert_block_destroy",
+            "moert_time_steps", "moert_time_kernel", "moert_fault_inject", "moert_pass_limit_inject", "moert_model_path", "moert_timeline_step", "moert_block_create", "moert_block_destroy",
             "moert_block_forward", "moert_block_time", "moert_block_forward_batched",
             "moert_block_experts_in_step", "moert_block_batched_kernel", "moert_block_fault_inject", "moert_block_time_batched", "moert_router_topk", "moert_argmax", "moert_gemv",
             "moert_dequant", "moert_rmsnorm", "moert_rope", "moert_attn_decode", "moert_attn_decode_noalloc",
@@ -609,6 +610,10 @@ class GpuModel:
         16 alone: the cache prefetch's copy wait) give up in the following launches, which still end normally
         (moert_fault_inject)."""
         check(lib().moert_fault_inject(self.h, bits))
+
+    def pass_limit_inject(self, positions: int):
+        """Test hook: no device memory for passes of more than `positions` positions (negative: no limit)."""
+        check(lib().moert_pass_limit_inject(self.h, positions))
 
 
 # ---- checkpoints ------------------------------------------------------------------------------------------------
