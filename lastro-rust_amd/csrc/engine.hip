@@ -1414,7 +1414,7 @@ static int mx_enqueue_read(moert_model* m) {
 struct MxCall {
   int pos0, n_prompt, n_new;
   uint64_t started_ms;
-  moert_model::Clock::time_point t0;
+  moert_model::Clock::time_point t0, t_mark;  // t_mark: when timing mark 0 was queued on an idle stream
 };
 
 // Fills the publisher from a completed read-back: state, context, speed and the cache fractions over the window
@@ -1423,10 +1423,24 @@ static void mx_consume(moert_model* m, const MxCall& c, moert_model::Clock::time
   const unsigned long long* st = (const unsigned long long*)m->mx_pin;
   const int* state = (const int*)(m->mx_pin + 8 * CS_WORDS);
   const int s = state[ST_POS] - c.pos0;  // steps completed
-  const double dt = std::chrono::duration<double>(now - m->mx_prev_t).count();
-  const int ds = s - m->mx_prev_pos;
   moert_metrics* mx = m->mx;
   const bool reading = s < c.n_prompt - 1;
+  const double dt_cache = std::chrono::duration<double>(now - m->mx_prev_t).count();
+  if (!reading && m->mx_prev_pos < c.n_prompt - 1 && s > c.n_prompt - 1) {
+    // the window holds the end of the prompt, whose tokens take a tenth of a new one's time when they are read in
+    // passes: the speed is that of the new ones, from the prompt's last position on (timing mark 1, behind which the
+    // read-back was queued)
+    float ms = 0;
+    if (hipEventElapsedTime(&ms, m->mx_t[0], m->mx_t[1]) == hipSuccess) {
+      m->mx_prev_t = std::max(m->mx_prev_t, c.t_mark + std::chrono::duration_cast<moert_model::Clock::duration>(
+                                                           std::chrono::duration<double, std::milli>(ms)));
+      m->mx_prev_pos = c.n_prompt - 1;
+    } else {
+      (void)hipGetLastError();
+    }
+  }
+  const double dt = std::chrono::duration<double>(now - m->mx_prev_t).count();
+  const int ds = s - m->mx_prev_pos;
   if (reading)
     (void)moert_metrics_set_state(mx, MOERT_STATE_READING, (uint64_t)s, (uint64_t)c.n_prompt, nullptr);
   else
@@ -1435,8 +1449,9 @@ static void mx_consume(moert_model* m, const MxCall& c, moert_model::Clock::time
   (void)moert_metrics_set_context(mx, (uint64_t)state[ST_POS], (uint64_t)m->max_len);
   if (dt > 0 && ds > 0) {
     moert_metrics_speed sp{};
-    sp.decode_now = reading ? 0.0 : ds / dt;
-    sp.prefill_now = reading ? ds / dt : 0.0;
+    const bool prompt = s < c.n_prompt;  // no new token's step yet
+    sp.decode_now = prompt ? 0.0 : ds / dt;
+    sp.prefill_now = prompt ? ds / dt : 0.0;
     sp.decode_last = m->mx_speed_last[0];
     sp.prefill_request = m->mx_speed_last[1];
     (void)moert_metrics_set_speed(mx, &sp);
@@ -1456,7 +1471,7 @@ static void mx_consume(moert_model* m, const MxCall& c, moert_model::Clock::time
     ca.slots_resident = (uint32_t)m->place->resident();
     ca.hit_frac = need > 0 ? dh / need : 0.0;
     ca.cpu_frac = need > 0 ? du / need : 0.0;
-    ca.h2d_gbs = dt > 0 ? (double)dc * m->cache.record_bytes / dt / 1e9 : 0.0;
+    ca.h2d_gbs = dt_cache > 0 ? (double)dc * m->cache.record_bytes / dt_cache / 1e9 : 0.0;
     ca.total_hits = st[CS_HITS];
     ca.total_copies = st[CS_COPIES];
     ca.total_cpu = st[3];
@@ -1473,7 +1488,7 @@ static void mx_consume(moert_model* m, const MxCall& c, moert_model::Clock::time
     ca.slots_resident = res;
     ca.hit_frac = need > 0 ? dh / need : 0.0;
     ca.copy_frac = need > 0 ? dc / need : 0.0;
-    ca.h2d_gbs = dt > 0 ? (double)(dc + dp) * m->cache.record_bytes / dt / 1e9 : 0.0;
+    ca.h2d_gbs = dt_cache > 0 ? (double)(dc + dp) * m->cache.record_bytes / dt_cache / 1e9 : 0.0;
     ca.total_hits = st[CS_HITS];
     ca.total_copies = st[CS_COPIES] + st[CS_PREFETCH];
     memcpy(m->mx_prev, st, sizeof m->mx_prev);
@@ -1680,6 +1695,7 @@ static int generate(moert_model* m, const int* prompt, int n_prompt, int n_new, 
                                   (uint64_t)(n_prompt > 1 ? n_prompt : n_new), nullptr);
     (void)moert_metrics_set_context(m->mx, (uint64_t)pos0, (uint64_t)m->max_len);
     mx_publish(m, moert_model::Clock::now(), true);
+    mc->t_mark = moert_model::Clock::now();
     MTRY(m, mx_mark(m, 0));
     if (n_prompt == 1) MTRY(m, mx_mark(m, 1));
   }
@@ -1737,7 +1753,7 @@ int moert_generate(moert_model* m, const int* prompt, int n_prompt, int n_new, i
   if (!m->mx) return generate(m, prompt, n_prompt, n_new, out_tokens, gaps, nullptr);
   // with a metrics publisher: state and counters while the steps run, then the request entry (Request,
   // rust/moe-monitor/src/snapshot.rs:121-135), an event and a forced publication
-  MxCall mc{0, n_prompt, n_new, 0, moert_model::Clock::now()};
+  MxCall mc{0, n_prompt, n_new, 0, moert_model::Clock::now(), {}};
   mc.started_ms = (uint64_t)std::chrono::duration_cast<std::chrono::milliseconds>(
                       std::chrono::system_clock::now().time_since_epoch())
                       .count();
@@ -1822,7 +1838,7 @@ int moert_model_attach_metrics(moert_model* m, moert_metrics* mx, int min_interv
   MTRY(m, mx_enqueue_read(m));
   MTRY(m, model_sync(m));
   memcpy(m->mx_prev, m->mx_pin, sizeof m->mx_prev);
-  MxCall mc{m->host_pos, 1, 0, 0, moert_model::Clock::now()};
+  MxCall mc{m->host_pos, 1, 0, 0, moert_model::Clock::now(), {}};
   m->mx_prev_pos = 0;
   m->mx_prev_t = mc.t0;
   mx_consume(m, mc, mc.t0);
