@@ -1566,12 +1566,19 @@ static int ensure_pass(moert_model* m, int mode, int n, int* cap) {
 }
 
 // Positions pos0 .. pos0 + n - 1 (tokens in b.seq) in equal passes of at most cap positions over the layers, of whole
-// steps of kGrpMaxPos positions (mode 1's results depend on its steps), the last one with the head.
-static int enqueue_blocks(moert_model* m, int pos0, int n, int cap, bool head) {
+// steps of kGrpMaxPos positions (mode 1's results depend on its steps), the last one with the head. With `mc`, the
+// progress is polled between passes.
+static int enqueue_blocks(moert_model* m, int pos0, int n, int cap, bool head, const MxCall* mc = nullptr) {
   static_assert(kPfBlock % kGrpMaxPos == 0 && kPfMaxPos % kGrpMaxPos == 0, "a pass is whole steps");
   const int passes = (n + cap - 1) / cap, steps = grp_steps(n);
   const int per = (steps + passes - 1) / passes * kGrpMaxPos;
-  for (int i = 0; i < n; i += per) MTRY(m, m->enqueue_batched(pos0 + i, std::min(per, n - i), head && i + per >= n));
+  for (int i = 0; i < n; i += per) {
+    MTRY(m, m->enqueue_batched(pos0 + i, std::min(per, n - i), head && i + per >= n));
+    if (mc && i + per < n) {
+      MTRY(m, m->set_state(pos0 + i + per, pos0 + n, nullptr, 0));  // the position that a read-back finds
+      MTRY(m, mx_poll(m, *mc));
+    }
+  }
   return MOERT_OK;
 }
 
@@ -1708,13 +1715,14 @@ static int generate(moert_model* m, const int* prompt, int n_prompt, int n_new, 
   if (cap) {
     i0 = n_prompt - 1;
     const int mode = std::exchange(m->batched_mode, 0);  // the passes that equal decode steps
-    const int rc = enqueue_blocks(m, pos0, i0, cap, false);
+    const int rc = enqueue_blocks(m, pos0, i0, cap, false, mc);
     m->batched_mode = mode;
     if (rc) return rc;
     st[0] = pos0 + i0;
     if (mc) MTRY(m, mx_mark(m, 1));
   }
   MTRY(m, model_copy_in(m, m->b.state, st, sizeof st));
+  if (mc && i0) MTRY(m, mx_poll(m, *mc));
   for (int i = i0; i < steps; i++) {
     MTRY(m, model_launch(m));
     if (mc) {

@@ -1,5 +1,5 @@
-"""Metrics while moert_generate reads a long prompt in passes: the speed of the new tokens does not count the
-prompt's."""
+"""Metrics while moert_generate reads a long prompt in passes: the progress through the prompt is published, and the
+speed of the new tokens does not count the prompt's."""
 import threading
 import time
 
@@ -11,7 +11,7 @@ import moert
 pytestmark = pytest.mark.gpu
 
 
-def test_speeds_of_a_prompt_read_in_passes(gpu, tmp_path):
+def test_progress_and_speeds_of_a_prompt_read_in_passes(gpu, tmp_path):
     """1500 prompt tokens (three passes) and 300 new ones, every read-back published; a thread reads the file
     throughout. A read-back waits behind the steps queued before it, so each publication stands for milliseconds.
     Prompt tokens cost about a tenth of a new one's step: a window that counted them as new tokens would show a decode
@@ -51,5 +51,7 @@ def test_speeds_of_a_prompt_read_in_passes(gpu, tmp_path):
     g.close()
     mx.close()
     assert (request["prompt_tokens"], request["output_tokens"]) == (1500, 300)
+    reading = [s for s, _ in distinct if s["kind"] == "reading"]
+    assert any(0 < s["done"] < 1500 for s in reading), reading
     now = [sp["decode_now"] for s, sp in distinct if s["kind"] == "generating"]
     assert now and max(now) < 4 * request["decode_tok_s"], (now, request)
