@@ -583,7 +583,7 @@ struct moert_model {
       (void)(mem(parts, &p.part) && mem((size_t)M * qd, &p.q) && mem((size_t)M * qd, &p.att) &&
              mem((size_t)M * H, &p.xn) && mem((size_t)M * K8, &p.ids) && mem((size_t)M * K8, &p.w) &&
              mem(64, &p.cnt) && mem((size_t)64 * M, &p.list) && mem((size_t)M * K8 * I, &p.act) &&
-             mem((size_t)M * K8 * H, &p.o) && mem((size_t)M * H, &p.h));
+             mem((size_t)M * K8 * H, &p.o) && mem((size_t)M * H, &p.h) && mem((size_t)kFewPos * kNormItems, &p.zpart));
       return e;
     });
   }
@@ -640,9 +640,10 @@ struct moert_model {
   // argmax of the last one, its hidden state left in b.h, as after a decode step.
   int enqueue_batched(int pos0, int nv, bool head) {
     CHECK_HIP(launch_embed_b(stream, embed, dims, pf, b.seq + pos0, nv, b.state, pos0 + nv - 1));
+    const bool few = batched_mode == 0 && nv <= few_positions(layers[0].gate_up.dtype);
     if (batched_mode == 1)
       CHECK_HIP(launch_norm_codes(stream, dims.hidden, nv, pf.h, layers[0].ln_attn, dims.eps, mg));
-    else
+    else if (!few)
       CHECK_HIP(launch_norm_b(stream, dims, pf, nv, layers[0].ln_attn));
     for (size_t l = 0; l < layers.size(); l++) {
       const float* next = l + 1 < layers.size() ? layers[l + 1].ln_attn : nullptr;
@@ -653,6 +654,8 @@ struct moert_model {
         g.qkv = tiled[l].qkv;
         g.oproj = tiled[l].o;
         CHECK_HIP(launch_layer_grouped(stream, layers[l], dims, pf, b.state, pos0, nv, b.rope, g, next));
+      } else if (few) {
+        CHECK_HIP(launch_layer_few(stream, layers[l], dims, pf, b.state, pos0, nv, b.rope));
       } else {
         CHECK_HIP(launch_layer_b(stream, layers[l], dims, pf, b.state, pos0, nv, b.rope, next));
       }
@@ -1669,9 +1672,9 @@ int moert_prefill(moert_model* m, const int* tokens, int n, float* logits, int* 
 }
 
 // Prompt tokens before the last one from which moert_generate reads them in passes over several positions instead of
-// one decode step each (a resident model; the results are the same bit for bit). A whole prompt and two new tokens,
-// steps against a pass: 1B 2 tokens before the last 2.48 / 2.57 ms, 3 3.08 / 2.64, 19 12.9 / 2.9; 3B 2 3.79 / 4.07,
-// 3 4.72 / 4.12, 19 19.7 / 4.7.
+// one decode step each (a resident model; the results are the same bit for bit). A whole prompt and two new tokens, ms,
+// steps / a pass, Q8_0 on the fastest decode path (one launch per layer): 1B 2 tokens before the last 1.93 / 1.97,
+// 3 2.40 / 2.09, 19 10.0 / 2.66; 3B 2 3.00 / 3.10, 3 3.74 / 3.27, 19 15.6 / 4.33.
 constexpr int kPromptPass = 3;
 
 static int generate(moert_model* m, const int* prompt, int n_prompt, int n_new, int* out_tokens, float* gaps,

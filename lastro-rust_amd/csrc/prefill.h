@@ -14,6 +14,18 @@ constexpr int kPfMaxPos = 32;  // positions of one step call (the reference's bl
 // of the 3B shape, 4 layers: passes of 32 positions 7915 us, 128: 3015, 256: 2375, 512: 2000 (of which gate/up
 // 4 x 183); the buffers of a pass grow with it (512 positions: 0.2 GB at 64 splits).
 constexpr int kPfBlock = 512;
+// Positions of a pass that goes through few.hip instead (its buffers hold kFewPos). A tile of 16 positions on the matrix
+// cores costs the same for one as for 16; few.hip's time grows with the positions. A whole call, 16 layers, us, few.hip
+// / tiles, at 0 cached positions:
+//   Q8_0  1B  1: 664 / 859   4: 855 / 1017   8: 1065 / 1099   9: 1113 / 1103   16: 1422 / 1150
+//         3B  1: 724 / 1052  4: 1053 / 1255  8: 1362 / 1368   9: 1454 / 1379   16: 1943 / 1505
+//   Q4_0  1B  1: 660 / 812   4: 833 / 982    8: 1013 / 1055   9: 1063 / 1061
+//         3B  1: 708 / 1042  4: 985 / 1235   8: 1284 / 1333   9: 1375 / 1335
+//   f32   1B  1: 724 / 987   8: 1273 / 1463  14: 1575 / 1586  16: 1657 / 1593
+//         3B  1: 843 / 1247  8: 1666 / 1983  14: 2098 / 2231  16: 2239 / 2326
+// (f32 rows need no dequantisation, and the tiles read them in shorter steps; 4000 cached positions move no line.)
+constexpr int kFewPos = 14;
+constexpr int few_positions(int dtype) { return dtype == DT_F32 ? kFewPos : 8; }
 
 // Device buffers of one multi-position step, sized for `cap` positions.
 struct PfBufs {
@@ -28,7 +40,8 @@ struct PfBufs {
   int* list;     // [64, cap] their slots: position * k + top-k rank
   float* act;    // [m, k, I] SwiGLU activations
   float* o;      // [m, k, H] expert outputs
-  int* ids;      // [m, k] routed experts, top-k order (grouped mode)
+  int* ids;      // [m, k] routed experts, top-k order (grouped mode, few positions)
+  float* zpart;  // [kFewPos, kNormItems] MoE-norm partials of each position (few positions)
 };
 
 // Embedding rows of the nv tokens at `toks` (device) into h; the step state becomes position `last` and first free
@@ -42,6 +55,10 @@ hipError_t launch_norm_b(hipStream_t s, const Dims& d, const PfBufs& p, int nv, 
 // with next_lnw the layer leaves rmsnorm(h, next_lnw) there for the next one.
 hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* state, int pos0,
                           int nv, const float* rope, const float* next_lnw);
+// The same layer for at most kFewPos positions (few.hip), which normalises its input h itself: nothing is expected in xn
+// and nothing left there.
+hipError_t launch_layer_few(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* state, int pos0,
+                            int nv, const float* rope);
 // The same layer in grouped mode: q/k/v, output projection and experts through the int8 MFMA kernels of grouped.h,
 // g holding the layer's tiled matrices. On entry g's codes are those of rmsnorm(h, L.ln_attn) (launch_norm_codes or
 // the previous layer's combine); with next_lnw the layer leaves the codes of rmsnorm(h, next_lnw) for the next one.
