@@ -222,3 +222,35 @@ def test_expert_member_groups_cover_every_member_once(m, k, E):
                 done[(e, c0 + j)] = done.get((e, c0 + j), 0) + 1
     assert done == {(e, c): 1 for e in order for c in range(bin(bits[e]).count("1"))}
     assert max(bin(bits[e]).count("1") for e in order) == m  # expert 0: every position, so z reaches m - 1
+
+
+@pytest.mark.parametrize("m", [33, 48, 64, 300, 511, 512])
+@pytest.mark.parametrize("rows", [1024, 1536, 2048, 2560])
+def test_dense_workgroups_of_a_pass_cover_rows_and_positions_once(m, rows):
+    """A pass of more than 32 positions: blockIdx.x = tile + tiles * group, group g taking positions 32 g .. 32 g + 31
+    (fewer in the last); a member's code row and its output row are those of position 32 g + c."""
+    tiles, NM = rows // 32, 32
+    seen = np.zeros((tiles, m), int)
+    for bx in range(tiles * ((m + 31) // 32)):
+        tile, c0 = bx % tiles, bx // tiles * NM
+        n = min(m - c0, NM)
+        assert 1 <= n <= NM
+        seen[tile, c0:c0 + n] += 1
+    assert (seen == 1).all()
+
+
+@pytest.mark.parametrize("m", [33, 64, 300, 512])
+def test_steps_of_a_pass_have_their_own_plans_and_slots(m):
+    """Position p of a pass is position p % 32 of step p / 32 (k_gd_combine, k_grp_plan): its slots are those of the
+    step, 256 to a step, inside the buffers of ceil(m / 32) steps."""
+    k = 8
+    steps = -(-m // M)
+    cap = 32
+    while cap < m:
+        cap *= 2
+    for p in range(m):
+        sb, pl = divmod(p, M)
+        assert sb < steps <= cap // M  # the plans: cap / 32 of them
+        top = sb * M * 8 + min(m - sb * M, M) * k - 1  # last slot of the step
+        assert top < cap * 8                           # the slot buffers: cap * 8 rows
+        assert pl * k + k <= 256                       # k_grp_plan: a thread per (position, expert) of a step

@@ -1,20 +1,20 @@
-"""CPU transcription of the index arithmetic of the multi-position step's row kernels (lastro-rust_amd/csrc/
-prefill.hip): the xor-swizzled LDS layout of staged activations (xslot), the staging of a group of positions
+"""CPU transcription of the index arithmetic of the row kernels of a step of few positions (lastro-rust_amd/csrc/
+few.hip): the xor-swizzled LDS layout of staged activations (xslot), the staging of a group of positions
 (stage_group, and the member staging of k_moe_up_b / k_moe_down_b), the per-position norms (wave_rms, rsv), the RoPE
-table rows (csv), the output projection's row buffer (hn) and the bounds of a partial last group, for every block
-size 1..32 and every row length and dtype the kernels are built for. Every LDS and global index is checked against
+table rows (csv), the output projection's row buffer (hn) and the bounds of a partial last group, for every step
+of 1..14 positions and every row length and dtype the kernels are built for. Every LDS and global index is checked against
 the array it addresses, and the swizzle against being a permutation inside each weight chunk (so each staged
 element is written once and read back where the unswizzled layout has it)."""
 import numpy as np
 import pytest
 
-PF_WAVES, PF_NT, PF_GROUP, PF_MAX_POS = 8, 512, 8, 32
+PF_WAVES, PF_NT, PF_GROUP, PF_MAX_POS = 8, 512, 8, 14  # kFewWaves, kFewNT, kFewGroup, kFewPos
 CHUNK = {"f32": 4, "q8_0": 16, "q4_0": 32}  # elements per 16-byte payload chunk (Fmt<DT>::kElems)
 ROW_LENGTHS = [128, 256, 512, 1024, 1536, 2048]
 
 
 def xslot(dt, s):
-    """xslot<DT>(s) of prefill.hip (vectorised)."""
+    """xslot<DT>(s) of few.hip (vectorised)."""
     nq = CHUNK[dt] // 4
     s = np.asarray(s)
     if nq == 1:
@@ -38,7 +38,7 @@ def test_swizzle_is_a_permutation_inside_each_chunk(dt, K):
 
 
 def _threads(total):
-    """The (thread, index) pairs of `for (i = threadIdx.x; i < total; i += kPfNT)` over one workgroup."""
+    """The (thread, index) pairs of `for (i = threadIdx.x; i < total; i += kFewNT)` over one workgroup."""
     return np.arange(total)
 
 
@@ -114,7 +114,7 @@ def test_output_projection_row_buffer(dt, H):
 @pytest.mark.parametrize("k", [1, 2, 8])
 def test_expert_member_staging(k):
     """k_moe_up_b / k_moe_down_b: members of an expert are the set bits of a 32-bit mask over positions; staging
-    c0 .. c0 + n - 1 (up: groups of 8 into xs[8][K]; down: all ne into xs[32][K]) reads member c through
+    c0 .. c0 + n - 1 (up: groups of 8 into xs[8][K]; down: all ne into xs[14][K]) reads member c through
     nth_bit64(members, c), always a position < nv; act / o rows (vpos * k + rank) * len stay below nv * k * len."""
     rng = np.random.default_rng(7)
 
@@ -137,3 +137,15 @@ def test_expert_member_staging(k):
                         assert (vpos * k + rank) < nv * k
             assert all(0 <= nth_bit(members, c) < nv for c in range(ne))
             assert nth_bit(members, ne) == -1
+
+
+def test_the_transcribed_constants_are_the_kernels():
+    import os
+    import re
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lastro-rust_amd", "csrc")
+    few, head = (open(os.path.join(csrc, f)).read() for f in ("few.hip", "prefill.h"))
+    assert int(re.search(r"kFewWaves = (\d+)", few)[1]) == PF_WAVES
+    assert int(re.search(r"kFewGroup = (\d+)", few)[1]) == PF_GROUP
+    assert int(re.search(r"kFewPos = (\d+)", head)[1]) == PF_MAX_POS
+    for name in ("xslot", "stage_group", "wave_rms", "load_xs", "nth_bit64", "k_moe_up_b", "k_moe_down_b"):
+        assert re.search(rf"\b{name}\b", few), name
