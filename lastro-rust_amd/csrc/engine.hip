@@ -657,7 +657,7 @@ struct moert_model {
       } else if (few) {
         CHECK_HIP(launch_layer_few(stream, layers[l], dims, pf, b.state, pos0, nv, b.rope));
       } else {
-        CHECK_HIP(launch_layer_b(stream, layers[l], dims, pf, b.state, pos0, nv, b.rope, next));
+        CHECK_HIP(launch_layer_b(stream, layers[l], dims, pf, b.state, pos0, nv, b.rope, next, cus));
       }
     }
     if (!head) return MOERT_OK;
@@ -2252,7 +2252,7 @@ int moert_block_create(int hidden, int inter, int experts, int top_k, const moer
     return bail(MOERT_E_DEVICE);
   }
   b->dims = Dims{hidden, inter, 1, 1, 64, hidden, experts, top_k, 64, 1, 0.0f, 1.0f, 1.0f, 1.0f, 1.0f};
-  // inputs and outputs of a step of kGrpMaxPos positions, routing and error word
+  // inputs, outputs and routing of a step of kGrpMaxPos positions (the one-launch step's error word is read apart)
   if (b->io.create((size_t)kGrpMaxPos * (2 * hidden + 2 * 8) * 4 + 4096) != hipSuccess) {
     set_err("pinned buffer for the results");
     return bail(MOERT_E_DEVICE);

@@ -1149,8 +1149,10 @@ hipError_t launch_attn_combine(hipStream_t s, const Dims& d, const StepBufs& b, 
 
 hipError_t launch_attn_unit(hipStream_t s, const float* q, const uint16_t* kc, const uint16_t* vc, int heads,
                             int kv_heads, int max_len, int len, float scale, int tps, float* part, float* out) {
-  // A length of at most 4 tiles in one launch, a workgroup per KV head: the second launch costs more than the tiles
-  // (100 positions, 16 heads, a call among others: 13.9 us as length, splits and combine, 7.2 as one).
+  // A length of at most 4 tiles in one launch, a workgroup per KV head (4 heads x 4 tiles are its 16 waves): the second
+  // launch costs more than the tiles. A call among others, us, one launch / splits and combine, any tiles per split:
+  // 16 heads over 8 1 tile 4.3 / 7.1, 3 4.5 / 7.1, 4 4.9-5.2 / 7.2; 24 over 8 4 tiles 5.4-5.6 / 7.2; 64 over 16 4.3 / 7.1,
+  // 4 tiles 5.6-5.9 / 7.1-7.9.
   const int G = heads / kv_heads, nb = (len + 63) / 64;
   if (max_len % 64) return hipErrorInvalidValue;
 #define ALL_CASE(GG, TT)                                                                                         \

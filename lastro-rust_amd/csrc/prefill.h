@@ -12,7 +12,8 @@ constexpr int kPfMaxPos = 32;  // positions of one step call (the reference's bl
 // Positions per pass over the layers of a longer prompt. A pass reads every weight once, and its row products work on
 // tiles of 16 or 32 positions per expert: more positions fill more of a tile and hide more of the reads. 512 tokens
 // of the 3B shape, 4 layers: passes of 32 positions 7915 us, 128: 3015, 256: 2375, 512: 2000 (of which gate/up
-// 4 x 183); the buffers of a pass grow with it (512 positions: 0.2 GB at 64 splits).
+// 4 x 184); the buffers of a pass grow with it (512 positions: 0.25 GB at 64 splits). Passes of 1024 were measured
+// too: 1024 tokens 3182 us against 3507 in two of 512, 4096 tokens 14.4 ms against 15.7, with twice the buffers.
 constexpr int kPfBlock = 512;
 // Positions of a pass that goes through few.hip instead (its buffers hold kFewPos). A tile of 16 positions on the matrix
 // cores costs the same for one as for 16; few.hip's time grows with the positions. A whole call, 16 layers, us, few.hip
@@ -52,9 +53,9 @@ hipError_t launch_embed_b(hipStream_t s, const DMat& emb, const Dims& d, const P
 hipError_t launch_norm_b(hipStream_t s, const Dims& d, const PfBufs& p, int nv, const float* lnw);
 // One layer for positions pos0 .. pos0 + nv - 1 (state[ST_POS] == pos0 + nv - 1 on the device), rope: the [max_len, 64] table; the
 // decode kernels' chains, so that the results equal nv decode steps bit for bit. On entry xn = rmsnorm(h, L.ln_attn);
-// with next_lnw the layer leaves rmsnorm(h, next_lnw) there for the next one.
+// with next_lnw the layer leaves rmsnorm(h, next_lnw) there for the next one. cus: the device's compute units.
 hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* state, int pos0,
-                          int nv, const float* rope, const float* next_lnw);
+                          int nv, const float* rope, const float* next_lnw, int cus);
 // The same layer for at most kFewPos positions (few.hip), which normalises its input h itself: nothing is expected in xn
 // and nothing left there.
 hipError_t launch_layer_few(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* state, int pos0,

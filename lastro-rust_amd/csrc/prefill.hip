@@ -37,8 +37,8 @@ namespace moert {
 // have, spread over all waves), one tree node per run goes to LDS, and every thread adds the NN nodes of its outputs.
 // Bound: instruction issue. f32 MFMAs (32 cycles for 1024 products, 127 TFLOP/s on 256 CUs) do not overlap with vector
 // instructions, so that a row's dequantisation, two of them an element and row tile, counts in full and serves NT
-// position tiles. 512 positions of the 3B shape: gate/up 185 us under the trace, 75 TFLOP/s, 77% of its issue bound; down 105, q/k/v
-// 58, output projection 36. 32 positions: 31, 18.5, 10, 10 us, where one vector fma chain per lane with the activations
+// position tiles. 512 positions of the 3B shape: gate/up 184 us under the trace, 75 TFLOP/s, 77% of its issue bound; down 105, q/k/v
+// 60, output projection 37. 32 positions: 31, 18.5, 10, 10 us, where one vector fma chain per lane with the activations
 // in LDS took 60, 47, 32, 28. Measured and not taken, all within 3%: activations laid out so that a B load takes 64
 // consecutive bytes per position, three waves to a SIMD without the register prefetch, K over two waves.
 typedef float xg_f16 __attribute__((ext_vector_type(16)));
@@ -543,12 +543,15 @@ hipError_t launch_embed_b(hipStream_t s, const DMat& emb, const Dims& d, const P
 }
 
 // One or two position tiles per workgroup of the dense products: two share a row's reads and dequantisation, one makes
-// twice the workgroups. With c workgroups on the fullest of 256 compute units one tile takes about 10.4 + 5.65 (c - 1)
-// us and two 14.4 + 9.6 (c - 1) (3B shape, q/k/v, one / two: 48 positions 10.6 / 14.4, 64 16.2 / 14.4, 128 22.2 / 24.0,
-// 192 28.2 / 24.3, 256 33.0 / 32.9, 512 61 / 53; output projection 64 10.0 / 14.0, 128 15.2 / 13.9, 256 21.4 / 22.6,
-// 512 38.6 / 32.8): two where 17 c2 < 10 c1, which takes the faster one at each of these.
-static bool two_tiles(int row_groups, int nv) {
-  const int c1 = cdiv((long)row_groups * cdiv(nv, 16), 256), c2 = cdiv((long)row_groups * cdiv(nv, 32), 256);
+// twice the workgroups. With c workgroups on the fullest of the device's `cus` compute units one tile takes about 10.4 +
+// 5.65 (c - 1) us and two 14.4 + 9.6 (c - 1) (rows of 1536): two where 17 c2 < 10 c1. One / two, Q8_0, 256 compute units:
+//   3B q/k/v  48 10.5 / 14.2   64 15.8 / 14.2  128 21.5 / 23.2  192 27.4 / 23.9  256 33.2 / 32.6  512 60.6 / 52.1
+//      output 64 9.8 / 13.0   128 15.3 / 12.9  256 21.2 / 22.1  512 38.4 / 32.6
+//   1B q/k/v  64 7.8 / 10.9   128 11.1 / 10.6  192 15.5 / 17.4  256 19.6 / 18.0  384 27.4 / 25.9  512 35.0 / 31.7
+//      output 128 7.4 / 9.7   192 11.0 / 9.9   256 11.1 / 10.0  384 15.2 / 17.0  512 19.2 / 17.1
+// It takes the faster one at each of these but 3B q/k/v at 256, where the two are 2% apart.
+static bool two_tiles(int row_groups, int nv, int cus) {
+  const int c1 = cdiv((long)row_groups * cdiv(nv, 16), cus), c2 = cdiv((long)row_groups * cdiv(nv, 32), cus);
   return 17 * c2 < 10 * c1;
 }
 
@@ -568,15 +571,15 @@ hipError_t launch_norm_b(hipStream_t s, const Dims& d, const PfBufs& p, int nv, 
 }
 
 hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const PfBufs& p, const int* state, int pos0,
-                          int nv, const float* rope, const float* next_lnw) {
-  if (nv < 1 || nv > p.cap || d.top_k > 8 || d.experts > 64 || d.head_dim != 64) return hipErrorInvalidValue;
+                          int nv, const float* rope, const float* next_lnw, int cus) {
+  if (nv < 1 || nv > p.cap || cus < 1 || d.top_k > 8 || d.experts > 64 || d.head_dim != 64) return hipErrorInvalidValue;
   if (L.qkv.rows != (d.heads + 2 * d.kv_heads) * 64 || d.hidden % 32 || d.inter % 16) return hipErrorInvalidValue;
 #define QKV(KK, NN)                                                                                                 \
   klaunch(k_qkv_x<DTC, KK, NN>, dim3(L.qkv.rows / 32, cdiv(nv, 16 * NN)), XGeo<DTC, KK>::NT_, 0, s, L.qkv, p.xn, pos0, \
           nv, rope, d.heads, d.kv_heads, d.max_len, p.q, L.k_cache, L.v_cache, p.cnt)
 #define BODY(KK)                                        \
   case KK: {                                            \
-    if (two_tiles(L.qkv.rows / 32, nv)) QKV(KK, 2);     \
+    if (two_tiles(L.qkv.rows / 32, nv, cus)) QKV(KK, 2);     \
     else QKV(KK, 1);                                    \
   } break;
   MOERT_DISPATCH(L.qkv.dtype, L.qkv.cols, BODY)
@@ -591,7 +594,7 @@ hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const
           d.res_mult, p.h)
 #define BODY(KK)                                        \
   case KK: {                                            \
-    if (two_tiles(L.o.rows / 32, nv)) OPROJ(KK, 2);     \
+    if (two_tiles(L.o.rows / 32, nv, cus)) OPROJ(KK, 2);     \
     else OPROJ(KK, 1);                                  \
   } break;
   MOERT_DISPATCH(L.o.dtype, L.o.cols, BODY)
@@ -607,8 +610,9 @@ hipError_t launch_layer_b(hipStream_t s, const LayerDev& L, const Dims& d, const
   MOERT_DISPATCH(L.router.dtype, L.router.cols, BODY)
 #undef BODY
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  // One position tile per workgroup while an expert has at most 16 members on average (3B shape, gate/up with one / two:
-  // 64 positions, 13 members, 38.0 / 43.0 us; 96, 19 members, 54.6 / 50.6; 512 189 / 166). The tiles of all experts are
+  // One position tile per workgroup while an expert has at most 16 members on average (gate/up with one / two, uniform
+  // tokens: 3B 64 positions, 13 members, 39.0 / 42.6 us; 96, 19 members, 51.9 / 50.6; 512 187 / 163. 1B 64, 16 members,
+  // 27.8 / 29.6; 96 34.8 / 32.7; 128 40.9 / 41.5; 512 126 / 115). The tiles of all experts are
   // at most the members' over a tile and one more per expert used; a workgroup past the last ends at once.
   const bool two = (long)nv * d.top_k > 16L * d.experts;
   const int slots = nv * d.top_k, tiles = slots / (two ? 32 : 16) + std::min(slots, d.experts);

@@ -246,3 +246,24 @@ def test_the_transcribed_names_are_the_kernels():
                  "const int j = 4 * ((st.r * X::KW + w) * X::SUB + st.u) + gq + G::LPR * st.jj;"):
         assert text in SOURCE, text
     assert not re.search(r"xslot|stage_group", SOURCE)  # those are few.hip's
+
+
+def test_one_or_two_position_tiles():
+    """two_tiles: by the workgroups on the fullest of the device's compute units (not a fixed number of them). At the
+    measured points of 256 units (us, one / two tiles) it is never more than 3% from the faster one."""
+    body = re.search(r"static bool two_tiles\(int row_groups, int nv, int cus\) \{(.*?)\n\}", SOURCE, re.S)[1]
+    assert "256" not in body and body.count(", cus)") == 2 and "return 17 * c2 < 10 * c1;" in body
+
+    def two(groups, nv, cus=256):
+        c1, c2 = (-(-groups * -(-nv // n) // cus) for n in (16, 32))
+        return 17 * c2 < 10 * c1
+
+    times = {(80, 48): (10.5, 14.2), (80, 64): (15.8, 14.2), (80, 128): (21.5, 23.2), (80, 192): (27.4, 23.9),
+             (80, 256): (33.2, 32.6), (80, 512): (60.6, 52.1), (48, 64): (9.8, 13.0), (48, 128): (15.3, 12.9),
+             (48, 256): (21.2, 22.1), (48, 512): (38.4, 32.6), (64, 64): (7.8, 10.9), (64, 128): (11.1, 10.6),
+             (64, 192): (15.5, 17.4), (64, 256): (19.6, 18.0), (64, 384): (27.4, 25.9), (64, 512): (35.0, 31.7),
+             (32, 128): (7.4, 9.7), (32, 192): (11.0, 9.9), (32, 256): (11.1, 10.0), (32, 384): (15.2, 17.0),
+             (32, 512): (19.2, 17.1)}
+    for (groups, nv), (one, both) in times.items():
+        assert (both if two(groups, nv) else one) <= 1.03 * min(one, both), (groups, nv)
+    assert two(80, 32, 32) and not two(80, 32, 256)  # an eighth of the device: its own count decides
