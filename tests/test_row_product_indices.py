@@ -266,4 +266,4 @@ def test_one_or_two_position_tiles():
              (32, 512): (19.2, 17.1)}
     for (groups, nv), (one, both) in times.items():
         assert (both if two(groups, nv) else one) <= 1.03 * min(one, both), (groups, nv)
-    assert two(80, 32, 32) and not two(80, 32, 256)  # an eighth of the device: its own count decides
+    assert two(48, 64, 32) and not two(48, 64, 256)  # an eighth of the device: its own count decides
