@@ -15,8 +15,8 @@
 //                  act[v][j] (j = the expert's top-k rank at position v)
 //   k_moe_down_b   per routed expert: its down rows once for its positions, o[v][j] = down . act[v][j]
 //   k_moe_comb_b   h[v] += res * sum over j in top-k order of w[v][j] * o[v][j]
-// Bound: latency, and the reads of the routed experts. 2 positions of the 3B shape, Q8_0, this / the tiles of 16 (us):
-// q/k/v 6.6 / 9.2, output projection 5.5 / 9.4, router 3.9 / 8.4, gate/up 12.5 / 14.8, down 9.1 / 8.8, combine 3.8 /
+// Bound: latency, and the reads of the routed experts. 4 positions of the 3B shape, Q8_0, this / the tiles of 16 (us):
+// q/k/v 8.1 / 9.3, output projection 7.1 / 9.2, router 4.1 / 7.7, gate/up 17.6 / 19.1, down 11.3 / 10.6, combine 4.1 /
 // 6.9.
 #include <algorithm>
 

@@ -12,7 +12,7 @@ constexpr int kPfMaxPos = 32;  // positions of one step call (the reference's bl
 // Positions per pass over the layers of a longer prompt. A pass reads every weight once, and its row products work on
 // tiles of 16 or 32 positions per expert: more positions fill more of a tile and hide more of the reads. 512 tokens
 // of the 3B shape, 4 layers: passes of 32 positions 7915 us, 128: 3015, 256: 2375, 512: 2000 (of which gate/up
-// 4 x 184); the buffers of a pass grow with it (512 positions: 0.25 GB at 64 splits). Passes of 1024 were measured
+// 4 x 183); the buffers of a pass grow with it (512 positions: 0.25 GB at 64 splits). Passes of 1024 were measured
 // too: 1024 tokens 3182 us against 3507 in two of 512, 4096 tokens 14.4 ms against 15.7, with twice the buffers.
 constexpr int kPfBlock = 512;
 // Positions of a pass that goes through few.hip instead (its buffers hold kFewPos). A tile of 16 positions on the matrix

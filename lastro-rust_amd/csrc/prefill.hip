@@ -5,6 +5,8 @@
 // fmaf chain, then the pairwise lane tree), so the step equals single-position decode steps bit for bit: the KV rows
 // it appends, every hidden state and the last position's logits.
 //
+// A step of few positions runs the kernels of few.hip instead.
+//
 // Kernels per layer (one stream, in order; xn holds the normalised input of the layer on entry):
 //   k_qkv_x        [q; k; v] of every position, RoPE, q to qb[v], k and v to row pos0 + v of the KV cache
 //   attention      attn_mm.hip over the positions, position v attending to pos0 + v + 1, and the decode combine
@@ -37,8 +39,8 @@ namespace moert {
 // have, spread over all waves), one tree node per run goes to LDS, and every thread adds the NN nodes of its outputs.
 // Bound: instruction issue. f32 MFMAs (32 cycles for 1024 products, 127 TFLOP/s on 256 CUs) do not overlap with vector
 // instructions, so that a row's dequantisation, two of them an element and row tile, counts in full and serves NT
-// position tiles. 512 positions of the 3B shape: gate/up 184 us under the trace, 75 TFLOP/s, 77% of its issue bound; down 105, q/k/v
-// 60, output projection 37. 32 positions: 31, 18.5, 10, 10 us, where one vector fma chain per lane with the activations
+// position tiles. 512 positions of the 3B shape: gate/up 183 us under the trace, 75 TFLOP/s, 77% of its issue bound; down 104, q/k/v
+// 59, output projection 37. 32 positions: 31, 18.5, 10, 10 us, where one vector fma chain per lane with the activations
 // in LDS took 60, 47, 32, 28. Measured and not taken, all within 3%: activations laid out so that a B load takes 64
 // consecutive bytes per position, three waves to a SIMD without the register prefetch, K over two waves.
 typedef float xg_f16 __attribute__((ext_vector_type(16)));
