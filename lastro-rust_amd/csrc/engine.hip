@@ -1435,8 +1435,8 @@ static void mx_consume(moert_model* m, const MxCall& c, moert_model::Clock::time
     // read-back was queued)
     float ms = 0;
     if (hipEventElapsedTime(&ms, m->mx_t[0], m->mx_t[1]) == hipSuccess) {
-      m->mx_prev_t = std::max(m->mx_prev_t, c.t_mark + std::chrono::duration_cast<moert_model::Clock::duration>(
-                                                           std::chrono::duration<double, std::milli>(ms)));
+      m->mx_prev_t = c.t_mark + std::chrono::duration_cast<moert_model::Clock::duration>(
+                                    std::chrono::duration<double, std::milli>(ms));
       m->mx_prev_pos = c.n_prompt - 1;
     } else {
       (void)hipGetLastError();

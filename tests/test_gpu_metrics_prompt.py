@@ -11,18 +11,19 @@ import moert
 pytestmark = pytest.mark.gpu
 
 
-def test_progress_and_speeds_of_a_prompt_read_in_passes(gpu, tmp_path):
-    """1500 prompt tokens (three passes) and 300 new ones, every read-back published; a thread reads the file
-    throughout. A read-back waits behind the steps queued before it, so each publication stands for milliseconds.
-    Prompt tokens cost about a tenth of a new one's step: a window that counted them as new tokens would show a decode
-    speed far above the request's."""
-    cfg = moert.Config(**{**moert.GRANITE_1B, "layers": 8, "vocab": 211})
-    m = moert.SynthModel(cfg, seed=3, std=0.05)
-    g = moert.GpuModel(m, 1856, attn_splits=8)
-    path = tmp_path / "metrics.json"
+@pytest.fixture(scope="module")
+def model(gpu):
+    cfg = moert.Config(**{**moert.GRANITE_1B, "layers": 16, "vocab": 211})
+    return moert.SynthModel(cfg, seed=3, std=0.05)
+
+
+def generate(m, path, n_new, gaps):
+    """1500 prompt tokens (three passes) and n_new new ones, every read-back published: the (state, speed) pairs that a
+    thread reading the file throughout saw, and the request."""
+    g = moert.GpuModel(m, 2560, attn_splits=8)
     mx = moert.Metrics(path)
     g.attach_metrics(mx, 0)
-    prompt = np.random.default_rng(8).integers(0, cfg.vocab, 1500)
+    prompt = np.random.default_rng(8).integers(0, m.cfg.vocab, 1500)
     g.generate(prompt, 8)  # the passes' buffers
     g.reset()
     seen, stop = [], threading.Event()
@@ -30,28 +31,38 @@ def test_progress_and_speeds_of_a_prompt_read_in_passes(gpu, tmp_path):
     def watch():
         while not stop.is_set():
             kind, s = moert.read_metrics(path)
-            if kind == "live":
+            if kind == "live" and (not seen or seen[-1] != (s["state"], s["speed"])):
                 seen.append((s["state"], s["speed"]))
             time.sleep(0.0001)
 
     t = threading.Thread(target=watch)
     t.start()
     try:
-        g.generate(prompt, 300)
+        g.generate(prompt, n_new, gaps=gaps)
     finally:
         stop.set()
         t.join()
     request = moert.read_metrics(path)[1]["requests"][0]
-    distinct = []
-    for s in seen:
-        if not distinct or distinct[-1] != s:
-            distinct.append(s)
-    print(request, *distinct, sep="\n")
+    print(request, *seen[:20], sep="\n")
     g.attach_metrics(None)
     g.close()
     mx.close()
-    assert (request["prompt_tokens"], request["output_tokens"]) == (1500, 300)
-    reading = [s for s, _ in distinct if s["kind"] == "reading"]
-    assert any(0 < s["done"] < 1500 for s in reading), reading
-    now = [sp["decode_now"] for s, sp in distinct if s["kind"] == "generating"]
-    assert now and max(now) < 4 * request["decode_tok_s"], (now, request)
+    assert (request["prompt_tokens"], request["output_tokens"]) == (1500, n_new)
+    return seen, request
+
+
+def test_progress_through_a_prompt_read_in_passes(model, tmp_path):
+    """The first pass's read-back is complete milliseconds before the last of 1000 steps is launched, and the next one
+    waits behind everything launched by then: the prompt's progress stands in the file for that long."""
+    seen, _ = generate(model, tmp_path / "metrics.json", 1000, False)
+    done = [s["done"] for s, _ in seen if s["kind"] == "reading"]
+    assert any(0 < d < 1500 for d in done), done
+
+
+def test_the_decode_speed_does_not_count_the_prompt(model, tmp_path):
+    """With gaps every step is waited for, so read-backs follow one another through the new tokens, the first of them
+    behind the prompt. A window that counted the prompt's tokens as new ones would show hundreds of times the decode
+    speed of the request."""
+    seen, request = generate(model, tmp_path / "metrics.json", 60, True)
+    now = [sp["decode_now"] for s, sp in seen if s["kind"] == "generating"]
+    assert len(now) > 2 and max(now) < 4 * request["decode_tok_s"], (now, request)
